@@ -108,7 +108,8 @@ typedef struct tmc_run_stats {
     uint64_t photons; /* photons walked */
     uint64_t interactions; /* absorption events (iterations of photon.c:20) */
     uint64_t truncated; /* photons stopped by max_interactions */
-    double kernel_ms; /* walk kernel time, HIP events on the library stream */
+    double kernel_ms; /* walk kernel time: HIP events on the library stream, or, for small runs, the device's
+                         real-time counter */
     double total_ms; /* whole call: clears, kernel, copies back */
     uint32_t grid, block, chunk; /* launch shape used */
     uint32_t sampler;

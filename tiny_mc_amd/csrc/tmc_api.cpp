@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "../../include/tiny_mc_gpu.h"
+#include "tmc_cohort.h"
 #include "tmc_context.h"
 #include "tmc_internal.h"
 
@@ -37,6 +38,9 @@ int destroy_context(Context* c)
     (void)hipSetDevice(c->device);
     if (c->d_work)
         tmc::release_device(c->d_work);
+    tmc::release_device(c->d_table);
+    tmc::release_host(c->h_out);
+    tmc::release_host(c->h_weight);
     if (c->ev_start)
         (void)hipEventDestroy(c->ev_start);
     if (c->ev_stop)
@@ -115,6 +119,19 @@ int ensure_work(Context* c)
         c->d_work = nullptr;
         return TMC_E_NOMEM;
     }
+    if (hipHostMalloc((void**)&c->h_out, tmc::run_work_words(TMC_MAX_SHELLS) * sizeof(unsigned long long),
+                      hipHostMallocCoherent)
+            != hipSuccess
+        || hipHostGetDevicePointer((void**)&c->d_out, c->h_out, 0) != hipSuccess
+        || hipHostMalloc((void**)&c->h_weight, tmc::kTableEntries * sizeof(float), hipHostMallocCoherent)
+            != hipSuccess
+        || hipHostGetDevicePointer((void**)&c->d_weight, c->h_weight, 0) != hipSuccess)
+        return TMC_E_NOMEM;
+    std::memset(c->h_out, 0, 8);
+    if (hipMalloc(&c->d_table, 16ull * tmc::kTableEntries) != hipSuccess) {
+        c->d_table = nullptr;
+        return TMC_E_NOMEM;
+    }
     return TMC_OK;
 }
 
@@ -146,6 +163,15 @@ void tmc::release_host(void* p)
         release([p]() { (void)hipHostFree(p); });
 }
 
+bool tmc::unless_serving(const std::function<void()>& fn)
+{
+    std::lock_guard<std::mutex> lock(g_release_mutex);
+    if (g_serving_kernels > 0)
+        return false;
+    fn();
+    return true;
+}
+
 void tmc::serving_kernel_started()
 {
     std::lock_guard<std::mutex> lock(g_release_mutex);
@@ -174,6 +200,94 @@ double u128_to_double(uint64_t lo, uint64_t hi)
 
 } // namespace
 
+namespace {
+
+/* Longest time a run spins on its result's token before it waits for the
+ * stream: the token comes 10 us before hipStreamSynchronize returns, which
+ * matters to runs of tens of microseconds. */
+constexpr std::chrono::microseconds kSpin(500);
+
+/* One binary32 run by the cohort walk: the sums, counts and times of a
+ * finished run.  TMC_E_UNSUPPORTED: this run is for the lane-per-photon walk. */
+int run_cohort(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* o, uint64_t kcap, uint64_t* tally,
+               tmc_run_stats* st)
+{
+    const uint32_t S = p->shells;
+    tmc::CohortShape shape;
+    if (!tmc::cohort_shape(p->photons, tmc::expected_interactions(p, kcap), S, (uint32_t)c->compute_units, &shape))
+        return TMC_E_UNSUPPORTED;
+    tmc::CohortArgs a;
+    std::memset(&a, 0, sizeof a);
+    /* the roulettes a photon of this run survives at most, but for one run
+     * in a thousand (its photon walks on without the table) */
+    uint32_t cuts = 3;
+    for (double n = (double)p->photons; n >= 1.0 && cuts < TMC_COHORT_CUTS; n *= 0.1)
+        ++cuts;
+    a.ncuts = tmc::weight_sequence(p, (uint32_t)tmc::kTableEntries, cuts, c->h_weight, a.cut, &a.w_end);
+    if (a.ncuts < cuts)
+        return TMC_E_UNSUPPORTED;
+    a.entries = a.cut[a.ncuts - 1];
+    a.weight = c->d_weight;
+    a.entry = c->d_table;
+    a.build = a.entries <= TMC_COHORT_BUILD ? a.entries : 0u;
+    a.seed = seed;
+    a.first_photon = o->first_photon;
+    a.photons = p->photons;
+    a.group = shape.group;
+    a.groups = shape.groups;
+    a.albedo = tmc::derived_albedo(p);
+    a.spm = tmc::derived_spm(p);
+    a.shell_max = (float)(S - 1);
+    a.shells = S;
+    a.kcap = (uint32_t)kcap;
+    a.drawing = shape.drawing;
+    a.moving = shape.moving;
+    a.copies = shape.copies;
+    a.token = ++c->token;
+    a.work = c->d_work;
+    a.out = c->d_out;
+    const uint32_t block = 64u * (a.drawing + a.moving + (a.build ? 1u : 0u));
+    if (tmc::cohort_lds_bytes(S, a.build) > 160u * 1024u)
+        return TMC_E_UNSUPPORTED;
+
+    int rc = TMC_OK;
+    const bool launched = tmc::unless_serving([&]() {
+        const bool zero = c->work_zero;
+        c->work_zero = false;
+        if ((!zero && tmc::launch_clear(c->d_work, tmc::run_work_words(TMC_MAX_SHELLS), c->stream) != hipSuccess)
+            || (!a.build && tmc::launch_cohort_table(a.weight, a.entries, c->d_table, c->stream) != hipSuccess)
+            || tmc::launch_cohort(o->sampler, o->math, a, shape.grid, block, c->stream) != hipSuccess)
+            rc = TMC_E_HIP;
+    });
+    if (!launched)
+        return TMC_E_UNSUPPORTED;
+    if (rc != TMC_OK) {
+        (void)hipStreamSynchronize(c->stream); /* h_weight may still be read */
+        return rc;
+    }
+    const auto t0 = std::chrono::steady_clock::now();
+    while (__atomic_load_n(&c->h_out[0], __ATOMIC_ACQUIRE) != a.token) {
+        if (std::chrono::steady_clock::now() - t0 > kSpin) {
+            if (hipStreamSynchronize(c->stream) != hipSuccess
+                || __atomic_load_n(&c->h_out[0], __ATOMIC_ACQUIRE) != a.token)
+                return TMC_E_HIP;
+        }
+    }
+    c->work_zero = true;
+    std::memcpy(tally, c->h_out + TMC_COHORT_COUNTERS, 4 * (size_t)S * sizeof(uint64_t));
+    if (st) {
+        st->interactions = c->h_out[1];
+        st->truncated = c->h_out[2];
+        st->kernel_ms = 1e-5 * (double)c->h_out[3]; /* 100 MHz ticks */
+        st->grid = shape.grid;
+        st->block = block;
+        st->chunk = a.group;
+    }
+    return TMC_OK;
+}
+
+} // namespace
+
 int tmc::run_walk(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* o, unsigned long long* work,
                   uint64_t* tally, tmc_run_stats* st)
 {
@@ -196,6 +310,22 @@ int tmc::run_walk(Context* c, const tmc_params* p, uint64_t seed, const tmc_opti
     if (o->reserved)
         return TMC_E_INVALID;
     const uint32_t table_k = tmc::weight_table_entries(p, o->precision, p->photons, o->weight_table);
+    /* the cohort walk: binary32 runs of the allocating entry point with no
+     * launch shape or table asked for (cohort_shape has the sizes) */
+    if (work == c->d_work && o->precision == TMC_PRECISION_FP32 && !o->block && !o->grid && !o->chunk
+        && !o->weight_table) {
+        const int rc = run_cohort(c, p, seed, o, kcap, tally, st);
+        if (rc == TMC_OK && st) {
+            st->photons = p->photons;
+            st->total_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+            st->sampler = o->sampler;
+            st->precision = o->precision;
+            st->math = o->math;
+            st->weight_table = table_k;
+        }
+        if (rc != TMC_E_UNSUPPORTED)
+            return rc;
+    }
     uint32_t grid = o->grid;
     if (grid == 0) {
         int per_cu = 0;
@@ -256,6 +386,9 @@ int tmc::run_walk(Context* c, const tmc_params* p, uint64_t seed, const tmc_opti
     a.table_k = table_k;
     a.counters = d_counters;
     a.tally = d_tally;
+
+    if (work == c->d_work)
+        c->work_zero = false;
 
     float kernel_ms = 0.0f;
     /* a fill kernel, not a memset: the same sequence serves callers that

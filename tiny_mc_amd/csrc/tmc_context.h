@@ -21,12 +21,22 @@ namespace tmc {
 constexpr size_t kRunCounterWords = 4;
 constexpr size_t run_work_words(uint32_t shells) { return kRunCounterWords + 4 * (size_t)shells; }
 
+/* Entries of the cohort walk's weight table (16 bytes each). */
+constexpr size_t kTableEntries = 1u << 20;
+
 struct Context {
     int device = -1;
     int compute_units = 0;
     char arch[64] = { 0 };
     hipStream_t stream = nullptr; /* default priority */
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
+    void* d_table = nullptr; /* weight table of the cohort walk (kTableEntries entries), allocated at the first run */
+    unsigned long long* h_out = nullptr; /* host-coherent result words of the cohort walk, and their device address */
+    unsigned long long* d_out = nullptr;
+    float* h_weight = nullptr; /* weights of the run's table (host-coherent memory), and their device address */
+    float* d_weight = nullptr;
+    uint64_t token = 0; /* of the last cohort walk */
+    bool work_zero = false; /* d_work holds zeros */
     unsigned long long* d_work = nullptr; /* run_work_words(TMC_MAX_SHELLS) words, allocated at the first run */
 };
 
@@ -60,6 +70,10 @@ int scratch_setup(int device);
 void release(std::function<void()> fn);
 void release_device(void* p); /* hipFree */
 void release_host(void* p); /* hipHostFree */
+/* Runs fn, which enqueues a kernel that needs whole compute units, unless a
+ * serving kernel is resident (false): the kernel would wait for it, where one
+ * of small workgroups finds room beside a server that reserves some. */
+bool unless_serving(const std::function<void()>& fn);
 void serving_kernel_started();
 void serving_kernel_left();
 

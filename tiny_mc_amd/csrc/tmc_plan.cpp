@@ -71,6 +71,24 @@ bool tmc::weight_cadence(const tmc_params* p, uint32_t limit, uint32_t* k1_out, 
     return true;
 }
 
+uint32_t tmc::weight_sequence(const tmc_params* p, uint32_t room, uint32_t max_cuts, float* weight, uint32_t* cut,
+                              float* w_end)
+{
+    const float a = derived_albedo(p);
+    float w = 1.0f;
+    uint32_t k = 0, n = 0;
+    while (n < max_cuts && k < room) {
+        weight[k++] = w;
+        w = w * a;
+        if (w < 0.001f) {
+            w = w / 0.1f;
+            cut[n++] = k;
+        }
+    }
+    *w_end = w;
+    return n;
+}
+
 /* Mean absorptions k1 + k2 p / (1 - p) with p the survival probability
  * 1677721 / 2^24 of the (0,1] uniform. */
 double tmc::expected_interactions(const tmc_params* p, uint64_t kcap)
@@ -91,6 +109,36 @@ double tmc::expected_interactions(const tmc_params* p, uint64_t kcap)
     if (kcap && mean > (double)kcap)
         mean = (double)kcap;
     return mean < 1.0 ? 1.0 : mean;
+}
+
+bool tmc::cohort_shape(uint64_t photons, double L, uint32_t shells, uint32_t cus, CohortShape* shape)
+{
+    if (photons == 0 || photons > TMC_COHORT_PHOTONS || cus == 0)
+        return false;
+    /* one workgroup per compute unit, and cohorts as small as that allows: a
+     * round of fewer photons is more absorptions of each, and costs little
+     * more.  But every workgroup has its sums to add to the others' at the
+     * end, 8 us for 256 of them, so short walks keep 16 photons together
+     * (1000 photons at default physics: 4 photons a cohort 30.8 us, 16: 29.3,
+     * 64: 34.2; 512 at albedo 0.99: 2: 68.9, 16: 83.2), and a handful of them
+     * in one workgroup, which has nobody to add to. */
+    const bool shortwalk = L < 200.0;
+    uint32_t group = shortwalk ? (photons <= 64 ? 64u : 16u) : 2u;
+    while (group < 64u && (photons + group - 1) / group > cus)
+        group *= 2u;
+    shape->group = group;
+    shape->groups = (uint32_t)((photons + group - 1) / group);
+    /* three coordinates of each photon, a lane each; with a weigher 16 waves */
+    shape->moving = (3u * group + 63u) / 64u;
+    shape->drawing = 15u - shape->moving;
+    shape->grid = std::min(shape->groups, cus);
+    /* blocks of sums: 8 take 256 workgroups' additions without much waiting
+     * (1: 40 us more, 32: 4 us more, for adding them up) */
+    shape->copies = std::min(8u, std::max(1u, shape->grid / 4u));
+    const uint64_t room = ((uint64_t)TMC_MAX_SHELLS * 4 + 4) / (4ull * shells + 4);
+    if (shape->copies > room)
+        shape->copies = (uint32_t)room;
+    return true;
 }
 
 /* Entries of the binary32 walk's weight table (0: the walk multiplies).

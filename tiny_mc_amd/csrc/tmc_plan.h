@@ -42,9 +42,38 @@ float derived_spm(const tmc_params* p);
  * the second (false if the first is longer than `limit`). */
 bool weight_cadence(const tmc_params* p, uint32_t limit, uint32_t* k1, uint32_t* k2);
 
+/* The binary32 weight sequence itself: weight[k] is deposited at absorption
+ * k, and cut[i] absorptions end with the i-th roulette, after which a survivor
+ * goes on with that weight divided by 0.1f.  Stops after max_cuts roulettes or
+ * `room` weights; returns the roulettes found (fewer than max_cuts: the
+ * weights end before the next one), *w_end the weight that would follow. */
+uint32_t weight_sequence(const tmc_params* p, uint32_t room, uint32_t max_cuts, float* weight, uint32_t* cut,
+                         float* w_end);
+
 /* Expected absorptions per photon of the FP32 weight cadence with the
  * roulette of photon.c:45-49, capped at kcap (scheduling estimate). */
 double expected_interactions(const tmc_params* p, uint64_t kcap);
+
+/* Launch shape of the cohort walk for a run. */
+struct CohortShape {
+    uint32_t group, groups; /* photons a cohort starts with, and cohorts */
+    uint32_t drawing, moving; /* waves of a workgroup, beside the weigher */
+    uint32_t grid, copies; /* workgroups, and blocks of sums they flush into */
+};
+
+/* Largest run of the cohort walk.  It walks 0.9 to 1.9e11 absorptions/s
+ * (default physics to albedo 0.99), a third of the lane-per-photon walk's rate
+ * on a full chip, which that walk only comes near with several photons a lane:
+ * both take time in proportion to a photon's absorptions, so the line is a
+ * number of photons.  Measured, cohort walk against lane per photon: 2^15
+ * photons 50 / 167 us at default physics, 167 / 1225 us at albedo 0.99; 2^17
+ * 121 / 185 us and 544 / 1218 us; 2^18 208 / 213 us and 1008 / 1484 us; 2^19
+ * 381 / 304 us and 1963 / 1880 us. */
+#define TMC_COHORT_PHOTONS (1ull << 17)
+
+/* The shape for `photons` photons of L expected absorptions each on cus
+ * compute units; false if the run is not one for the cohort walk. */
+bool cohort_shape(uint64_t photons, double L, uint32_t shells, uint32_t cus, CohortShape* shape);
 
 /* Entries of the single run's weight table for these parameters and the
  * caller's request (tmc_options.weight_table; 0: none). */
