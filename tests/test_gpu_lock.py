@@ -1,0 +1,71 @@
+"""The lockstep walk of large binary32 runs (more than 49,152 photons, analytic
+sampler) against the oracle's mirror: ragged sizes on either side of its
+levels, photon indices across a multiple of 2^32, caps at and beside a
+roulette, several slices, and the walk of the same photons in two runs (GPU
+tests, bit-exact)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+DEFAULT = dict(mu_a=2.0, mu_s=20.0, shells=101, microns_per_shell=50.0)
+HIGHALB = dict(mu_a=0.5, mu_s=50.0, shells=201, microns_per_shell=20.0)
+LOWALB = dict(mu_a=10.0, mu_s=10.0, shells=51, microns_per_shell=100.0)
+
+
+def check(tmc, orc, hw_tables, phys, photons, seed, first=0, math=0, kmax=0):
+    print(f"lock: {phys} photons={photons} seed={seed} first={first} math={math} kmax={kmax}", flush=True)
+    tally, st = tmc.run_raw(tmc.Params(photons=photons, **phys), seed, first_photon=first, math=math,
+                            max_interactions=kmax)
+    kw = dict(max_k=kmax) if kmax else {}
+    want, n = orc.mirror32(orc.params(**phys), seed, photons, first=first, sampler=0,
+                           tables=hw_tables if math == 0 else None, **kw)
+    assert st.interactions == n
+    np.testing.assert_array_equal(tally, want)
+    return st
+
+
+@pytest.mark.parametrize("math", [0, 1])
+@pytest.mark.parametrize("phys,photons", [(DEFAULT, 49153), (DEFAULT, 65535), (DEFAULT, 400001), (DEFAULT, 4000037),
+                                          (LOWALB, 524289), (LOWALB, 9000001), (HIGHALB, 60000),
+                                          (dict(DEFAULT, shells=450, microns_per_shell=9.0), 70000),
+                                          (dict(DEFAULT, shells=1), 50000),
+                                          (dict(mu_a=100.0, mu_s=1e-30, shells=3, microns_per_shell=50.0), 60000)])
+def test_sizes(tmc, orc, hw_tables, phys, photons, math):
+    check(tmc, orc, hw_tables, phys, photons, 71 + photons, math=math)
+
+
+@pytest.mark.parametrize("first", [(1 << 32) - 100000, (1 << 32) - 1, 5 << 32, (1 << 33) - 199990])
+def test_index_crossings(tmc, orc, hw_tables, first):
+    check(tmc, orc, hw_tables, DEFAULT, 200000, (7 << 40) + 3, first=first)
+
+
+@pytest.mark.parametrize("kmax", [1, 72, 73, 74, 96, 97, 98, 121, 122, 200])
+def test_caps_beside_the_roulettes(tmc, orc, hw_tables, kmax):
+    st = check(tmc, orc, hw_tables, DEFAULT, 600000, 5, kmax=kmax)
+    assert st.truncated > 0 or kmax == 200  # past six roulettes 0.6 photons are expected
+
+
+def test_more_than_one_slice(tmc):
+    """2^26 + 12,345 photons (two slices of 2^26) equal the sum of the two
+    parts of the range run alone, which other sizes of launch walk."""
+    n, a = (1 << 26) + 12345, 41000003
+    whole, st = tmc.run_raw(tmc.Params(photons=n, **DEFAULT), 99)
+    lo, s1 = tmc.run_raw(tmc.Params(photons=a, **DEFAULT), 99)
+    hi, s2 = tmc.run_raw(tmc.Params(photons=n - a, **DEFAULT), 99, first_photon=a)
+    other, s3 = tmc.run_raw(tmc.Params(photons=n, **DEFAULT), 99, weight_table=649)  # lane per photon
+    assert st.interactions == s1.interactions + s2.interactions == s3.interactions
+    np.testing.assert_array_equal(whole, other)
+
+    def big(t):
+        return [int(t[2 * i]) + (int(t[2 * i + 1]) << 64) for i in range(2 * 101)]
+
+    assert big(whole) == [x + y for x, y in zip(big(lo), big(hi))]
+
+
+def test_alternating_runs(tmc, orc, hw_tables):
+    """Large and small runs of different physics and sizes, one after the
+    other: each finds its words clear and its lists large enough."""
+    for i, (phys, photons) in enumerate([(DEFAULT, 70000), (HIGHALB, 300), (LOWALB, 3000000), (DEFAULT, 50000),
+                                         (DEFAULT, 20), (HIGHALB, 70000)]):
+        check(tmc, orc, hw_tables, phys, photons, 160 + i)

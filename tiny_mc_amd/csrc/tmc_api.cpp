@@ -39,6 +39,7 @@ int destroy_context(Context* c)
     if (c->d_work)
         tmc::release_device(c->d_work);
     tmc::release_device(c->d_table);
+    tmc::release_device(c->d_lists);
     tmc::release_host(c->h_out);
     tmc::release_host(c->h_weight);
     if (c->ev_start)
@@ -207,56 +208,67 @@ namespace {
  * matters to runs of tens of microseconds. */
 constexpr std::chrono::microseconds kSpin(500);
 
-/* One binary32 run by the cohort walk: the sums, counts and times of a
- * finished run.  TMC_E_UNSUPPORTED: this run is for the lane-per-photon walk. */
-int run_cohort(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* o, uint64_t kcap, uint64_t* tally,
-               tmc_run_stats* st)
+/* The weight table of a run and the arguments its launches share.  `cuts`:
+ * roulettes the table is to span.  False if it does not fit. */
+bool weigh(Context* c, const tmc_params* p, uint64_t seed, uint64_t kcap, uint32_t cuts, tmc::CohortArgs* a)
 {
-    const uint32_t S = p->shells;
-    tmc::CohortShape shape;
-    if (!tmc::cohort_shape(p->photons, tmc::expected_interactions(p, kcap), S, (uint32_t)c->compute_units, &shape))
-        return TMC_E_UNSUPPORTED;
-    tmc::CohortArgs a;
-    std::memset(&a, 0, sizeof a);
-    /* the roulettes a photon of this run survives at most, but for one run
-     * in a thousand (its photon walks on without the table) */
-    uint32_t cuts = 3;
-    for (double n = (double)p->photons; n >= 1.0 && cuts < TMC_COHORT_CUTS; n *= 0.1)
-        ++cuts;
-    a.ncuts = tmc::weight_sequence(p, (uint32_t)tmc::kTableEntries, cuts, c->h_weight, a.cut, &a.w_end);
-    if (a.ncuts < cuts)
-        return TMC_E_UNSUPPORTED;
-    a.entries = a.cut[a.ncuts - 1];
-    a.weight = c->d_weight;
-    a.entry = c->d_table;
-    a.build = a.entries <= TMC_COHORT_BUILD ? a.entries : 0u;
-    a.seed = seed;
-    a.first_photon = o->first_photon;
-    a.photons = p->photons;
-    a.group = shape.group;
-    a.groups = shape.groups;
-    a.albedo = tmc::derived_albedo(p);
-    a.spm = tmc::derived_spm(p);
-    a.shell_max = (float)(S - 1);
-    a.shells = S;
-    a.kcap = (uint32_t)kcap;
-    a.drawing = shape.drawing;
-    a.moving = shape.moving;
-    a.copies = shape.copies;
-    a.token = ++c->token;
-    a.work = c->d_work;
-    a.out = c->d_out;
-    const uint32_t block = 64u * (a.drawing + a.moving + (a.build ? 1u : 0u));
-    if (tmc::cohort_lds_bytes(S, a.build) > 160u * 1024u)
-        return TMC_E_UNSUPPORTED;
+    std::memset(a, 0, sizeof *a);
+    a->ncuts = tmc::weight_sequence(p, (uint32_t)tmc::kTableEntries - 2u, cuts, c->h_weight, a->cut, &a->w_end);
+    if (a->ncuts < cuts)
+        return false;
+    a->entries = a->cut[a->ncuts - 1];
+    a->weight = c->d_weight;
+    a->entry = c->d_table;
+    a->seed = seed;
+    a->albedo = tmc::derived_albedo(p);
+    a->spm = tmc::derived_spm(p);
+    a->shell_max = (float)(p->shells - 1);
+    a->shells = p->shells;
+    a->kcap = (uint32_t)kcap;
+    a->work = c->d_work;
+    a->out = c->d_out;
+    return true;
+}
 
+/* Roulettes the table of a run of n photons spans: as many as one of its
+ * photons survives but in one run in a thousand (that photon walks on without
+ * the table). */
+uint32_t cuts_for(double n)
+{
+    uint32_t cuts = 3;
+    for (; n >= 1.0 && cuts < TMC_COHORT_CUTS; n *= 0.1)
+        ++cuts;
+    return cuts;
+}
+
+/* About the absorptions of a photon's first cycle (the weight falls to a
+ * thousandth), at most kcap. */
+double first_cycle(const tmc_params* p, uint64_t kcap)
+{
+    const double a = (double)tmc::derived_albedo(p);
+    const double k = a > 0.0 ? std::log(0.001) / std::log(a) : 1.0;
+    return std::min(std::max(k, 1.0), (double)kcap);
+}
+
+void use_shape(const tmc::CohortShape& s, tmc::CohortArgs* a)
+{
+    a->group = s.group;
+    a->drawing = s.drawing;
+    a->moving = s.moving;
+    a->copies = s.copies;
+}
+
+/* Enqueues a run by `launches` behind what clears the device words, unless a
+ * serving kernel is resident (TMC_E_UNSUPPORTED), and waits for its result. */
+int finish_enqueued(Context* c, uint64_t token, uint32_t shells, uint64_t* tally, tmc_run_stats* st,
+                    const std::function<bool()>& launches)
+{
     int rc = TMC_OK;
     const bool launched = tmc::unless_serving([&]() {
         const bool zero = c->work_zero;
         c->work_zero = false;
         if ((!zero && tmc::launch_clear(c->d_work, tmc::run_work_words(TMC_MAX_SHELLS), c->stream) != hipSuccess)
-            || (!a.build && tmc::launch_cohort_table(a.weight, a.entries, c->d_table, c->stream) != hipSuccess)
-            || tmc::launch_cohort(o->sampler, o->math, a, shape.grid, block, c->stream) != hipSuccess)
+            || !launches())
             rc = TMC_E_HIP;
     });
     if (!launched)
@@ -266,24 +278,237 @@ int run_cohort(Context* c, const tmc_params* p, uint64_t seed, const tmc_options
         return rc;
     }
     const auto t0 = std::chrono::steady_clock::now();
-    while (__atomic_load_n(&c->h_out[0], __ATOMIC_ACQUIRE) != a.token) {
+    while (__atomic_load_n(&c->h_out[0], __ATOMIC_ACQUIRE) != token) {
         if (std::chrono::steady_clock::now() - t0 > kSpin) {
             if (hipStreamSynchronize(c->stream) != hipSuccess
-                || __atomic_load_n(&c->h_out[0], __ATOMIC_ACQUIRE) != a.token)
+                || __atomic_load_n(&c->h_out[0], __ATOMIC_ACQUIRE) != token)
                 return TMC_E_HIP;
         }
     }
     c->work_zero = true;
-    std::memcpy(tally, c->h_out + TMC_COHORT_COUNTERS, 4 * (size_t)S * sizeof(uint64_t));
+    std::memcpy(tally, c->h_out + TMC_COHORT_COUNTERS, 4 * (size_t)shells * sizeof(uint64_t));
     if (st) {
         st->interactions = c->h_out[1];
         st->truncated = c->h_out[2];
         st->kernel_ms = 1e-5 * (double)c->h_out[3]; /* 100 MHz ticks */
+    }
+    return TMC_OK;
+}
+
+/* One binary32 run by the cohort walk.  TMC_E_UNSUPPORTED: not one for it. */
+int run_cohort(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* o, uint64_t kcap, uint64_t* tally,
+               tmc_run_stats* st)
+{
+    tmc::CohortShape shape;
+    const uint64_t most = o->sampler == TMC_SAMPLER_ANALYTIC ? TMC_COHORT_PHOTONS : TMC_COHORT_PHOTONS_REJECTION;
+    if (!tmc::cohort_shape(p->photons, most, first_cycle(p, kcap), p->shells, (uint32_t)c->compute_units, &shape))
+        return TMC_E_UNSUPPORTED;
+    tmc::CohortArgs a;
+    if (!weigh(c, p, seed, kcap, cuts_for((double)p->photons), &a))
+        return TMC_E_UNSUPPORTED;
+    a.build = a.entries <= TMC_COHORT_BUILD ? a.entries : 0u;
+    if (tmc::cohort_lds_bytes(p->shells, a.build) > 160u * 1024u)
+        return TMC_E_UNSUPPORTED;
+    a.first_photon = o->first_photon;
+    a.photons = p->photons;
+    a.finish = 1;
+    a.token = ++c->token;
+    use_shape(shape, &a);
+    const uint32_t block = 64u * (a.drawing + a.moving + (a.build ? 1u : 0u));
+    const int rc = finish_enqueued(c, a.token, p->shells, tally, st, [&]() {
+        return (a.build
+                || tmc::launch_cohort_table(a.weight, a.entries, c->d_table, nullptr, 0, nullptr, c->stream)
+                    == hipSuccess)
+            && tmc::launch_cohort(o->sampler, o->math, a, shape.grid, block, c->stream) == hipSuccess;
+    });
+    if (rc == TMC_OK && st) {
         st->grid = shape.grid;
         st->block = block;
         st->chunk = a.group;
     }
-    return TMC_OK;
+    return rc;
+}
+
+/* Survivors of a large run that the cohort walk takes over: with fewer, the
+ * lockstep waves leave most of the chip idle.  Flat from 40,000 to 250,000 (2^20
+ * photons 236 and 233 us, 2^26 8.59 and 8.61 ms); 15,000 cost 2^20 photons 5 us. */
+constexpr uint32_t kHandOver = 40000;
+
+/* Photons whose survivors share one of `stripes` stripes, at most: those of
+ * every stripes-th workgroup, with room for waves that claim more than
+ * others. */
+uint32_t list_photons(uint32_t photons, uint32_t stripes)
+{
+    const uint32_t share = photons / stripes;
+    return share + share / 8u + 4096u;
+}
+
+/* Places of a stripe of a survivor list, for n photons that share it: a tenth
+ * survive a roulette, so an eighth and a slack of 256 for the first list, an
+ * eighth of that for the second. */
+uint32_t list_cap(uint32_t which, uint32_t n) { return (which ? n / 64u : n / 8u) + 256u; }
+
+/* One large binary32 run by lockstep waves, level by level, and the cohort
+ * walk for the last survivors.  TMC_E_UNSUPPORTED: not one for it. */
+int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* o, uint64_t kcap, uint64_t* tally,
+             tmc_run_stats* st)
+{
+    /* (from 450 shells on, fewer than 5 waves' sums fit a SIMD's share of LDS) */
+    if (p->photons <= TMC_COHORT_PHOTONS || p->photons > (1ull << 40) || p->shells > 450)
+        return TMC_E_UNSUPPORTED;
+    /* many photons of short walks: launching them 64 at a time and appending
+     * the survivors costs what the step saves (albedo 0.5: 2^23 photons 951 us
+     * lane per photon, 306 us here; 2^27 2841 and 2897 us) */
+    if (p->photons > (1ull << 26) && first_cycle(p, kcap) < 32.0)
+        return TMC_E_UNSUPPORTED;
+    const uint64_t slice = std::min<uint64_t>(p->photons, 1ull << tmc::kSliceLog);
+    uint32_t levels = 1;
+    double rest = 0.1 * (double)slice; /* survivors the cohort walk takes over */
+    for (; rest > (double)kHandOver; rest *= 0.1)
+        ++levels;
+    tmc::CohortArgs a;
+    if (!weigh(c, p, seed, kcap, levels + cuts_for(rest), &a))
+        return TMC_E_UNSUPPORTED;
+    if (tmc::cohort_lds_bytes(p->shells, 0) > 160u * 1024u)
+        return TMC_E_UNSUPPORTED;
+    /* the lists, counters and start time, kept for the next such run */
+    uint32_t log = 20;
+    while ((1ull << log) < slice)
+        ++log;
+    const uint32_t most = list_photons(1u << log, tmc::kStripes);
+    const size_t places[2] = { (size_t)tmc::kStripes * list_cap(0, most), (size_t)tmc::kStripes * list_cap(1, most) };
+    if (!c->d_lists || c->lists_log < log) {
+        tmc::release_device(c->d_lists);
+        c->d_lists = nullptr;
+        const size_t bytes = 28 * (places[0] + places[1]) + 4ull * tmc::kRunCounters + 8;
+        if (hipMalloc(&c->d_lists, bytes) != hipSuccess) {
+            c->d_lists = nullptr;
+            return TMC_E_UNSUPPORTED;
+        }
+        c->lists_log = log;
+    }
+    unsigned long long* const start = (unsigned long long*)c->d_lists;
+    uint32_t* const counters = (uint32_t*)(start + 1);
+    tmc::PhotonList lists[2];
+    float* at = (float*)(counters + tmc::kRunCounters);
+    for (uint32_t w = 0; w < 2; ++w) {
+        lists[w].photon = (uint32_t*)at;
+        at += places[w];
+        for (float*& f : lists[w].state) {
+            f = at;
+            at += places[w];
+        }
+    }
+    /* slices: at most `slice` photons, none across a multiple of 2^32 */
+    struct Slice {
+        uint64_t first;
+        uint32_t photons;
+    };
+    std::vector<Slice> slices;
+    for (uint64_t done = 0; done < p->photons;) {
+        const uint64_t first = o->first_photon + done;
+        const uint64_t n = std::min<uint64_t>(std::min<uint64_t>(slice, p->photons - done),
+                                              (1ull << 32) - (first & 0xFFFFFFFFull));
+        slices.push_back({ first, (uint32_t)n });
+        done += n;
+    }
+    const uint32_t words = tmc::kStripes * TMC_LOCK_LINE; /* of a level's counts */
+    const uint32_t per_slice = levels * words + TMC_LOCK_RANGES * TMC_LOCK_LINE;
+    if (slices.size() * per_slice > tmc::kRunCounters)
+        return TMC_E_UNSUPPORTED;
+
+    const uint32_t block = 256, cus = (uint32_t)c->compute_units;
+    /* (the batches go round the resident waves, so a workgroup that had to wait
+     * for another to end would double the launch's time) */
+    int per_cu = 0;
+    if (tmc::lock_occupancy(o->math, block, p->shells, &per_cu) != hipSuccess || per_cu <= 0)
+        return TMC_E_HIP;
+    const uint32_t grid_most = (uint32_t)per_cu * cus;
+    tmc::CohortShape shape;
+    tmc::cohort_shape((uint64_t)std::max(1.0, rest), kHandOver + 1u, first_cycle(p, kcap), p->shells, cus, &shape);
+    use_shape(shape, &a);
+    a.copies = 8; /* (at most 450 shells: they fit) */
+    a.token = ++c->token;
+    a.start = start;
+    a.list = lists[(levels - 1) & 1u];
+    a.seg0 = levels;
+
+    tmc::LockArgs l;
+    std::memset(&l, 0, sizeof l);
+    l.seed = seed;
+    l.albedo = a.albedo;
+    l.spm = a.spm;
+    l.shell_max = a.shell_max;
+    l.shells = a.shells;
+    l.kcap = a.kcap;
+    l.entry = c->d_table;
+    l.work = c->d_work;
+    l.copies = a.copies;
+    uint32_t grid0 = 0;
+    auto launches = [&]() {
+        /* two more entries than the steps read ahead of the last cut */
+        if (tmc::launch_cohort_table(a.weight, a.entries, c->d_table, counters, (uint32_t)slices.size() * per_slice,
+                                     start, c->stream)
+            != hipSuccess)
+            return false;
+        for (size_t si = 0; si < slices.size(); ++si) {
+            uint32_t* const count = counters + si * per_slice; /* survivors by level */
+            double n = (double)slices[si].photons;
+            bool capped = false;
+            const uint32_t wgs = (uint32_t)std::min<double>(grid_most, std::ceil(n / 256.0));
+            /* at least eight workgroups a stripe, or one stripe */
+            l.stripes = std::min(std::min(tmc::kStripes, cus), std::max(1u, wgs / 8u));
+            const uint32_t per = list_photons(slices[si].photons, l.stripes);
+            l.first_photon = slices[si].first;
+            l.photons = slices[si].photons;
+            for (uint32_t lv = 0; lv < levels && !capped; ++lv, n *= 0.1) {
+                l.level = lv;
+                l.k0 = lv ? a.cut[lv - 1] : 0u;
+                l.k1 = std::min(a.cut[lv], a.kcap);
+                l.cut_ends = a.cut[lv] <= a.kcap;
+                l.cap_ends = a.kcap <= a.cut[lv];
+                capped = l.cap_ends;
+                l.in = lists[(lv + 1) & 1u];
+                l.out = lists[lv & 1u];
+                l.in_count = count + (lv ? lv - 1 : 0) * words;
+                l.in_cap = l.out_cap;
+                l.out_count = count + lv * words;
+                l.out_cap = list_cap(lv & 1u, per);
+                const double waves = std::ceil(n / 64.0);
+                const uint32_t grid = std::max(l.stripes, (uint32_t)std::min<double>(grid_most, std::ceil(waves / 4.0)));
+                l.chunk = 0;
+                if (lv == 0) {
+                    grid0 = grid;
+                    const uint64_t each = (uint64_t)waves / (4u * grid); /* batches a wave */
+                    if (each >= 8) {
+                        l.chunk = 64u * (uint32_t)std::min<uint64_t>(32, std::max<uint64_t>(1, each / 32));
+                        l.range = (slices[si].photons / TMC_LOCK_RANGES + 64u) / 64u * 64u;
+                        l.cursor = count + levels * words;
+                    }
+                }
+                if (tmc::launch_lock(o->math, l, grid, block, c->stream) != hipSuccess)
+                    return false;
+            }
+            a.finish = si + 1 == slices.size();
+            a.first_photon = slices[si].first;
+            a.list_count = count + (levels - 1) * words;
+            a.list_cap = list_cap((levels - 1) & 1u, per);
+            a.stripes = l.stripes;
+            if (tmc::launch_cohort(o->sampler, o->math, a, cus, 64u * (a.drawing + a.moving), c->stream)
+                != hipSuccess)
+                return false;
+        }
+        return true;
+    };
+    const int rc = finish_enqueued(c, a.token, p->shells, tally, st, launches);
+    if (rc == TMC_OK && c->h_out[2] >= TMC_LOCK_OVERFLOW)
+        return TMC_E_UNSUPPORTED;
+    if (rc == TMC_OK && st) {
+        st->grid = grid0;
+        st->block = block;
+        st->chunk = 64;
+    }
+    return rc;
 }
 
 } // namespace
@@ -310,11 +535,13 @@ int tmc::run_walk(Context* c, const tmc_params* p, uint64_t seed, const tmc_opti
     if (o->reserved)
         return TMC_E_INVALID;
     const uint32_t table_k = tmc::weight_table_entries(p, o->precision, p->photons, o->weight_table);
-    /* the cohort walk: binary32 runs of the allocating entry point with no
-     * launch shape or table asked for (cohort_shape has the sizes) */
+    /* the cohort and lockstep walks: binary32 runs of the allocating entry point
+     * with no launch shape or table asked for (cohort_shape has the sizes) */
     if (work == c->d_work && o->precision == TMC_PRECISION_FP32 && !o->block && !o->grid && !o->chunk
         && !o->weight_table) {
-        const int rc = run_cohort(c, p, seed, o, kcap, tally, st);
+        int rc = run_cohort(c, p, seed, o, kcap, tally, st);
+        if (rc == TMC_E_UNSUPPORTED && o->sampler == TMC_SAMPLER_ANALYTIC)
+            rc = run_lock(c, p, seed, o, kcap, tally, st);
         if (rc == TMC_OK && st) {
             st->photons = p->photons;
             st->total_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();

@@ -22,11 +22,16 @@ namespace tmc {
 #endif
 #define TMC_COHORT_ROWS (16u * TMC_COHORT_WAVE_ROWS)
 
+/* Photons between two roulettes: index in the slice, position and direction. */
+struct PhotonList {
+    uint32_t* photon;
+    float* state[6]; /* x, y, z, then the direction */
+};
+
 struct CohortArgs {
     uint64_t seed; /* Philox key */
     uint64_t first_photon; /* photon index of cohort 0's first photon */
     uint64_t photons; /* photons in this launch */
-    uint32_t groups; /* cohorts: ceil(photons / group) */
     float albedo, spm, shell_max; /* as WalkArgs */
     uint32_t shells;
     uint32_t kcap; /* stop a photon after kcap absorptions */
@@ -41,6 +46,13 @@ struct CohortArgs {
     uint32_t cut[TMC_COHORT_CUTS];
     float w_end; /* the weight with which a survivor of the last one goes on */
     uint32_t copies; /* copies of the sums the workgroups flush into */
+    /* cohorts from a list (list.photon not null) of photons first_photon + i
+     * after their seg0-th roulette, instead of first_photon, first_photon + 1, ... */
+    PhotonList list;
+    const uint32_t* list_count; /* photons of each stripe of the list (LockArgs), or more if it overflowed */
+    uint32_t list_cap, stripes, seg0;
+    uint32_t finish; /* this launch ends the run: result to `out` */
+    const unsigned long long* start; /* real-time ticks at the run's start; null: this launch's */
     uint64_t token; /* written to out[0] when the result is there */
     unsigned long long* work; /* `copies` blocks of 4 counters ([0] workgroups done, [1] interactions, [2] truncated,
                                  [3] of the first: blocks done) and 4*shells words of 128-bit sums (lo, hi); zero
@@ -50,8 +62,56 @@ struct CohortArgs {
 
 size_t cohort_lds_bytes(uint32_t shells, uint32_t entries);
 
-/* Converts n weights (host memory) to table entries of 16 bytes. */
-hipError_t launch_cohort_table(const float* weight, uint32_t n, void* entry, hipStream_t stream);
+/* Words between two stripes' counts: a cache line. */
+#define TMC_LOCK_LINE 16u
+/* Parts of a slice the waves claim from: workgroup b, on XCD b mod 8, claims
+ * from part b mod 8. */
+#define TMC_LOCK_RANGES 8u
+
+/* Set in a block's truncated photons when a list had no room for a survivor:
+ * the run is repeated by the other walk.  (The lists hold an eighth of a stripe's
+ * photons and a slack, where a tenth survive: never seen.) */
+#define TMC_LOCK_OVERFLOW (1ull << 56)
+
+/* One level of a large run (walk_lock): the photons of a slice, or of the list
+ * the level before left, from absorption k0 to k1. */
+struct LockArgs {
+    uint64_t seed; /* Philox key */
+    uint64_t first_photon; /* index of the slice's photon 0 */
+    float albedo, spm, shell_max; /* as WalkArgs */
+    uint32_t shells;
+    uint32_t kcap; /* stop a photon after kcap absorptions */
+    uint32_t chunk; /* level 0: photons a wave claims at a time, a multiple of 64, from one of TMC_LOCK_RANGES parts of
+                       `range` photons (a multiple of 64 too); 0: the batches go round the waves */
+    uint32_t range;
+    uint32_t* cursor; /* claims, TMC_LOCK_LINE words apart */
+    uint32_t level; /* 0: the slice's photons, else the list's */
+    uint32_t photons; /* of the slice (< 2^31) */
+    uint32_t k0, k1;
+    uint32_t cut_ends, cap_ends; /* whether k1 is a roulette, and the cap */
+    const void* entry; /* table of pairs of images, at least two entries beyond k1 */
+    /* the lists and their counts are split into stripes, workgroup b reading
+     * and appending to stripe b mod `stripes`, of in_cap and out_cap places;
+     * counts TMC_LOCK_LINE words apart */
+    uint32_t stripes;
+    PhotonList in, out;
+    const uint32_t* in_count;
+    uint32_t* out_count;
+    uint32_t in_cap, out_cap;
+    uint32_t copies;
+    unsigned long long* work; /* as CohortArgs */
+};
+
+size_t lock_lds_bytes(uint32_t shells, uint32_t block);
+/* Resident workgroups per CU of walk_lock. */
+hipError_t lock_occupancy(uint32_t math, uint32_t block, uint32_t shells, int* wg_per_cu);
+hipError_t launch_lock(uint32_t math, const LockArgs& a, uint32_t grid, uint32_t block, hipStream_t stream);
+
+/* Converts n weights (host memory) to table entries of 16 bytes, zeroes
+ * `counters` 32-bit words at `counter`, and notes the real time at *start
+ * (null: neither). */
+hipError_t launch_cohort_table(const float* weight, uint32_t n, void* entry, uint32_t* counter, uint32_t counters,
+                               unsigned long long* start, hipStream_t stream);
 hipError_t launch_cohort(uint32_t sampler, uint32_t math, const CohortArgs& a, uint32_t grid, uint32_t block,
                          hipStream_t stream);
 

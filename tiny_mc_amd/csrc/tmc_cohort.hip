@@ -90,12 +90,18 @@ __device__ __forceinline__ Images images_of(float w)
 }
 
 /* Converts a set's weights (host memory) to table entries in device memory,
- * for the sets whose table does not fit the LDS. */
-__global__ void __launch_bounds__(256) cohort_table(const float* weight, uint32_t n, Images* entry)
+ * for the runs whose table does not fit the LDS or is read by several
+ * launches, and clears a run's counters. */
+__global__ void __launch_bounds__(256) cohort_table(const float* weight, uint32_t n, Images* entry, uint32_t* counter,
+                                                    uint32_t counters, unsigned long long* start)
 {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i < n)
         entry[i] = images_of(weight[i]);
+    if (i < counters)
+        counter[i] = 0u;
+    if (i == 0u && start)
+        *start = __builtin_amdgcn_s_memrealtime();
 }
 
 /* ------------------------------------------------------------------------ */
@@ -109,6 +115,7 @@ namespace {
  * k0 + kk.  Wave-uniform, and the same in every wave of the workgroup. */
 struct Round {
     uint32_t k0, T, lg, P, flags;
+    uint32_t at; /* the cohort's first photon in the list */
     uint64_t base; /* photon index of the cohort's first photon */
 };
 
@@ -224,7 +231,7 @@ __device__ __forceinline__ void finish_run(const CohortArgs& a, unsigned long lo
     unsigned long long* const mine = a.work + (size_t)(blockIdx.x % a.copies) * block;
     ulonglong2* const out = (ulonglong2*)(a.out + TMC_COHORT_COUNTERS);
     __syncthreads();
-    if (gridDim.x == 1 && !flushed) {
+    if (a.finish && !a.list.photon && gridDim.x == 1 && !flushed) {
         const uint32_t last = a.shells - 1u;
         for (uint32_t s = threadIdx.x; s < a.shells; s += blockDim.x) {
             unsigned long long h = lds[2u * s], h2 = lds[2u * s + 1u];
@@ -252,6 +259,8 @@ __device__ __forceinline__ void finish_run(const CohortArgs& a, unsigned long lo
         /* agent-scope atomics: once they have completed, the count may
          * follow (a release fence would write the L2 back, once a wave: 20 us
          * a workgroup) */
+        if (!a.finish)
+            return;
         wait_vmem();
         __syncthreads();
         if (threadIdx.x == 0) {
@@ -304,7 +313,7 @@ __device__ __forceinline__ void finish_run(const CohortArgs& a, unsigned long lo
                 out[i - TMC_COHORT_COUNTERS / 2u] = ulonglong2{ lo, hi };
         }
         if (threadIdx.x == 0)
-            a.out[3] = __builtin_amdgcn_s_memrealtime() - *(volatile unsigned long long*)(flag + 2);
+            a.out[3] = __builtin_amdgcn_s_memrealtime() - (a.start ? *a.start : *(volatile unsigned long long*)(flag + 2));
     }
     wait_vmem(); /* every thread's result words before the token */
     __syncthreads();
@@ -430,7 +439,19 @@ __global__ void __launch_bounds__(1024) walk_cohort(CohortArgs a)
     bool flushed = false;
 
     /* the schedule: every wave steps the same one */
-    uint32_t group = blockIdx.x; /* next cohort */
+    const bool listed = a.list.photon != nullptr;
+    uint32_t group = blockIdx.x, stride = gridDim.x; /* next cohort, and from one to the next */
+    uint32_t photons = (uint32_t)a.photons, place = 0; /* place: of the stripe's first photon in the list */
+    if (listed) {
+        /* (at least as many workgroups as stripes, or one stripe) */
+        const uint32_t stripe = blockIdx.x % a.stripes;
+        const uint32_t n = a.list_count[stripe * TMC_LOCK_LINE];
+        photons = rfl32(n < a.list_cap ? n : a.list_cap);
+        place = stripe * a.list_cap;
+        group = blockIdx.x / a.stripes;
+        stride = (gridDim.x - stripe + a.stripes - 1u) / a.stripes;
+    }
+    const uint32_t groups = (photons + a.group - 1u) / a.group;
     Round prev = {}, cur = {}, next = {};
     bool alive = false;
     uint32_t k = 0, seg = 0, cut = 0, P = 0, lg = 0, par = 0;
@@ -497,15 +518,22 @@ __global__ void __launch_bounds__(1024) walk_cohort(CohortArgs a)
                 next.flags = R_PACKED;
             }
         }
-        if (!alive && group < a.groups) {
-            const uint64_t off = (uint64_t)group * a.group;
-            base = a.first_photon + off;
-            P = rfl32(a.photons - off < a.group ? (uint32_t)(a.photons - off) : a.group);
+        if (!alive && group < groups) {
+            const uint32_t off = group * a.group;
+            P = rfl32(photons - off < a.group ? photons - off : a.group);
             lg = ceil_log2(P);
             pid = lane & ((1u << lg) - 1u);
+            base = a.first_photon;
             k = 0;
-            seg = 0;
-            group += gridDim.x;
+            if (listed) {
+                pid = a.list.photon[place + off + (pid < P ? pid : 0u)];
+                k = rfl32(cuts[a.seg0 - 1u]);
+            } else {
+                base += off;
+            }
+            next.at = place + off;
+            seg = a.seg0;
+            group += stride;
             next.flags = R_FRESH;
             alive = true;
             changed = true;
@@ -611,6 +639,10 @@ __global__ void __launch_bounds__(1024) walk_cohort(CohortArgs a)
             if (cur.flags & R_FRESH) {
                 x = 0.0f;
                 u = c == 2u ? 1.0f : 0.0f;
+                if (listed && in) {
+                    x = a.list.state[c][cur.at + p];
+                    u = a.list.state[3u + c][cur.at + p];
+                }
             } else if ((cur.flags & R_PACKED) && in) {
                 x = from[c * 64u + p];
                 u = from[(3u + c) * 64u + p];
@@ -679,9 +711,12 @@ CohortKernel cohort_kernel(uint32_t sampler, uint32_t math)
 
 } // namespace
 
-hipError_t launch_cohort_table(const float* weight, uint32_t n, void* entry, hipStream_t stream)
+hipError_t launch_cohort_table(const float* weight, uint32_t n, void* entry, uint32_t* counter, uint32_t counters,
+                               unsigned long long* start, hipStream_t stream)
 {
-    hipLaunchKernelGGL(cohort_table, dim3((n + 255u) / 256u), dim3(256), 0, stream, weight, n, (Images*)entry);
+    const uint32_t most = n > counters ? n : counters;
+    hipLaunchKernelGGL(cohort_table, dim3((most + 255u) / 256u), dim3(256), 0, stream, weight, n, (Images*)entry,
+                       counter, counters, start);
     return hipGetLastError();
 }
 

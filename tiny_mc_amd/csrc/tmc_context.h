@@ -24,6 +24,11 @@ constexpr size_t run_work_words(uint32_t shells) { return kRunCounterWords + 4 *
 /* Entries of the cohort walk's weight table (16 bytes each). */
 constexpr size_t kTableEntries = 1u << 20;
 
+/* Photons of a slice of a large run (log2), and the counters of all its slices. */
+constexpr uint32_t kSliceLog = 26;
+constexpr uint32_t kRunCounters = 1u << 21;
+constexpr uint32_t kStripes = 64; /* parts of a slice and of the survivor lists */
+
 struct Context {
     int device = -1;
     int compute_units = 0;
@@ -35,6 +40,8 @@ struct Context {
     unsigned long long* d_out = nullptr;
     float* h_weight = nullptr; /* weights of the run's table (host-coherent memory), and their device address */
     float* d_weight = nullptr;
+    void* d_lists = nullptr; /* survivor lists of large runs, for slices of 2^lists_log photons */
+    uint32_t lists_log = 0;
     uint64_t token = 0; /* of the last cohort walk */
     bool work_zero = false; /* d_work holds zeros */
     unsigned long long* d_work = nullptr; /* run_work_words(TMC_MAX_SHELLS) words, allocated at the first run */

@@ -1,0 +1,375 @@
+/* Large binary32 runs with the analytic sampler: waves that carry 64 photons
+ * in lockstep from one roulette to the next.
+ *
+ * Photons launched together reach every roulette at the same absorption
+ * (tmc_cohort.hip), so a wave that launches 64 photons at once walks them
+ * through a whole cycle with one absorption count: no lane ends on the way,
+ * nothing is compared, refilled or masked, and what depends on the count
+ * alone leaves the vector unit.  Rounds 1 and 2 of the generator's half that
+ * holds the count are scalar (three 32 x 32 products fewer a step), and the
+ * weight's images come from the set's table by one load of a single address.
+ * At the roulette the tenth that survives is appended to a list in device
+ * memory, which the next launch walks through the next cycle, again 64 at a
+ * time; when few are left the cohort walk takes the list to its end.
+ *
+ * What bounds it: vector issue.  66 instructions an absorption of 64 photons
+ * (76 in walk_f32), of which the 16 products take 4.6 cycles each on a full
+ * SIMD, the 15 three-input XORs, conversions and compares 4.1, the five
+ * transcendentals 8, and the additions and multiplications of three vector
+ * registers 2.2 (4 with a scalar operand).  Measured on MI355X, whole calls,
+ * walk_f32 -> this walk: 2^20 photons at default physics 425 -> 236 us,
+ * 3,000,017 638 -> 500 us, 2^26 8.72 -> 7.87 ms; 2^20 at albedo 0.99 2.73 ->
+ * 1.38 ms; 2^17 at albedo 0.9999 117 -> 22 ms; 2^23 at albedo 0.5 951 -> 306
+ * us.
+ *
+ * Same words, same operations and the same integer sums as step(): results
+ * are bit-identical.
+ */
+#include "tmc_cohort.h"
+#include "tmc_device.h"
+#include "tmc_math.h"
+#include "tmc_philox.h"
+#include "tmc_step.h"
+
+namespace tmc {
+
+/* Copies of the overflow shell's sums in a wave's slot (16: 1% slower). */
+#define TMC_LOCK_HOT 8u
+static_assert(TMC_LOCK_HOT <= TMC_CHECK_HOT, "the shell check covers every overflow copy");
+
+/* Steps between two flushes of a wave's slot: a word takes fewer than 2^20
+ * deposits of at most 2^43 each, so it stays below 2^63. */
+#define TMC_LOCK_FLUSH_STEPS 16383u
+
+__host__ __device__ __forceinline__ size_t lock_slot_words(uint32_t shells)
+{
+    return 2u * ((size_t)shells - 1u + TMC_LOCK_HOT);
+}
+
+size_t lock_lds_bytes(uint32_t shells, uint32_t block) { return (block / 64u) * lock_slot_words(shells) * 8u; }
+
+namespace {
+
+typedef uint32_t Images __attribute__((ext_vector_type(4)));
+
+/* Philox block (k, 0) of photons with one high counter word and one k (both
+ * wave-uniform): what rounds 1 and 2 make of k is scalar.  c3k1: the high
+ * counter word ^ key1. */
+__device__ __forceinline__ tmc_u32x4 block0_uniform(uint32_t k, uint32_t c3k1, const tmc_philox_photon& pp,
+                                                    const tmc_philox_keys& ks)
+{
+    const uint64_t q0 = (uint64_t)k * TMC_PHILOX_M0;
+    const uint64_t p1 = (uint64_t)((uint32_t)(q0 >> 32) ^ c3k1) * TMC_PHILOX_M1;
+    uint32_t c0 = pp.c1r1 ^ ((uint32_t)(p1 >> 32) ^ ks.k0[1]), c2 = pp.c2r2k ^ (uint32_t)q0;
+    uint64_t a = (uint64_t)c0 * TMC_PHILOX_M0, b = (uint64_t)c2 * TMC_PHILOX_M1;
+    c0 = (uint32_t)(b >> 32) ^ ((uint32_t)p1 ^ ks.k0[2]);
+    c2 = tmc_xor3((uint32_t)(a >> 32), pp.c3r2, ks.k1[2]);
+    uint32_t c1 = (uint32_t)b, c3 = (uint32_t)a;
+#pragma unroll
+    for (int round = 3; round < 10; ++round) {
+        a = (uint64_t)c0 * TMC_PHILOX_M0;
+        b = (uint64_t)c2 * TMC_PHILOX_M1;
+        c0 = tmc_xor3((uint32_t)(b >> 32), c1, ks.k0[round]);
+        c2 = tmc_xor3((uint32_t)(a >> 32), c3, ks.k1[round]);
+        c1 = (uint32_t)b;
+        c3 = (uint32_t)a;
+    }
+    return tmc_u32x4{ c0, c1, c2, c3 };
+}
+
+/* Moves a wave's slot into its block of the global sums and zeroes it. */
+__device__ __forceinline__ void lock_flush(unsigned long long* slot, unsigned long long* g, uint32_t shells,
+                                           uint32_t lane)
+{
+    const uint32_t last = shells - 1u;
+    for (uint32_t q = lane; q < last + TMC_LOCK_HOT; q += 64u) {
+        const unsigned long long a = slot[2u * q], b = slot[2u * q + 1u];
+        slot[2u * q] = 0;
+        slot[2u * q + 1u] = 0;
+        const uint32_t s = q < last ? q : last;
+        unsigned long long oa = 0, ob = 0;
+        if (a)
+            oa = atomicAdd(g + 2u * s, a);
+        if (b)
+            ob = atomicAdd(g + 2u * shells + 2u * s, b);
+        if (oa + a < oa)
+            atomicAdd(g + 2u * s + 1u, 1ull);
+        if (ob + b < ob)
+            atomicAdd(g + 2u * shells + 2u * s + 1u, 1ull);
+    }
+}
+
+/* The block of global sums this wave flushes into. */
+__device__ __forceinline__ unsigned long long* lock_block(const LockArgs& a, uint32_t wave)
+{
+    return a.work
+        + (size_t)((blockIdx.x * (blockDim.x >> 6) + wave) % a.copies) * (TMC_COHORT_COUNTERS + 4u * a.shells);
+}
+
+/* The kernel's arguments where a path between two cycles uses them: read
+ * through the argument block's pointer passed through an empty asm, so that
+ * no load is hoisted into the step loop, whose scalar registers hold the
+ * round keys. */
+__device__ __forceinline__ const LockArgs& args_here()
+{
+    typedef const __attribute__((address_space(4))) LockArgs* ConstArgs;
+    ConstArgs p = (ConstArgs)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const LockArgs*)p;
+}
+
+/* Photon state of a lane. */
+struct LockPhoton {
+    float x, y, z, u, v, w;
+    uint32_t x3; /* the last absorption's roulette word */
+};
+
+/* What a photon draws for one absorption. */
+struct Drawn {
+    float t, u, v, w; /* step length, then the direction it leaves with */
+    uint32_t x3;
+};
+
+template <uint32_t MATH>
+__device__ __forceinline__ Drawn lock_draw(uint32_t k, uint32_t c3k1, const tmc_philox_photon& pp,
+                                           const Physics& phys)
+{
+    const tmc_u32x4 r = block0_uniform(k, c3k1, pp, phys.keys);
+    Drawn d;
+    d.t = step_length<MATH>(r.x0);
+    d.u = tmc_u11(r.x1);
+    const float s = sin_polar<MATH>(d.u);
+    float sn, cs;
+    sincos_turn<MATH>(r.x2, &sn, &cs);
+    d.v = s * cs;
+    d.w = s * sn;
+    d.x3 = r.x3;
+    return d;
+}
+
+/* Moves the photon by its direction and the step length of d, and takes d's
+ * direction; returns the squared radius. */
+__device__ __forceinline__ float lock_move(LockPhoton& p, const Drawn& d)
+{
+    p.x = __builtin_fmaf(d.t, p.u, p.x);
+    p.y = __builtin_fmaf(d.t, p.v, p.y);
+    p.z = __builtin_fmaf(d.t, p.w, p.z);
+    p.u = d.u;
+    p.v = d.v;
+    p.w = d.w;
+    p.x3 = d.x3;
+    return __builtin_fmaf(p.z, p.z, __builtin_fmaf(p.y, p.y, p.x * p.x));
+}
+
+__device__ __forceinline__ void lock_add(const LaneTally& lt, uint32_t q, const Images& e)
+{
+    tally_add(lt, q, ((uint64_t)e.y << 32) | e.x, ((uint64_t)e.w << 32) | e.z);
+}
+
+/* Absorption k (wave-uniform) of every lane, its images in e. */
+template <uint32_t MATH>
+__device__ __forceinline__ void lock_step(LockPhoton& p, uint32_t k, uint32_t c3k1, const tmc_philox_photon& pp,
+                                          const Physics& phys, const LaneTally& lt, const Images& e)
+{
+    const float r2 = lock_move(p, lock_draw<MATH>(k, c3k1, pp, phys));
+    lock_add(lt, shell_index(r2, phys, lt.fmax), e);
+}
+
+/* Absorptions k and k + 1: both draws ahead of both moves, so that a wave has
+ * four independent chains of products to issue from (with few waves on a
+ * SIMD the products' latency is what a step costs). */
+template <uint32_t MATH>
+__device__ __forceinline__ void lock_step2(LockPhoton& p, uint32_t k, uint32_t c3k1, const tmc_philox_photon& pp,
+                                           const Physics& phys, const LaneTally& lt, const Images& e0,
+                                           const Images& e1)
+{
+    const Drawn a = lock_draw<MATH>(k, c3k1, pp, phys), b = lock_draw<MATH>(k + 1u, c3k1, pp, phys);
+    const float ra = lock_move(p, a), rb = lock_move(p, b);
+    bool sa, sb;
+    float fa = shell_coord_short(ra, phys, lt.fmax, &sa), fb = shell_coord_short(rb, phys, lt.fmax, &sb);
+    if (__builtin_expect(__ballot(!(sa && sb)) != 0, 0)) {
+        fa = (float)shell_index(ra, phys, lt.fmax);
+        fb = (float)shell_index(rb, phys, lt.fmax);
+    }
+    lock_add(lt, (uint32_t)fa, e0);
+    lock_add(lt, (uint32_t)fb, e1);
+}
+
+} // namespace
+
+/* (LockArgs must stay the only parameter: args_here) */
+template <uint32_t MATH>
+__global__ void __launch_bounds__(256) walk_lock(LockArgs a)
+{
+    extern __shared__ unsigned long long lds[];
+    const uint32_t lane = __lane_id();
+    const uint32_t wave = rfl32(threadIdx.x >> 6);
+    unsigned long long* const slot = lds + wave * lock_slot_words(a.shells);
+    for (uint32_t i = lane; i < lock_slot_words(a.shells); i += 64u)
+        slot[i] = 0;
+
+    Physics phys = {};
+    phys.albedo = a.albedo;
+    phys.spm = a.spm;
+    phys.shell_max = a.shell_max;
+    phys.key0 = (uint32_t)a.seed;
+    phys.key1 = (uint32_t)(a.seed >> 32);
+    set_derived<true>(phys);
+    LaneTally lt = { slot, tally_fmax(a.shell_max, lane & (TMC_LOCK_HOT - 1u)), ~0ull };
+    /* the photons' high index word is the launch's */
+    const uint32_t c3k1 = (uint32_t)(a.first_photon >> 32) ^ phys.key1;
+    const uint32_t k0 = a.k0, k1 = a.k1;
+    /* images: loaded with a vector offset of zero, so that they arrive in the
+     * registers the atomics want, and not through scalar ones */
+    const char* const table = (const char*)a.entry;
+    uint32_t zero = 0;
+    asm volatile("" : "+v"(zero));
+
+    /* photons of this level: the slice's, or this stripe's part of the list.
+     * A stripe's counts and photons are those of one XCD's workgroups, and few
+     * enough waves append to one count: additions to one address take 7 to
+     * 16 ns each (with one count, albedo 0.5 ran at a tenth of the rate).
+     * The batches of 64 go round the waves, which take about the same time for
+     * one; where a wave has many of them, it claims a few at a time, from the
+     * part of the slice of its XCD's waves (2^26 photons at default physics:
+     * 8.6 ms round the waves, 8.2 claimed; 2^20: 0.22 and 0.37 ms). */
+    const uint32_t stripe = blockIdx.x % a.stripes, waves_per_wg = blockDim.x >> 6;
+    uint32_t photons = a.photons, place = 0, at = 64u * (blockIdx.x * waves_per_wg + wave),
+             stride = 64u * waves_per_wg * gridDim.x, claimed = 0;
+    const bool claims = a.chunk != 0u;
+    if (a.level) {
+        const uint32_t n = a.in_count[stripe * TMC_LOCK_LINE];
+        photons = rfl32(n < a.in_cap ? n : a.in_cap);
+        place = stripe * a.in_cap;
+        at = 64u * (blockIdx.x / a.stripes * waves_per_wg + wave);
+        stride = 64u * waves_per_wg * ((gridDim.x - stripe + a.stripes - 1u) / a.stripes);
+    }
+    uint64_t interactions = 0, truncated = 0;
+    uint32_t room = TMC_LOCK_FLUSH_STEPS; /* steps to the next flush */
+
+    if (claims) {
+        /* range of this XCD's claims; `claimed`: where the current one ends */
+        const uint32_t x = blockIdx.x % TMC_LOCK_RANGES;
+        place = x * a.range;
+        photons = place >= a.photons ? 0u : a.photons - place < a.range ? a.photons - place : a.range;
+        stride = 64u;
+        at = 0;
+    }
+    for (;; at += stride) {
+        if (claims && at >= claimed) {
+            const LockArgs& c = args_here();
+            uint32_t got = 0;
+            if (lane == 0)
+                got = atomicAdd(c.cursor + blockIdx.x % TMC_LOCK_RANGES * TMC_LOCK_LINE, c.chunk);
+            at = rfl32(got);
+            claimed = at + c.chunk;
+        }
+        if (at >= photons)
+            break;
+        const uint64_t in = photons - at >= 64u ? ~0ull : (1ull << (photons - at)) - 1ull;
+        lt.deposit = in;
+        LockPhoton p = { 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 1.0f, ~0u };
+        tmc_philox_photon pp;
+        {
+            const LockArgs& c = args_here();
+            uint32_t off = place + at + lane;
+            if (c.level && __builtin_amdgcn_inverse_ballot_w64(in)) {
+                const uint32_t i = off;
+                off = c.in.photon[i];
+                p.x = c.in.state[0][i];
+                p.y = c.in.state[1][i];
+                p.z = c.in.state[2][i];
+                p.u = c.in.state[3][i];
+                p.v = c.in.state[4][i];
+                p.w = c.in.state[5][i];
+            }
+            const uint64_t photon = c.first_photon + off;
+            pp = tmc_philox_photon_init((uint32_t)photon, (uint32_t)(photon >> 32), phys.key0, phys.key1);
+        }
+        /* (lanes without a photon walk a stale one, their deposits masked) */
+        for (uint32_t k = k0; k != k1;) {
+            const uint32_t left = k1 - k, n = rfl32(left < room ? left : room);
+            room -= n;
+            const char* from = table + 16ull * k;
+            Images e0 = *(const Images*)(from + zero), e1 = *(const Images*)(from + 16u + zero);
+            const uint32_t stop = k + (n & ~1u);
+            for (; k != stop; k += 2u) {
+                from += 32u;
+                lock_step2<MATH>(p, k, c3k1, pp, phys, lt, e0, e1);
+                e0 = *(const Images*)(from + zero);
+                e1 = *(const Images*)(from + 16u + zero);
+            }
+            if (n & 1u) {
+                lock_step<MATH>(p, k, c3k1, pp, phys, lt, e0);
+                ++k;
+            }
+            if (room == 0u) {
+                const LockArgs& c = args_here();
+                lock_flush(slot, lock_block(c, wave) + TMC_COHORT_COUNTERS, c.shells, lane);
+                room = TMC_LOCK_FLUSH_STEPS;
+            }
+        }
+        interactions += (uint64_t)__popcll(in) * (k1 - k0);
+        const LockArgs& c = args_here();
+        uint64_t S = c.cut_ends ? in & __ballot(p.x3 < TMC_ROULETTE_KILL_R) : in;
+        if (c.cap_ends) {
+            truncated += (uint64_t)__popcll(S);
+            S = 0;
+        }
+        if (S != 0) {
+            /* the survivors go to the list */
+            const uint32_t n = (uint32_t)__popcll(S);
+            uint32_t base = 0;
+            if (lane == 0)
+                base = atomicAdd(c.out_count + stripe * TMC_LOCK_LINE, n);
+            base = rfl32(base);
+            const uint32_t to = base + mask_rank(S);
+            const bool lives = __builtin_amdgcn_inverse_ballot_w64(S);
+            uint32_t off = place + at + lane;
+            if (c.level && lives)
+                off = c.in.photon[off];
+            if (lives && to < c.out_cap) {
+                const uint32_t i = stripe * c.out_cap + to;
+                c.out.photon[i] = off;
+                c.out.state[0][i] = p.x;
+                c.out.state[1][i] = p.y;
+                c.out.state[2][i] = p.z;
+                c.out.state[3][i] = p.u;
+                c.out.state[4][i] = p.v;
+                c.out.state[5][i] = p.w;
+            }
+            if (base + n > c.out_cap && lane == 0)
+                atomicOr(lock_block(c, wave) + 2, TMC_LOCK_OVERFLOW);
+        }
+    }
+    const LockArgs& c = args_here();
+    unsigned long long* const block = lock_block(c, wave);
+    lock_flush(slot, block + TMC_COHORT_COUNTERS, c.shells, lane);
+    if (lane == 0) {
+        atomicAdd(block + 1, (unsigned long long)interactions);
+        if (truncated)
+            atomicAdd(block + 2, (unsigned long long)truncated);
+    }
+}
+
+namespace {
+
+using LockKernel = void (*)(LockArgs);
+
+LockKernel lock_kernel(uint32_t math) { return math == TMC_MATH_OWN ? walk_lock<TMC_MATH_OWN> : walk_lock<TMC_MATH_HARDWARE>; }
+
+} // namespace
+
+hipError_t launch_lock(uint32_t math, const LockArgs& a, uint32_t grid, uint32_t block, hipStream_t stream)
+{
+    hipLaunchKernelGGL(lock_kernel(math), dim3(grid), dim3(block), lock_lds_bytes(a.shells, block), stream, a);
+    return hipGetLastError();
+}
+
+hipError_t lock_occupancy(uint32_t math, uint32_t block, uint32_t shells, int* wg_per_cu)
+{
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(wg_per_cu, lock_kernel(math), (int)block,
+                                                        lock_lds_bytes(shells, block));
+}
+
+} // namespace tmc

@@ -111,9 +111,9 @@ double tmc::expected_interactions(const tmc_params* p, uint64_t kcap)
     return mean < 1.0 ? 1.0 : mean;
 }
 
-bool tmc::cohort_shape(uint64_t photons, double L, uint32_t shells, uint32_t cus, CohortShape* shape)
+bool tmc::cohort_shape(uint64_t photons, uint64_t most, double L, uint32_t shells, uint32_t cus, CohortShape* shape)
 {
-    if (photons == 0 || photons > TMC_COHORT_PHOTONS || cus == 0)
+    if (photons == 0 || photons > most || cus == 0)
         return false;
     /* one workgroup per compute unit, and cohorts as small as that allows: a
      * round of fewer photons is more absorptions of each, and costs little

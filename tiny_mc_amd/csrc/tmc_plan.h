@@ -61,19 +61,23 @@ struct CohortShape {
     uint32_t grid, copies; /* workgroups, and blocks of sums they flush into */
 };
 
-/* Largest run of the cohort walk.  It walks 0.9 to 1.9e11 absorptions/s
- * (default physics to albedo 0.99), a third of the lane-per-photon walk's rate
- * on a full chip, which that walk only comes near with several photons a lane:
- * both take time in proportion to a photon's absorptions, so the line is a
- * number of photons.  Measured, cohort walk against lane per photon: 2^15
- * photons 50 / 167 us at default physics, 167 / 1225 us at albedo 0.99; 2^17
- * 121 / 185 us and 544 / 1218 us; 2^18 208 / 213 us and 1008 / 1484 us; 2^19
- * 381 / 304 us and 1963 / 1880 us. */
-#define TMC_COHORT_PHOTONS (1ull << 17)
+/* Largest run of the cohort walk, with the analytic sampler and with the
+ * rejection sampler.  It walks 0.9 to 1.9e11 absorptions/s (default physics to
+ * albedo 0.99), a third of a full chip's rate, which the other walks only come
+ * near with several photons a lane: all take time in proportion to a photon's
+ * absorptions, so the lines are numbers of photons.  Measured, cohort walk
+ * against lockstep waves (walk_lock): 2^15 photons 48 / 59 us at default
+ * physics, 154 / 185 us at albedo 0.99; 49,152 62 / 66 us and 227 / 203 us;
+ * 2^16 71 / 71 us and 275 / 205 us; 2^17 119 / 89 us and 526 / 287 us.  Against
+ * lane per photon (walk_f32), which the rejection sampler keeps: 2^17 121 / 185
+ * us and 544 / 1218 us; 2^18 208 / 213 us and 1008 / 1484 us; 2^19 381 / 304 us
+ * and 1963 / 1880 us. */
+#define TMC_COHORT_PHOTONS 49152ull
+#define TMC_COHORT_PHOTONS_REJECTION (1ull << 17)
 
-/* The shape for `photons` photons of L expected absorptions each on cus
- * compute units; false if the run is not one for the cohort walk. */
-bool cohort_shape(uint64_t photons, double L, uint32_t shells, uint32_t cus, CohortShape* shape);
+/* The shape for `photons` photons (at most `most`) of about L absorptions each
+ * on cus compute units; false if the run is not one for the cohort walk. */
+bool cohort_shape(uint64_t photons, uint64_t most, double L, uint32_t shells, uint32_t cus, CohortShape* shape);
 
 /* Entries of the single run's weight table for these parameters and the
  * caller's request (tmc_options.weight_table; 0: none). */
