@@ -19,6 +19,16 @@
  * tenth of the work join the next larger class), and each group runs as a
  * launch of its own, one after the other on the same stream, with its own
  * chunk queue and cursor; the tallies and counters are shared.
+ *
+ * Lockstep: with the analytic sampler and automatic options the launches are
+ * those of tmc_lock.hip and tmc_cohort.hip instead: waves carry 64 photons of
+ * a set in lockstep to the first roulette, and append the tenth that survives
+ * to the set's places in a list; where a batch leaves enough of them they are
+ * walked to the second roulette the same way, and workgroups carry what is
+ * left to its end as cohorts.  Measured on MI355X, walk_multi -> this:
+ * 64 sets, 1.1e6 photons, planned, run and released 11.1 -> 3.9 ms; a kept
+ * plan of 512 sets, 5.6e7 photons 232 -> 144 ms (its lanes idle 1% of the
+ * steps, 24% before).
  */
 #include <hip/hip_runtime.h>
 
@@ -31,7 +41,9 @@
 
 #include "../../include/tiny_mc_gpu.h"
 #include "tmc_batch_internal.h"
+#include "tmc_cohort.h"
 #include "tmc_context.h"
+#include "tmc_internal.h"
 
 #define TMC_EXPORT extern "C" __attribute__((visibility("default")))
 
@@ -47,6 +59,40 @@ struct PassPlan {
     double work = 0.0;
     tmc::BatchArgs args;
 };
+
+/* The lockstep launches of a batch: its sets in parts of at most kPart
+ * photons, the parts in slices that share the lists. */
+struct LockSlice {
+    uint32_t first[3] = { 0, 0, 0 }, chunks[3] = { 0, 0, 0 }; /* queue of the first cycle, of the second, of the cohorts */
+};
+
+struct LockPlan {
+    bool on = false;
+    std::vector<LockSlice> slices;
+    uint32_t cycles = 1; /* walked in lockstep before the cohorts */
+    uint32_t grid = 0, cus = 0; /* workgroups of the lockstep launches and of the cohorts */
+    void* d = nullptr; /* parts, heads, chunks, lists and tables */
+    uint32_t* counts = nullptr; /* per part and list, then the cursors: TMC_LOCK_LINE words each */
+    uint64_t count_words = 0; /* of 64 bits */
+    uint32_t parts = 0;
+    tmc::LockSetArgs args;
+    tmc::PhotonList list[2];
+};
+
+/* Photons of a part (its survivors' places fit a slice). */
+constexpr uint64_t kPart = 1ull << 26;
+/* Places of a slice's first list: 0.9 GB. */
+constexpr uint64_t kSlicePlaces = 1ull << 25;
+/* Entries of the weight tables of a batch: 1 GB. */
+constexpr uint64_t kTableEntries = 1ull << 26;
+/* Expected survivors of a roulette from which on the next cycle is walked by
+ * lockstep waves too: with fewer, their 64-photon batches leave most of the
+ * chip's 8192 waves without one. */
+constexpr double kSecondCycle = 200000.0;
+/* Absorptions of a wave in its shortest chunk (a chunk of another set costs
+ * a flush of the slot, about 10 us). */
+constexpr double kChunkSteps = 512.0;
+constexpr uint32_t kLockBlock = 256;
 
 } // namespace
 
@@ -71,6 +117,7 @@ struct tmc_batch_plan {
     unsigned long long* h_counters = nullptr; /* pinned, TMC_BATCH_COUNTERS words */
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
+    LockPlan lock;
 };
 
 namespace {
@@ -92,20 +139,62 @@ void plan_free(tmc_batch_plan* p)
                 (void)hipGraphDestroy(graph);
         });
     }
-    for (void* d : { (void*)p->d_sets, (void*)p->d_chunks, (void*)p->d_tally, (void*)p->d_done, (void*)p->d_counters })
+    for (void* d : { (void*)p->d_sets, (void*)p->d_chunks, (void*)p->d_tally, (void*)p->d_done, (void*)p->d_counters,
+                     p->lock.d })
         tmc::release_device(d);
     tmc::release_host(p->h_tally);
     tmc::release_host(p->h_counters);
     delete p;
 }
 
+/* Enqueues the lockstep launches. */
+hipError_t enqueue_lock(const tmc_batch_plan* p, hipStream_t stream)
+{
+    const LockPlan& l = p->lock;
+    uint32_t* cursor = l.counts + 2ull * l.parts * TMC_LOCK_LINE;
+    for (const LockSlice& s : l.slices) {
+        for (uint32_t level = 0; level < 3u; ++level, cursor += TMC_LOCK_LINE) {
+            if (!s.chunks[level])
+                continue;
+            tmc::LockSetArgs a = l.args;
+            a.chunks += s.first[level];
+            a.nchunks = s.chunks[level];
+            a.cursor = cursor;
+            a.level = std::min(level, l.cycles);
+            if (a.level) {
+                a.in = l.list[a.level - 1u];
+                a.in_count = l.counts + (uint64_t)(a.level - 1u) * l.parts * TMC_LOCK_LINE;
+            }
+            hipError_t e;
+            if (level < 2u) {
+                a.out = l.list[level];
+                a.out_count = l.counts + (uint64_t)level * l.parts * TMC_LOCK_LINE;
+                const uint32_t per = kLockBlock / 64u;
+                e = tmc::launch_lock_sets(p->math, a, std::min(l.grid, (a.nchunks + per - 1u) / per), kLockBlock, stream);
+            } else {
+                e = tmc::launch_cohort_sets(p->math, a, std::min(l.cus, a.nchunks), stream);
+            }
+            if (e != hipSuccess)
+                return e;
+        }
+    }
+    return hipSuccess;
+}
+
 /* Enqueues clear + walk + copies on `stream`. */
-hipError_t enqueue_run(tmc_batch_plan* p, hipStream_t stream)
+hipError_t enqueue_run(tmc_batch_plan* p, bool lock, hipStream_t stream)
 {
     hipError_t e = tmc::launch_batch_clear(p->d_tally, p->tally_words, p->d_done, p->nsets, p->d_counters, stream);
     if (e != hipSuccess)
         return e;
-    for (uint32_t j = 0; j < p->npasses; ++j) {
+    if (lock) {
+        e = tmc::launch_clear((unsigned long long*)p->lock.counts, p->lock.count_words, stream);
+        if (e == hipSuccess)
+            e = enqueue_lock(p, stream);
+        if (e != hipSuccess)
+            return e;
+    }
+    for (uint32_t j = 0; j < p->npasses && !lock; ++j) {
         const PassPlan& q = p->pass[j];
         if (!q.nchunks)
             continue;
@@ -153,6 +242,202 @@ hipError_t launch_shape(const tmc_batch_plan* p, const tmc_batch_options* o, uin
         return hipSuccess;
     }
     return hipSuccess;
+}
+
+/* Roulettes of a weight table for n photons: three more than the last of
+ * them is expected to survive. */
+uint32_t cuts_for(double n)
+{
+    uint32_t cuts = 3;
+    for (; n >= 1.0 && cuts < TMC_COHORT_CUTS; n *= 0.1)
+        ++cuts;
+    return cuts;
+}
+
+/* Plans the lockstep launches of a batch; leaves p->lock off where they don't
+ * apply: with the rejection sampler, with a cap on the absorptions, where the
+ * caller chose a launch shape, where fewer than 5 waves' sums fit a SIMD's
+ * share of LDS (tmc_api.cpp's line), and where the weight tables or a first
+ * cycle are longer than is worth laying out.  TMC_OK, or TMC_E_HIP. */
+int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_batch_options* o, uint64_t kcap,
+              const std::vector<tmc::BatchSet>& hs, tmc_batch_plan* p)
+{
+    LockPlan& l = p->lock;
+    if (o->sampler != TMC_SAMPLER_ANALYTIC || o->block || o->waves_per_simd || o->copies || o->chunk_work
+        || kcap != 0xFFFFFFFFull || p->shells_max > 450u || p->photons == 0)
+        return TMC_OK;
+
+    /* the sets' cadences and tables, and their parts */
+    struct Part {
+        uint32_t set;
+        uint64_t first, count; /* photons of the set */
+    };
+    struct Cadence {
+        uint32_t k1, k2;
+    };
+    std::vector<tmc::LockSet> ls;
+    std::vector<Part> parts;
+    std::vector<Cadence> cad(nsets);
+    l.cycles = 0.1 * (double)p->photons >= kSecondCycle ? 2u : 1u;
+    uint64_t entries = 0;
+    double steps = 0.0; /* of 64 photons, in the first cycles */
+    for (uint32_t i = 0; i < nsets; ++i) {
+        const uint64_t n = sets[i].params.photons;
+        if (n == 0)
+            continue;
+        if (!tmc::weight_cadence(&sets[i].params, 1u << 20, &cad[i].k1, &cad[i].k2))
+            return TMC_OK;
+        const uint32_t cuts = std::max(cuts_for((double)n), l.cycles + 2u);
+        /* (later cycles can be a step longer than the second; two entries are
+         * read ahead of the last) */
+        const uint64_t room = cad[i].k1 + (uint64_t)(cuts - 1u) * (cad[i].k2 + 2u) + 64u;
+        tmc::LockSet s;
+        std::memset(&s, 0, sizeof s);
+        s.seed = hs[i].seed;
+        s.tally = hs[i].tally_offset;
+        s.entry = entries;
+        s.albedo = hs[i].albedo;
+        s.spm = hs[i].spm;
+        s.shell_max = hs[i].shell_max;
+        s.shells = hs[i].shells;
+        s.head = i;
+        s.entries = (uint32_t)room;
+        s.cuts = cuts;
+        entries += room + 2u;
+        if (entries > kTableEntries)
+            return TMC_OK;
+        for (uint64_t done = 0; done < n;) {
+            s.first_photon = hs[i].first_photon + done;
+            const uint64_t count =
+                std::min<uint64_t>(std::min<uint64_t>(kPart, n - done), (1ull << 32) - (s.first_photon & 0xFFFFFFFFull));
+            parts.push_back({ i, done, count });
+            ls.push_back(s);
+            s.cuts = 0; /* the first part builds the table */
+            done += count;
+            steps += (double)cad[i].k1 * std::ceil((double)count / 64.0);
+        }
+    }
+    if (parts.size() > 1u << 20)
+        return TMC_OK;
+    l.parts = (uint32_t)parts.size();
+
+    /* launch shape */
+    int per_cu = 0;
+    if (tmc::lock_sets_occupancy(p->math, kLockBlock, p->shells_max, &per_cu) != hipSuccess)
+        return TMC_E_HIP;
+    if (per_cu <= 0)
+        return TMC_OK;
+    l.cus = (uint32_t)c->compute_units;
+    l.grid = (uint32_t)per_cu * l.cus;
+
+    /* slices, places and queues: chunks of a wave's 32nd of the work, longest first */
+    const double target = std::max(kChunkSteps, steps / ((double)l.grid * (kLockBlock / 64u)) / 32.0);
+    struct Chunk {
+        double steps;
+        tmc::LockChunk chunk;
+    };
+    std::vector<tmc::LockChunk> queue;
+    uint64_t places[2] = { 0, 0 };
+    for (size_t i = 0; i < parts.size();) {
+        LockSlice slice;
+        uint64_t used[2] = { 0, 0 };
+        std::vector<Chunk> chunks[3];
+        auto cut = [&](uint32_t level, uint32_t part, uint64_t n, double cycle, double each) {
+            const uint64_t batches = std::max<uint64_t>(1, (uint64_t)std::min(1e6, std::ceil(each / cycle)));
+            for (uint64_t first = 0; first < n; first += 64u * batches) {
+                const uint32_t count = (uint32_t)std::min<uint64_t>(64u * batches, n - first);
+                chunks[level].push_back(
+                    { cycle * std::ceil((double)count / 64.0), { part, (uint32_t)first, count, 0u } });
+            }
+        };
+        for (; i < parts.size(); ++i) {
+            /* places for an eighth of the photons and a slack, where a tenth
+             * survive, and for a 64th after the second roulette */
+            const uint64_t n = parts[i].count;
+            const uint32_t cap[2] = { (uint32_t)(n / 8u + 64u), (uint32_t)(n / 64u + 64u) };
+            if (used[0] && used[0] + cap[0] > kSlicePlaces)
+                break;
+            const Cadence& k = cad[parts[i].set];
+            for (uint32_t w = 0; w < 2u; ++w) {
+                ls[i].place[w] = (uint32_t)used[w];
+                ls[i].cap[w] = cap[w];
+                used[w] += cap[w];
+            }
+            cut(0, (uint32_t)i, n, (double)k.k1, target);
+            if (l.cycles > 1u)
+                cut(1, (uint32_t)i, cap[0], (double)k.k2, target);
+            cut(2, (uint32_t)i, cap[l.cycles - 1u], (double)k.k2, 1.0);
+        }
+        for (uint32_t level = 0; level < 3u; ++level) {
+            std::stable_sort(chunks[level].begin(), chunks[level].end(),
+                             [](const Chunk& x, const Chunk& y) { return x.steps > y.steps; });
+            slice.first[level] = (uint32_t)queue.size();
+            slice.chunks[level] = (uint32_t)chunks[level].size();
+            for (const Chunk& ch : chunks[level])
+                queue.push_back(ch.chunk);
+            if (queue.size() > 1u << 26)
+                return TMC_OK;
+        }
+        for (uint32_t w = 0; w < 2u; ++w)
+            places[w] = std::max(places[w], used[w]);
+        l.slices.push_back(slice);
+    }
+    if (l.cycles < 2u)
+        places[1] = 0;
+
+    /* one block of device memory; what the host writes comes first */
+    uint64_t bytes = 0;
+    auto take = [&](uint64_t n) {
+        const uint64_t at = bytes;
+        bytes += (n + 255u) / 256u * 256u;
+        return at;
+    };
+    const uint64_t at_sets = take(ls.size() * sizeof(tmc::LockSet));
+    const uint64_t at_queue = take(queue.size() * sizeof(tmc::LockChunk));
+    const uint64_t written = bytes;
+    const uint64_t at_heads = take(nsets * sizeof(tmc::CohortHead));
+    l.count_words = (2ull * l.parts + 3ull * l.slices.size()) * TMC_LOCK_LINE / 2u;
+    const uint64_t at_counts = take(l.count_words * 8u);
+    const uint64_t at_entries = take(entries * 16u);
+    const uint64_t at_lists = take(28u * (places[0] + places[1]));
+    if (hipMalloc(&l.d, bytes) != hipSuccess) {
+        l.d = nullptr;
+        (void)hipGetLastError();
+        return TMC_OK;
+    }
+    std::vector<char> stage(written);
+    std::memcpy(stage.data() + at_sets, ls.data(), ls.size() * sizeof(tmc::LockSet));
+    std::memcpy(stage.data() + at_queue, queue.data(), queue.size() * sizeof(tmc::LockChunk));
+    char* const d = (char*)l.d;
+    float* at = (float*)(d + at_lists);
+    for (uint32_t w = 0; w < 2u; ++w) {
+        l.list[w].photon = (uint32_t*)at;
+        at += places[w];
+        for (float*& f : l.list[w].state) {
+            f = at;
+            at += places[w];
+        }
+    }
+    l.counts = (uint32_t*)(d + at_counts);
+    tmc::LockSetArgs& a = l.args;
+    std::memset(&a, 0, sizeof a);
+    a.sets = (const tmc::LockSet*)(d + at_sets);
+    a.heads = (const tmc::CohortHead*)(d + at_heads);
+    a.chunks = (const tmc::LockChunk*)(d + at_queue);
+    a.entry = d + at_entries;
+    a.shells_max = p->shells_max;
+    a.tally = p->d_tally;
+    a.counters = p->d_counters;
+    hipError_t e = hipMemcpyAsync(d, stage.data(), written, hipMemcpyHostToDevice, c->stream);
+    /* (beside a resident serving kernel a plan is made without waiting for it,
+     * and keeps to walk_multi) */
+    if (e == hipSuccess)
+        l.on = tmc::unless_serving([&]() {
+            e = tmc::launch_weigh_sets(a.sets, l.parts, (tmc::CohortHead*)(d + at_heads), d + at_entries, c->stream);
+        });
+    if (e != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess)
+        return TMC_E_HIP;
+    return TMC_OK;
 }
 
 int plan_create_locked(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_batch_options* o,
@@ -293,13 +578,19 @@ int plan_create_locked(tmc::Context* c, const tmc_set* sets, uint32_t nsets, con
         a.done = p->d_done;
     }
 
+    const int lrc = plan_lock(c, sets, nsets, o, kcap, hs, p);
+    if (lrc != TMC_OK) {
+        plan_free(p);
+        return lrc;
+    }
+
     if (p->use_graph) {
         hipStream_t s = c->stream;
         if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) {
             plan_free(p);
             return TMC_E_HIP;
         }
-        const hipError_t e1 = enqueue_run(p, s);
+        const hipError_t e1 = enqueue_run(p, p->lock.on, s);
         const hipError_t e2 = hipStreamEndCapture(s, &p->graph);
         if (e1 != hipSuccess || e2 != hipSuccess
             || hipGraphInstantiate(&p->exec, p->graph, nullptr, nullptr, 0) != hipSuccess) {
@@ -311,19 +602,40 @@ int plan_create_locked(tmc::Context* c, const tmc_set* sets, uint32_t nsets, con
     return TMC_OK;
 }
 
+/* Runs the plan's launches once, by the lockstep walk or the other. */
+int plan_launch(tmc::Context* c, tmc_batch_plan* p, bool lock)
+{
+    if (hipEventRecord(c->ev_start, c->stream) != hipSuccess)
+        return TMC_E_HIP;
+    if (p->use_graph && lock == p->lock.on) {
+        if (hipGraphLaunch(p->exec, c->stream) != hipSuccess)
+            return TMC_E_HIP;
+    } else if (enqueue_run(p, lock, c->stream) != hipSuccess) {
+        return TMC_E_HIP;
+    }
+    if (hipEventRecord(c->ev_stop, c->stream) != hipSuccess)
+        return TMC_E_HIP;
+    return TMC_OK;
+}
+
 int plan_run_locked(tmc::Context* c, tmc_batch_plan* p, uint64_t* tallies, tmc_batch_stats* st)
 {
     const auto t0 = std::chrono::steady_clock::now();
-    if (hipEventRecord(c->ev_start, c->stream) != hipSuccess)
-        return TMC_E_HIP;
-    if (p->use_graph) {
-        if (hipGraphLaunch(p->exec, c->stream) != hipSuccess)
+    int rc = TMC_OK;
+    /* (the cohorts' workgroups need whole compute units, and would wait for a
+     * resident serving kernel) */
+    bool lock = p->lock.on && tmc::unless_serving([&]() { rc = plan_launch(c, p, true); });
+    for (;;) {
+        if (!lock)
+            rc = plan_launch(c, p, false);
+        if (rc != TMC_OK)
+            return rc;
+        if (hipStreamSynchronize(c->stream) != hipSuccess)
             return TMC_E_HIP;
-    } else if (enqueue_run(p, c->stream) != hipSuccess) {
-        return TMC_E_HIP;
+        if (!lock || p->h_counters[2] < TMC_LOCK_OVERFLOW)
+            break;
+        lock = false; /* a list had no room for a survivor */
     }
-    if (hipEventRecord(c->ev_stop, c->stream) != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess)
-        return TMC_E_HIP;
     float ms = 0.0f;
     if (hipEventElapsedTime(&ms, c->ev_start, c->ev_stop) != hipSuccess)
         return TMC_E_HIP;
@@ -487,7 +799,10 @@ TMC_EXPORT int tmc_batch_autotune(const tmc_set* sets, uint32_t nsets, const tmc
     auto time_on = [&](const std::vector<tmc_set>& r, double sc, const tmc_batch_options& o, double mult,
                        int reps) -> double {
         tmc_batch_options t = o;
-        t.chunk_work = (uint64_t)std::max(4096.0, mult * (double)auto_cw * sc);
+        /* (the automatic value as such: with automatic options throughout, the
+         * lockstep walk is the candidate that the others have to beat) */
+        if (mult != 1.0 || b0.chunk_work)
+            t.chunk_work = (uint64_t)std::max(4096.0, mult * (double)auto_cw * sc);
         tmc_batch_plan* plan = nullptr;
         if (tmc_batch_plan_create(r.data(), nsets, &t, &plan) != TMC_OK)
             return 1e300;

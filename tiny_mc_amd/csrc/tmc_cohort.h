@@ -28,6 +28,54 @@ struct PhotonList {
     float* state[6]; /* x, y, z, then the direction */
 };
 
+/* A parameter set of a batch, or a part of its photons, as the set kernels
+ * read it.  The photons' high index word is one for all of them. */
+struct LockSet {
+    uint64_t seed; /* Philox key */
+    uint64_t first_photon; /* stream index of its photon 0 */
+    uint64_t tally; /* word offset of the set's 4*shells sums */
+    uint64_t entry; /* offset of the set's weight table, in entries */
+    float albedo, spm, shell_max; /* as WalkArgs */
+    uint32_t shells;
+    uint32_t head; /* the set's CohortHead */
+    uint32_t entries, cuts; /* room of the weight table, and roulettes wanted (0: an earlier part builds it) */
+    uint32_t place[2], cap[2]; /* its places in the two survivor lists */
+    uint32_t pad;
+};
+static_assert(sizeof(LockSet) == 80, "LockSet layout");
+
+/* The roulettes of a set's weight table, built on the device: the i-th follows
+ * absorption cut[i] - 1; w_end is the weight with which a survivor of the last
+ * one goes on. */
+struct CohortHead {
+    uint32_t ncuts;
+    float w_end;
+    uint32_t cut[TMC_COHORT_CUTS];
+};
+
+/* Photons first .. first + count - 1 of a set (level 0), or of its places in
+ * the list of its level. */
+struct LockChunk {
+    uint32_t set, first, count, pad;
+};
+
+/* One level of a batch: sets, queue, and what the launches of a run share. */
+struct LockSetArgs {
+    const LockSet* sets;
+    const CohortHead* heads;
+    const void* entry; /* pool of pairs of images */
+    const LockChunk* chunks;
+    uint32_t nchunks;
+    uint32_t* cursor; /* of this launch */
+    uint32_t level; /* roulettes the photons of the queue have survived */
+    uint32_t shells_max;
+    PhotonList in, out; /* level > 0: the survivors of `level` roulettes; a lock level: those of one more */
+    const uint32_t* in_count; /* photons appended to a set's places, TMC_LOCK_LINE words apart */
+    uint32_t* out_count;
+    unsigned long long* tally; /* tally pool */
+    unsigned long long* counters; /* [1] interactions, [2] truncated (TMC_LOCK_OVERFLOW), [4] idle lane-steps */
+};
+
 struct CohortArgs {
     uint64_t seed; /* Philox key */
     uint64_t first_photon; /* photon index of cohort 0's first photon */
@@ -106,6 +154,15 @@ size_t lock_lds_bytes(uint32_t shells, uint32_t block);
 /* Resident workgroups per CU of walk_lock. */
 hipError_t lock_occupancy(uint32_t math, uint32_t block, uint32_t shells, int* wg_per_cu);
 hipError_t launch_lock(uint32_t math, const LockArgs& a, uint32_t grid, uint32_t block, hipStream_t stream);
+
+/* The same for the sets of a batch: a level by lockstep waves (0 or 1), and
+ * the survivors of a.level roulettes by cohorts, to their end.  Analytic
+ * sampler, no cap. */
+hipError_t lock_sets_occupancy(uint32_t math, uint32_t block, uint32_t shells_max, int* wg_per_cu);
+hipError_t launch_lock_sets(uint32_t math, const LockSetArgs& a, uint32_t grid, uint32_t block, hipStream_t stream);
+hipError_t launch_cohort_sets(uint32_t math, const LockSetArgs& a, uint32_t grid, hipStream_t stream);
+/* Builds the weight tables of nsets sets. */
+hipError_t launch_weigh_sets(const LockSet* sets, uint32_t nsets, CohortHead* heads, void* entry, hipStream_t stream);
 
 /* Converts n weights (host memory) to table entries of 16 bytes, zeroes
  * `counters` 32-bit words at `counter`, and notes the real time at *start

@@ -392,39 +392,59 @@ __device__ __forceinline__ void move_chain(float& x, float& u, const float4* t, 
  * the next. */
 #define TMC_COHORT_AHEAD 256u
 
-template <uint32_t SAMPLER, uint32_t MATH>
-__global__ void __launch_bounds__(1024) walk_cohort(CohortArgs a)
-{
-    extern __shared__ unsigned long long lds_words[];
-    Images* const built = (Images*)lds_words;
-    unsigned long long* const lds = lds_words + 2u * (size_t)a.build;
-    float* const rounds = (float*)(lds + cohort_tally_words(a.shells));
-    float* const states = rounds + 2u * TMC_COHORT_ROUND;
-    unsigned long long* const surv = (unsigned long long*)(states + 2u * TMC_COHORT_STATE);
-    uint32_t* const cuts = (uint32_t*)(surv + 2);
-    uint32_t* const flag = cuts + TMC_COHORT_CUTS; /* finish_run's word, then the start time */
+namespace {
 
+/* LDS of a workgroup. */
+struct CohortLds {
+    Images* built; /* the weight table, where the kernel builds it */
+    unsigned long long* tally;
+    float *rounds, *states;
+    unsigned long long* surv;
+    uint32_t *cuts, *flag; /* flag: finish_run's word, then the start time */
+    __device__ __forceinline__ CohortLds(unsigned long long* words, uint32_t shells, uint32_t build)
+    {
+        built = (Images*)words;
+        tally = words + 2u * (size_t)build;
+        rounds = (float*)(tally + cohort_tally_words(shells));
+        states = rounds + 2u * TMC_COHORT_ROUND;
+        surv = (unsigned long long*)(states + 2u * TMC_COHORT_STATE);
+        cuts = (uint32_t*)(surv + 2);
+        flag = cuts + TMC_COHORT_CUTS;
+    }
+};
+
+/* What a workgroup walks: the cohorts first, first + stride, ... of `photons`
+ * photons, at `place` of the list if there is one. */
+struct CohortTask {
+    uint32_t group, stride, photons, place;
+};
+
+/* What a wave counts (the first mover's counts are the workgroup's). */
+struct CohortCounts {
+    uint64_t interactions, truncated;
+    uint64_t idle; /* lanes of the rows without an absorption (batches) */
+    bool flushed; /* sums have been moved to `tally` */
+};
+
+/* Walks a task's cohorts.  a.cut is in LDS (l.cuts); a.build: the weigher's
+ * first weights are in `weights`. */
+template <uint32_t SAMPLER, uint32_t MATH, bool BATCH>
+__device__ __forceinline__ void walk_cohorts(const CohortArgs& a, const PhotonList& list, CohortTask task,
+                                             const CohortLds& l,
+                                             unsigned long long* tally, float (&weights)[TMC_COHORT_AHEAD / 64u],
+                                             CohortCounts& counts)
+{
+    Images* const built = l.built;
+    unsigned long long* const lds = l.tally;
+    float *const rounds = l.rounds, *const states = l.states;
+    unsigned long long* const surv = l.surv;
+    const uint32_t* const cuts = l.cuts;
     const uint32_t lane = __lane_id();
     const uint32_t wave = rfl32(threadIdx.x >> 6);
-    const uint32_t drawing = a.drawing; /* waves 0 .. drawing - 1 draw and tally, then come the movers */
+    const uint32_t drawing = a.drawing;
     const bool weigher = wave >= drawing + a.moving;
-    if (threadIdx.x == 0)
-        *(unsigned long long*)(flag + 2) = __builtin_amdgcn_s_memrealtime();
-
-    for (uint32_t i = threadIdx.x; i < cohort_tally_words(a.shells); i += blockDim.x)
-        lds[i] = 0;
-    if (threadIdx.x < TMC_COHORT_CUTS)
-        cuts[threadIdx.x] = a.cut[threadIdx.x];
     const uint32_t ncuts = a.ncuts;
-    /* the weigher's next weights, on their way from the host's memory */
-    float weights[TMC_COHORT_AHEAD / 64u];
     uint32_t weighed = 0;
-    if (weigher) {
-#pragma unroll
-        for (uint32_t i = 0; i < TMC_COHORT_AHEAD / 64u; ++i)
-            weights[i] = 64u * i + lane < a.entries ? a.weight[64u * i + lane] : 0.0f;
-    }
-    __syncthreads();
 
     Physics phys = {};
     phys.albedo = a.albedo;
@@ -434,23 +454,11 @@ __global__ void __launch_bounds__(1024) walk_cohort(CohortArgs a)
     phys.key1 = (uint32_t)(a.seed >> 32);
     set_derived(phys);
     const LaneTally lt = { lds, tally_fmax(a.shell_max, lane & (TMC_COHORT_HOT - 1)), ~0ull };
-    unsigned long long* const tally =
-        a.work + (size_t)(blockIdx.x % a.copies) * (TMC_COHORT_COUNTERS + 4u * a.shells) + TMC_COHORT_COUNTERS;
-    bool flushed = false;
 
     /* the schedule: every wave steps the same one */
-    const bool listed = a.list.photon != nullptr;
-    uint32_t group = blockIdx.x, stride = gridDim.x; /* next cohort, and from one to the next */
-    uint32_t photons = (uint32_t)a.photons, place = 0; /* place: of the stripe's first photon in the list */
-    if (listed) {
-        /* (at least as many workgroups as stripes, or one stripe) */
-        const uint32_t stripe = blockIdx.x % a.stripes;
-        const uint32_t n = a.list_count[stripe * TMC_LOCK_LINE];
-        photons = rfl32(n < a.list_cap ? n : a.list_cap);
-        place = stripe * a.list_cap;
-        group = blockIdx.x / a.stripes;
-        stride = (gridDim.x - stripe + a.stripes - 1u) / a.stripes;
-    }
+    const bool listed = list.photon != nullptr;
+    uint32_t group = task.group; /* next cohort */
+    const uint32_t photons = task.photons, place = task.place;
     const uint32_t groups = (photons + a.group - 1u) / a.group;
     Round prev = {}, cur = {}, next = {};
     bool alive = false;
@@ -469,11 +477,6 @@ __global__ void __launch_bounds__(1024) walk_cohort(CohortArgs a)
     for (uint32_t j = 0; j < M; ++j)
         image[j] = image_next[j] = Images{ 0u, 0u, 0u, 0u };
     float x = 0.0f, u = 0.0f;
-    uint64_t interactions = 0, truncated = 0;
-
-    /* the movers' chain is what a round waits for */
-    if (wave >= drawing && !weigher)
-        __builtin_amdgcn_s_setprio(3);
 
     for (;;) {
         /* positions of the lane's item of the previous round, on their way
@@ -500,7 +503,7 @@ __global__ void __launch_bounds__(1024) walk_cohort(CohortArgs a)
             const uint64_t all = cur.P == 64u ? ~0ull : (1ull << cur.P) - 1ull;
             S = cur.flags & R_CUT ? rfl64(surv[par]) : all;
             if (cur.flags & R_CAP) {
-                truncated += (uint64_t)__popcll(S);
+                counts.truncated += (uint64_t)__popcll(S);
                 S = 0;
             }
             const uint64_t go = cur.flags & R_LAST ? 0ull : S;
@@ -526,14 +529,14 @@ __global__ void __launch_bounds__(1024) walk_cohort(CohortArgs a)
             base = a.first_photon;
             k = 0;
             if (listed) {
-                pid = a.list.photon[place + off + (pid < P ? pid : 0u)];
+                pid = list.photon[place + off + (pid < P ? pid : 0u)];
                 k = rfl32(cuts[a.seg0 - 1u]);
             } else {
                 base += off;
             }
             next.at = place + off;
             seg = a.seg0;
-            group += stride;
+            group += task.stride;
             next.flags = R_FRESH;
             alive = true;
             changed = true;
@@ -594,7 +597,7 @@ __global__ void __launch_bounds__(1024) walk_cohort(CohortArgs a)
                 if (since_flush >= TMC_COHORT_FLUSH - 64u * TMC_COHORT_ROWS) {
                     cohort_flush(lds, tally, a.shells, wave * 64u + lane, drawing * 64u);
                     since_flush = 0;
-                    flushed = true;
+                    counts.flushed = true;
                 }
             }
             /* ---- draw the next round (lanes past its items draw unused ones) ---- */
@@ -640,15 +643,20 @@ __global__ void __launch_bounds__(1024) walk_cohort(CohortArgs a)
                 x = 0.0f;
                 u = c == 2u ? 1.0f : 0.0f;
                 if (listed && in) {
-                    x = a.list.state[c][cur.at + p];
-                    u = a.list.state[3u + c][cur.at + p];
+                    x = list.state[c][cur.at + p];
+                    u = list.state[3u + c][cur.at + p];
                 }
             } else if ((cur.flags & R_PACKED) && in) {
                 x = from[c * 64u + p];
                 u = from[(3u + c) * 64u + p];
             }
-            if (wave == drawing)
-                interactions += (uint64_t)cur.P * cur.T;
+            if (wave == drawing) {
+                counts.interactions += (uint64_t)cur.P * cur.T;
+                if constexpr (BATCH) {
+                    const uint32_t rows = (((cur.T - 1u) << cur.lg) >> 6) + 1u;
+                    counts.idle += 64ull * rows - (uint64_t)cur.P * cur.T;
+                }
+            }
             if (in) {
                 const float* const t = rounds + par * TMC_COHORT_ROUND + p * row_floats(cur.lg);
                 move_chain(x, u, (const float4*)t, (float4*)(t + (1u + c) * TMC_COHORT_ARRAY), cur.T);
@@ -682,10 +690,13 @@ __global__ void __launch_bounds__(1024) walk_cohort(CohortArgs a)
                     ph.weight = a.w_end;
                 }
                 while (__ballot(live) != 0) {
-                    interactions += (uint64_t)__popcll(__ballot(live && absorbs<SAMPLER>(ph)));
+                    const uint32_t n = (uint32_t)__popcll(__ballot(live && absorbs<SAMPLER>(ph)));
+                    counts.interactions += n;
+                    if constexpr (BATCH)
+                        counts.idle += 64u - n;
                     if (live)
                         live = step<SAMPLER, MATH>(ph, phys, lt);
-                    truncated += (uint64_t)__popcll(__ballot(live && ph.k >= a.kcap));
+                    counts.truncated += (uint64_t)__popcll(__ballot(live && ph.k >= a.kcap));
                     live = live && ph.k < a.kcap;
                 }
             }
@@ -695,12 +706,188 @@ __global__ void __launch_bounds__(1024) walk_cohort(CohortArgs a)
         par ^= 1u;
         weighed += TMC_COHORT_AHEAD;
     }
-    finish_run(a, lds, flag, wave == drawing && lane == 0, interactions, truncated, flushed);
+}
+
+} // namespace
+
+template <uint32_t SAMPLER, uint32_t MATH>
+__global__ void __launch_bounds__(1024) walk_cohort(CohortArgs a)
+{
+    extern __shared__ unsigned long long lds_words[];
+    const CohortLds l(lds_words, a.shells, a.build);
+
+    const uint32_t lane = __lane_id();
+    const uint32_t wave = rfl32(threadIdx.x >> 6);
+    const uint32_t drawing = a.drawing; /* waves 0 .. drawing - 1 draw and tally, then come the movers */
+    const bool weigher = wave >= drawing + a.moving;
+    if (threadIdx.x == 0)
+        *(unsigned long long*)(l.flag + 2) = __builtin_amdgcn_s_memrealtime();
+
+    for (uint32_t i = threadIdx.x; i < cohort_tally_words(a.shells); i += blockDim.x)
+        l.tally[i] = 0;
+    if (threadIdx.x < TMC_COHORT_CUTS)
+        l.cuts[threadIdx.x] = a.cut[threadIdx.x];
+    /* the weigher's next weights, on their way from the host's memory */
+    float weights[TMC_COHORT_AHEAD / 64u];
+    if (weigher) {
+#pragma unroll
+        for (uint32_t i = 0; i < TMC_COHORT_AHEAD / 64u; ++i)
+            weights[i] = 64u * i + lane < a.entries ? a.weight[64u * i + lane] : 0.0f;
+    }
+    __syncthreads();
+
+    CohortTask task = { blockIdx.x, gridDim.x, (uint32_t)a.photons, 0u };
+    if (a.list.photon) {
+        /* (at least as many workgroups as stripes, or one stripe) */
+        const uint32_t stripe = blockIdx.x % a.stripes;
+        const uint32_t n = a.list_count[stripe * TMC_LOCK_LINE];
+        task.photons = rfl32(n < a.list_cap ? n : a.list_cap);
+        task.place = stripe * a.list_cap;
+        task.group = blockIdx.x / a.stripes;
+        task.stride = (gridDim.x - stripe + a.stripes - 1u) / a.stripes;
+    }
+    unsigned long long* const tally =
+        a.work + (size_t)(blockIdx.x % a.copies) * (TMC_COHORT_COUNTERS + 4u * a.shells) + TMC_COHORT_COUNTERS;
+    CohortCounts counts = { 0, 0, 0, false };
+    /* the movers' chain is what a round waits for */
+    if (wave >= drawing && !weigher)
+        __builtin_amdgcn_s_setprio(3);
+    walk_cohorts<SAMPLER, MATH, false>(a, a.list, task, l, tally, weights, counts);
+    finish_run(a, l.tally, l.flag, wave == drawing && lane == 0, counts.interactions, counts.truncated, counts.flushed);
+}
+
+/* Waves that draw and that move in a workgroup of a batch: cohorts of 64. */
+#define TMC_COHORT_SETS_MOVING 3u
+#define TMC_COHORT_SETS_DRAWING 13u
+
+/* The rest of a batch's photons, from their a.level-th roulette to the end:
+ * each workgroup claims a run of at most 64 places of a set's part of the
+ * list, walks the photons there as one cohort, and adds its sums to the
+ * set's. */
+template <uint32_t MATH>
+__global__ void __launch_bounds__(1024) walk_cohort_sets(LockSetArgs a)
+{
+    extern __shared__ unsigned long long lds_words[];
+    const CohortLds l(lds_words, a.shells_max, 0u);
+    const uint32_t lane = __lane_id();
+    const uint32_t wave = rfl32(threadIdx.x >> 6);
+    for (uint32_t i = threadIdx.x; i < cohort_tally_words(a.shells_max); i += blockDim.x)
+        l.tally[i] = 0;
+    CohortCounts counts = { 0, 0, 0, false };
+    float weights[TMC_COHORT_AHEAD / 64u] = {};
+    const uint32_t in = a.level - 1u;
+    if (wave >= TMC_COHORT_SETS_DRAWING)
+        __builtin_amdgcn_s_setprio(3);
+    for (;;) {
+        __syncthreads(); /* the last task's flush, and its claim's readers */
+        if (threadIdx.x == 0) {
+            /* the next chunk with photons in it */
+            uint32_t got, n = 0;
+            do {
+                got = atomicAdd(a.cursor, 1u);
+                if (got < a.nchunks) {
+                    const LockChunk& ch = a.chunks[got];
+                    const uint32_t cap = a.sets[ch.set].cap[in], filled = a.in_count[ch.set * TMC_LOCK_LINE];
+                    n = filled < cap ? filled : cap;
+                    n = ch.first < n ? n - ch.first : 0u;
+                    n = n < ch.count ? n : ch.count;
+                }
+            } while (got < a.nchunks && n == 0u);
+            l.flag[0] = got;
+            l.flag[1] = n;
+        }
+        __syncthreads();
+        const uint32_t got = rfl32(l.flag[0]), n = rfl32(l.flag[1]);
+        if (got >= a.nchunks)
+            break;
+        const LockChunk& ch = a.chunks[got];
+        const LockSet& s = a.sets[rfl32(ch.set)];
+        const CohortHead& h = a.heads[s.head];
+        if (threadIdx.x < TMC_COHORT_CUTS)
+            l.cuts[threadIdx.x] = h.cut[threadIdx.x];
+        CohortArgs c = {};
+        c.seed = rfl64(s.seed);
+        c.first_photon = rfl64(s.first_photon);
+        c.albedo = s.albedo;
+        c.spm = s.spm;
+        c.shell_max = s.shell_max;
+        c.shells = rfl32(s.shells);
+        c.kcap = ~0u;
+        c.group = 64u;
+        c.drawing = TMC_COHORT_SETS_DRAWING;
+        c.moving = TMC_COHORT_SETS_MOVING;
+        c.entry = (const Images*)a.entry + rfl64(s.entry);
+        c.ncuts = rfl32(h.ncuts);
+        c.w_end = h.w_end;
+        c.seg0 = a.level;
+        unsigned long long* const tally = a.tally + rfl64(s.tally);
+        __syncthreads();
+        walk_cohorts<0u, MATH, true>(c, a.in, { 0u, 1u, n, s.place[in] + ch.first }, l, tally, weights, counts);
+        __syncthreads();
+        cohort_flush(l.tally, tally, c.shells, threadIdx.x, blockDim.x);
+    }
+    if (wave == TMC_COHORT_SETS_DRAWING && lane == 0) {
+        atomicAdd(a.counters + 1, (unsigned long long)counts.interactions);
+        atomicAdd(a.counters + 4, (unsigned long long)counts.idle);
+        if (counts.truncated)
+            atomicAdd(a.counters + 2, (unsigned long long)counts.truncated);
+    }
+}
+
+/* The weight table of a set: one wave walks the recurrence W[k+1] = RN(W[k] a),
+ * every lane alike, 64 absorptions at a time, and lane i keeps the i-th weight.
+ * (8 ns an absorption; on the host 1.3 ns, but for one set after the other.) */
+__global__ void __launch_bounds__(64) weigh_sets(const LockSet* sets, CohortHead* heads, Images* pool)
+{
+    const LockSet& s = sets[blockIdx.x];
+    if (s.cuts == 0u)
+        return;
+    CohortHead& h = heads[s.head];
+    Images* const entry = pool + s.entry;
+    const uint32_t lane = __lane_id();
+    const float a = s.albedo;
+    float w = 1.0f;
+    uint32_t n = 0;
+    for (uint32_t k = 0; n < s.cuts && k < s.entries; k += 64u) {
+        float v = w, mine = w;
+        uint32_t me = lane;
+        asm volatile("" : "+v"(me)); /* (64 comparisons kept from one pass for the next would not fit) */
+#pragma unroll
+        for (uint32_t i = 0; i < 64u; ++i) {
+            if (me == i)
+                mine = v;
+            v = v * a;
+        }
+        if (v < 0.001f) {
+            /* a roulette among them (the weight never grows between two) */
+            v = w;
+            for (uint32_t i = 0; i < 64u && n < s.cuts && k + i < s.entries; ++i) {
+                if (lane == i)
+                    mine = v;
+                v = v * a;
+                if (v < 0.001f) {
+                    v = v / 0.1f;
+                    if (lane == 0)
+                        h.cut[n] = k + i + 1u;
+                    ++n;
+                }
+            }
+        }
+        w = v;
+        if (k + lane < s.entries)
+            entry[k + lane] = images_of(mine);
+    }
+    if (lane == 0) {
+        h.ncuts = n;
+        h.w_end = w;
+    }
 }
 
 namespace {
 
 using CohortKernel = void (*)(CohortArgs);
+
+using SetsKernel = void (*)(LockSetArgs);
 
 CohortKernel cohort_kernel(uint32_t sampler, uint32_t math)
 {
@@ -725,6 +912,20 @@ hipError_t launch_cohort(uint32_t sampler, uint32_t math, const CohortArgs& a, u
 {
     hipLaunchKernelGGL(cohort_kernel(sampler, math), dim3(grid), dim3(block), cohort_lds_bytes_of(a.shells, a.build),
                        stream, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_cohort_sets(uint32_t math, const LockSetArgs& a, uint32_t grid, hipStream_t stream)
+{
+    const SetsKernel k = math == TMC_MATH_OWN ? walk_cohort_sets<TMC_MATH_OWN> : walk_cohort_sets<TMC_MATH_HARDWARE>;
+    hipLaunchKernelGGL(k, dim3(grid), dim3(64u * (TMC_COHORT_SETS_DRAWING + TMC_COHORT_SETS_MOVING)),
+                       cohort_lds_bytes_of(a.shells_max, 0u), stream, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_weigh_sets(const LockSet* sets, uint32_t nsets, CohortHead* heads, void* entry, hipStream_t stream)
+{
+    hipLaunchKernelGGL(weigh_sets, dim3(nsets), dim3(64), 0, stream, sets, heads, (Images*)entry);
     return hipGetLastError();
 }
 

@@ -110,12 +110,13 @@ __device__ __forceinline__ unsigned long long* lock_block(const LockArgs& a, uin
  * through the argument block's pointer passed through an empty asm, so that
  * no load is hoisted into the step loop, whose scalar registers hold the
  * round keys. */
-__device__ __forceinline__ const LockArgs& args_here()
+template <class Args>
+__device__ __forceinline__ const Args& args_here()
 {
-    typedef const __attribute__((address_space(4))) LockArgs* ConstArgs;
+    typedef const __attribute__((address_space(4))) Args* ConstArgs;
     ConstArgs p = (ConstArgs)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(p));
-    return *(const LockArgs*)p;
+    return *(const Args*)p;
 }
 
 /* Photon state of a lane. */
@@ -195,6 +196,73 @@ __device__ __forceinline__ void lock_step2(LockPhoton& p, uint32_t k, uint32_t c
     lock_add(lt, (uint32_t)fb, e1);
 }
 
+/* The wave's photons from absorption k0 to k1 (lanes without one walk a stale
+ * one, their deposits masked).  `table`: the set's weight table; `room`: steps
+ * to the next flush of the slot, which `flush` does. */
+template <uint32_t MATH, class Flush>
+__device__ __forceinline__ void lock_cycle(LockPhoton& p, uint32_t k0, uint32_t k1, const char* table, uint32_t zero,
+                                           uint32_t c3k1, const tmc_philox_photon& pp, const Physics& phys,
+                                           const LaneTally& lt, uint32_t& room, const Flush& flush)
+{
+    for (uint32_t k = k0; k != k1;) {
+        const uint32_t left = k1 - k, n = rfl32(left < room ? left : room);
+        room -= n;
+        const char* from = table + 16ull * k;
+        Images e0 = *(const Images*)(from + zero), e1 = *(const Images*)(from + 16u + zero);
+        const uint32_t stop = k + (n & ~1u);
+        for (; k != stop; k += 2u) {
+            from += 32u;
+            lock_step2<MATH>(p, k, c3k1, pp, phys, lt, e0, e1);
+            e0 = *(const Images*)(from + zero);
+            e1 = *(const Images*)(from + 16u + zero);
+        }
+        if (n & 1u) {
+            lock_step<MATH>(p, k, c3k1, pp, phys, lt, e0);
+            ++k;
+        }
+        if (room == 0u) {
+            flush();
+            room = TMC_LOCK_FLUSH_STEPS;
+        }
+    }
+}
+
+/* Loads the lane's photon from place i of a list; returns its index. */
+__device__ __forceinline__ uint32_t lock_load(LockPhoton& p, const PhotonList& l, uint32_t i)
+{
+    p.x = l.state[0][i];
+    p.y = l.state[1][i];
+    p.z = l.state[2][i];
+    p.u = l.state[3][i];
+    p.v = l.state[4][i];
+    p.w = l.state[5][i];
+    return l.photon[i];
+}
+
+/* Appends the photons of the lanes in S (not empty), of index `off`, to the
+ * `cap` places from `place` of a list; false if not all of them had room. */
+__device__ __forceinline__ bool lock_append(uint64_t S, uint32_t off, const LockPhoton& p, const PhotonList& l,
+                                            uint32_t* count, uint32_t place, uint32_t cap, uint32_t lane)
+{
+    const uint32_t n = (uint32_t)__popcll(S);
+    uint32_t base = 0;
+    if (lane == 0)
+        base = atomicAdd(count, n);
+    base = rfl32(base);
+    const uint32_t to = base + mask_rank(S);
+    if (__builtin_amdgcn_inverse_ballot_w64(S) && to < cap) {
+        const uint32_t i = place + to;
+        l.photon[i] = off;
+        l.state[0][i] = p.x;
+        l.state[1][i] = p.y;
+        l.state[2][i] = p.z;
+        l.state[3][i] = p.u;
+        l.state[4][i] = p.v;
+        l.state[5][i] = p.w;
+    }
+    return base + n <= cap;
+}
+
 } // namespace
 
 /* (LockArgs must stay the only parameter: args_here) */
@@ -257,7 +325,7 @@ __global__ void __launch_bounds__(256) walk_lock(LockArgs a)
     }
     for (;; at += stride) {
         if (claims && at >= claimed) {
-            const LockArgs& c = args_here();
+            const LockArgs& c = args_here<LockArgs>();
             uint32_t got = 0;
             if (lane == 0)
                 got = atomicAdd(c.cursor + blockIdx.x % TMC_LOCK_RANGES * TMC_LOCK_LINE, c.chunk);
@@ -271,84 +339,148 @@ __global__ void __launch_bounds__(256) walk_lock(LockArgs a)
         LockPhoton p = { 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 1.0f, ~0u };
         tmc_philox_photon pp;
         {
-            const LockArgs& c = args_here();
+            const LockArgs& c = args_here<LockArgs>();
             uint32_t off = place + at + lane;
-            if (c.level && __builtin_amdgcn_inverse_ballot_w64(in)) {
-                const uint32_t i = off;
-                off = c.in.photon[i];
-                p.x = c.in.state[0][i];
-                p.y = c.in.state[1][i];
-                p.z = c.in.state[2][i];
-                p.u = c.in.state[3][i];
-                p.v = c.in.state[4][i];
-                p.w = c.in.state[5][i];
-            }
+            if (c.level && __builtin_amdgcn_inverse_ballot_w64(in))
+                off = lock_load(p, c.in, off);
             const uint64_t photon = c.first_photon + off;
             pp = tmc_philox_photon_init((uint32_t)photon, (uint32_t)(photon >> 32), phys.key0, phys.key1);
         }
-        /* (lanes without a photon walk a stale one, their deposits masked) */
-        for (uint32_t k = k0; k != k1;) {
-            const uint32_t left = k1 - k, n = rfl32(left < room ? left : room);
-            room -= n;
-            const char* from = table + 16ull * k;
-            Images e0 = *(const Images*)(from + zero), e1 = *(const Images*)(from + 16u + zero);
-            const uint32_t stop = k + (n & ~1u);
-            for (; k != stop; k += 2u) {
-                from += 32u;
-                lock_step2<MATH>(p, k, c3k1, pp, phys, lt, e0, e1);
-                e0 = *(const Images*)(from + zero);
-                e1 = *(const Images*)(from + 16u + zero);
-            }
-            if (n & 1u) {
-                lock_step<MATH>(p, k, c3k1, pp, phys, lt, e0);
-                ++k;
-            }
-            if (room == 0u) {
-                const LockArgs& c = args_here();
-                lock_flush(slot, lock_block(c, wave) + TMC_COHORT_COUNTERS, c.shells, lane);
-                room = TMC_LOCK_FLUSH_STEPS;
-            }
-        }
+        lock_cycle<MATH>(p, k0, k1, table, zero, c3k1, pp, phys, lt, room, [&]() {
+            const LockArgs& c = args_here<LockArgs>();
+            lock_flush(slot, lock_block(c, wave) + TMC_COHORT_COUNTERS, c.shells, lane);
+        });
         interactions += (uint64_t)__popcll(in) * (k1 - k0);
-        const LockArgs& c = args_here();
+        const LockArgs& c = args_here<LockArgs>();
         uint64_t S = c.cut_ends ? in & __ballot(p.x3 < TMC_ROULETTE_KILL_R) : in;
         if (c.cap_ends) {
             truncated += (uint64_t)__popcll(S);
             S = 0;
         }
         if (S != 0) {
-            /* the survivors go to the list */
-            const uint32_t n = (uint32_t)__popcll(S);
-            uint32_t base = 0;
-            if (lane == 0)
-                base = atomicAdd(c.out_count + stripe * TMC_LOCK_LINE, n);
-            base = rfl32(base);
-            const uint32_t to = base + mask_rank(S);
-            const bool lives = __builtin_amdgcn_inverse_ballot_w64(S);
             uint32_t off = place + at + lane;
-            if (c.level && lives)
+            if (c.level && __builtin_amdgcn_inverse_ballot_w64(S))
                 off = c.in.photon[off];
-            if (lives && to < c.out_cap) {
-                const uint32_t i = stripe * c.out_cap + to;
-                c.out.photon[i] = off;
-                c.out.state[0][i] = p.x;
-                c.out.state[1][i] = p.y;
-                c.out.state[2][i] = p.z;
-                c.out.state[3][i] = p.u;
-                c.out.state[4][i] = p.v;
-                c.out.state[5][i] = p.w;
-            }
-            if (base + n > c.out_cap && lane == 0)
+            if (!lock_append(S, off, p, c.out, c.out_count + stripe * TMC_LOCK_LINE, stripe * c.out_cap, c.out_cap, lane)
+                && lane == 0)
                 atomicOr(lock_block(c, wave) + 2, TMC_LOCK_OVERFLOW);
         }
     }
-    const LockArgs& c = args_here();
+    const LockArgs& c = args_here<LockArgs>();
     unsigned long long* const block = lock_block(c, wave);
     lock_flush(slot, block + TMC_COHORT_COUNTERS, c.shells, lane);
     if (lane == 0) {
         atomicAdd(block + 1, (unsigned long long)interactions);
         if (truncated)
             atomicAdd(block + 2, (unsigned long long)truncated);
+    }
+}
+
+/* A level of a batch: each wave claims chunks of the queue, each a run of
+ * photons of one set, longest first, and moves its slot's sums into the set's
+ * when the next chunk is of another set.  (LockSetArgs must stay the only
+ * parameter: args_here) */
+template <uint32_t MATH>
+__global__ void __launch_bounds__(256) walk_lock_sets(LockSetArgs a)
+{
+    extern __shared__ unsigned long long lds[];
+    const uint32_t lane = __lane_id();
+    const uint32_t wave = rfl32(threadIdx.x >> 6);
+    unsigned long long* const slot = lds + wave * lock_slot_words(a.shells_max);
+    for (uint32_t i = lane; i < lock_slot_words(a.shells_max); i += 64u)
+        slot[i] = 0;
+    uint32_t zero = 0;
+    asm volatile("" : "+v"(zero));
+
+    Physics phys = {};
+    LaneTally lt = { slot, 0.0f, ~0ull };
+    uint32_t set = ~0u, k0 = 0, k1 = 0, hi = 0;
+    const char* table = nullptr;
+    uint64_t interactions = 0, idle = 0;
+    uint32_t room = TMC_LOCK_FLUSH_STEPS;
+    auto flush = [&]() {
+        const LockSetArgs& c = args_here<LockSetArgs>();
+        const LockSet& s = c.sets[set];
+        lock_flush(slot, c.tally + s.tally, s.shells, lane);
+    };
+
+    for (;;) {
+        uint32_t first, count;
+        {
+            const LockSetArgs& c = args_here<LockSetArgs>();
+            uint32_t got = 0;
+            if (lane == 0)
+                got = atomicAdd(c.cursor, 1u);
+            got = rfl32(got);
+            if (got >= c.nchunks)
+                break;
+            const LockChunk& ch = c.chunks[got];
+            const uint32_t next = rfl32(ch.set);
+            first = rfl32(ch.first);
+            count = rfl32(ch.count);
+            if (c.level) {
+                /* of the set's places, those that were filled */
+                const uint32_t cap = c.sets[next].cap[c.level - 1u], n = c.in_count[next * TMC_LOCK_LINE];
+                const uint32_t have = rfl32(n < cap ? n : cap);
+                if (first >= have)
+                    continue;
+                count = have - first < count ? have - first : count;
+            }
+            if (next != set) {
+                if (set != ~0u)
+                    flush();
+                set = next;
+                const LockSet& s = c.sets[set];
+                phys.key0 = rfl32((uint32_t)s.seed);
+                phys.key1 = rfl32((uint32_t)(s.seed >> 32));
+                phys.albedo = s.albedo;
+                phys.spm = s.spm;
+                phys.shell_max = s.shell_max;
+                set_derived<true>(phys);
+                lt.fmax = tally_fmax(s.shell_max, lane & (TMC_LOCK_HOT - 1u));
+                const CohortHead& h = c.heads[s.head];
+                k0 = rfl32(c.level ? h.cut[c.level - 1u] : 0u);
+                k1 = rfl32(h.cut[c.level]);
+                hi = rfl32((uint32_t)(s.first_photon >> 32));
+                table = (const char*)c.entry + 16ull * rfl64(s.entry);
+                room = TMC_LOCK_FLUSH_STEPS;
+            }
+        }
+        for (uint32_t at = 0; at < count; at += 64u) {
+            const uint64_t in = count - at >= 64u ? ~0ull : (1ull << (count - at)) - 1ull;
+            lt.deposit = in;
+            LockPhoton p = { 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 1.0f, ~0u };
+            tmc_philox_photon pp;
+            uint32_t off = first + at + lane;
+            {
+                const LockSetArgs& c = args_here<LockSetArgs>();
+                const LockSet& s = c.sets[set];
+                if (c.level && __builtin_amdgcn_inverse_ballot_w64(in))
+                    off = lock_load(p, c.in, s.place[c.level - 1u] + off);
+                const uint64_t photon = s.first_photon + off;
+                pp = tmc_philox_photon_init((uint32_t)photon, hi, phys.key0, phys.key1);
+            }
+            lock_cycle<MATH>(p, k0, k1, table, zero, hi ^ phys.key1, pp, phys, lt, room, flush);
+            const uint32_t n = (uint32_t)__popcll(in);
+            interactions += (uint64_t)n * (k1 - k0);
+            idle += (uint64_t)(64u - n) * (k1 - k0);
+            const uint64_t S = in & __ballot(p.x3 < TMC_ROULETTE_KILL_R);
+            if (S != 0) {
+                const LockSetArgs& c = args_here<LockSetArgs>();
+                const LockSet& s = c.sets[set];
+                if (!lock_append(S, off, p, c.out, c.out_count + set * TMC_LOCK_LINE, s.place[c.level],
+                                 s.cap[c.level], lane)
+                    && lane == 0)
+                    atomicOr(c.counters + 2, TMC_LOCK_OVERFLOW);
+            }
+        }
+    }
+    if (set != ~0u)
+        flush();
+    if (lane == 0) {
+        const LockSetArgs& c = args_here<LockSetArgs>();
+        atomicAdd(c.counters + 1, (unsigned long long)interactions);
+        atomicAdd(c.counters + 4, (unsigned long long)idle);
     }
 }
 
@@ -370,6 +502,29 @@ hipError_t lock_occupancy(uint32_t math, uint32_t block, uint32_t shells, int* w
 {
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(wg_per_cu, lock_kernel(math), (int)block,
                                                         lock_lds_bytes(shells, block));
+}
+
+namespace {
+
+using LockSetsKernel = void (*)(LockSetArgs);
+
+LockSetsKernel lock_sets_kernel(uint32_t math)
+{
+    return math == TMC_MATH_OWN ? walk_lock_sets<TMC_MATH_OWN> : walk_lock_sets<TMC_MATH_HARDWARE>;
+}
+
+} // namespace
+
+hipError_t launch_lock_sets(uint32_t math, const LockSetArgs& a, uint32_t grid, uint32_t block, hipStream_t stream)
+{
+    hipLaunchKernelGGL(lock_sets_kernel(math), dim3(grid), dim3(block), lock_lds_bytes(a.shells_max, block), stream, a);
+    return hipGetLastError();
+}
+
+hipError_t lock_sets_occupancy(uint32_t math, uint32_t block, uint32_t shells_max, int* wg_per_cu)
+{
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(wg_per_cu, lock_sets_kernel(math), (int)block,
+                                                        lock_lds_bytes(shells_max, block));
 }
 
 } // namespace tmc
