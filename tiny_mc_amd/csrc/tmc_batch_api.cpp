@@ -26,7 +26,7 @@
  * to the set's places in a list; where a batch leaves enough of them they are
  * walked to the second roulette the same way, and workgroups carry what is
  * left to its end as cohorts.  Measured on MI355X, walk_multi -> this:
- * 64 sets, 1.1e6 photons, planned, run and released 11.1 -> 3.9 ms; a kept
+ * 64 sets, 1.1e6 photons, planned, run and released 11.1 -> 3.1 ms; a kept
  * plan of 512 sets, 5.6e7 photons 232 -> 144 ms (its lanes idle 1% of the
  * steps, 24% before).
  */
@@ -93,6 +93,12 @@ constexpr double kSecondCycle = 200000.0;
  * a flush of the slot, about 10 us). */
 constexpr double kChunkSteps = 512.0;
 constexpr uint32_t kLockBlock = 256;
+
+/* Absorptions to a set's first roulette, and from there to the second (0: the
+ * first is further than is walked out, tmc::expected_interactions). */
+struct Cadence {
+    uint32_t k1 = 0, k2 = 0;
+};
 
 } // namespace
 
@@ -260,7 +266,7 @@ uint32_t cuts_for(double n)
  * share of LDS (tmc_api.cpp's line), and where the weight tables or a first
  * cycle are longer than is worth laying out.  TMC_OK, or TMC_E_HIP. */
 int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_batch_options* o, uint64_t kcap,
-              const std::vector<tmc::BatchSet>& hs, tmc_batch_plan* p)
+              const std::vector<tmc::BatchSet>& hs, const std::vector<Cadence>& cad, tmc_batch_plan* p)
 {
     LockPlan& l = p->lock;
     if (o->sampler != TMC_SAMPLER_ANALYTIC || o->block || o->waves_per_simd || o->copies || o->chunk_work
@@ -272,12 +278,8 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
         uint32_t set;
         uint64_t first, count; /* photons of the set */
     };
-    struct Cadence {
-        uint32_t k1, k2;
-    };
     std::vector<tmc::LockSet> ls;
     std::vector<Part> parts;
-    std::vector<Cadence> cad(nsets);
     l.cycles = 0.1 * (double)p->photons >= kSecondCycle ? 2u : 1u;
     uint64_t entries = 0;
     double steps = 0.0; /* of 64 photons, in the first cycles */
@@ -285,7 +287,7 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
         const uint64_t n = sets[i].params.photons;
         if (n == 0)
             continue;
-        if (!tmc::weight_cadence(&sets[i].params, 1u << 20, &cad[i].k1, &cad[i].k2))
+        if (cad[i].k1 == 0)
             return TMC_OK;
         const uint32_t cuts = std::max(cuts_for((double)n), l.cycles + 2u);
         /* (later cycles can be a step longer than the second; two entries are
@@ -332,23 +334,23 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
 
     /* slices, places and queues: chunks of a wave's 32nd of the work, longest first */
     const double target = std::max(kChunkSteps, steps / ((double)l.grid * (kLockBlock / 64u)) / 32.0);
-    struct Chunk {
+    struct Run { /* chunks of a part, of one length */
         double steps;
-        tmc::LockChunk chunk;
+        uint32_t part, first, each, chunks;
     };
     std::vector<tmc::LockChunk> queue;
     uint64_t places[2] = { 0, 0 };
     for (size_t i = 0; i < parts.size();) {
         LockSlice slice;
         uint64_t used[2] = { 0, 0 };
-        std::vector<Chunk> chunks[3];
+        std::vector<Run> runs[3];
         auto cut = [&](uint32_t level, uint32_t part, uint64_t n, double cycle, double each) {
             const uint64_t batches = std::max<uint64_t>(1, (uint64_t)std::min(1e6, std::ceil(each / cycle)));
-            for (uint64_t first = 0; first < n; first += 64u * batches) {
-                const uint32_t count = (uint32_t)std::min<uint64_t>(64u * batches, n - first);
-                chunks[level].push_back(
-                    { cycle * std::ceil((double)count / 64.0), { part, (uint32_t)first, count, 0u } });
-            }
+            const uint32_t full = (uint32_t)(n / (64u * batches)), rest = (uint32_t)(n - 64u * batches * full);
+            if (full)
+                runs[level].push_back({ cycle * (double)batches, part, 0u, (uint32_t)(64u * batches), full });
+            if (rest)
+                runs[level].push_back({ cycle * std::ceil((double)rest / 64.0), part, (uint32_t)(n - rest), rest, 1u });
         };
         for (; i < parts.size(); ++i) {
             /* places for an eighth of the photons and a slack, where a tenth
@@ -369,14 +371,16 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
             cut(2, (uint32_t)i, cap[l.cycles - 1u], (double)k.k2, 1.0);
         }
         for (uint32_t level = 0; level < 3u; ++level) {
-            std::stable_sort(chunks[level].begin(), chunks[level].end(),
-                             [](const Chunk& x, const Chunk& y) { return x.steps > y.steps; });
+            std::stable_sort(runs[level].begin(), runs[level].end(),
+                             [](const Run& x, const Run& y) { return x.steps > y.steps; });
             slice.first[level] = (uint32_t)queue.size();
-            slice.chunks[level] = (uint32_t)chunks[level].size();
-            for (const Chunk& ch : chunks[level])
-                queue.push_back(ch.chunk);
-            if (queue.size() > 1u << 26)
-                return TMC_OK;
+            for (const Run& r : runs[level]) {
+                if (queue.size() + r.chunks > 1u << 26)
+                    return TMC_OK;
+                for (uint32_t j = 0; j < r.chunks; ++j)
+                    queue.push_back({ r.part, r.first + j * r.each, r.each, 0u });
+            }
+            slice.chunks[level] = (uint32_t)queue.size() - slice.first[level];
         }
         for (uint32_t w = 0; w < 2u; ++w)
             places[w] = std::max(places[w], used[w]);
@@ -425,6 +429,7 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
     a.heads = (const tmc::CohortHead*)(d + at_heads);
     a.chunks = (const tmc::LockChunk*)(d + at_queue);
     a.entry = d + at_entries;
+    a.cus = l.cus;
     a.shells_max = p->shells_max;
     a.tally = p->d_tally;
     a.counters = p->d_counters;
@@ -465,6 +470,7 @@ int plan_create_locked(tmc::Context* c, const tmc_set* sets, uint32_t nsets, con
     /* set table */
     std::vector<tmc::BatchSet> hs(nsets);
     std::vector<tmc::PlanSet> ps(nsets);
+    std::vector<Cadence> cad(nsets);
     uint64_t off = 0;
     double work = 0.0;
     uint32_t shells_max = 1;
@@ -485,7 +491,7 @@ int plan_create_locked(tmc::Context* c, const tmc_set* sets, uint32_t nsets, con
         d.kcap = (uint32_t)kcap;
         off += 4 * (uint64_t)q.shells;
         shells_max = std::max(shells_max, q.shells);
-        ps[i] = { q.shells, q.photons, tmc::expected_interactions(&q, kcap) };
+        ps[i] = { q.shells, q.photons, tmc::expected_interactions(&q, kcap, &cad[i].k1, &cad[i].k2) };
         work += ps[i].L * (double)q.photons;
         p->photons += q.photons;
     }
@@ -578,7 +584,7 @@ int plan_create_locked(tmc::Context* c, const tmc_set* sets, uint32_t nsets, con
         a.done = p->d_done;
     }
 
-    const int lrc = plan_lock(c, sets, nsets, o, kcap, hs, p);
+    const int lrc = plan_lock(c, sets, nsets, o, kcap, hs, cad, p);
     if (lrc != TMC_OK) {
         plan_free(p);
         return lrc;

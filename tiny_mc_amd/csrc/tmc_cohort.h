@@ -66,6 +66,7 @@ struct LockSetArgs {
     const void* entry; /* pool of pairs of images */
     const LockChunk* chunks;
     uint32_t nchunks;
+    uint32_t cus;
     uint32_t* cursor; /* of this launch */
     uint32_t level; /* roulettes the photons of the queue have survived */
     uint32_t shells_max;

@@ -834,50 +834,63 @@ __global__ void __launch_bounds__(1024) walk_cohort_sets(LockSetArgs a)
     }
 }
 
-/* The weight table of a set: one wave walks the recurrence W[k+1] = RN(W[k] a),
- * every lane alike, 64 absorptions at a time, and lane i keeps the i-th weight.
- * (8 ns an absorption; on the host 1.3 ns, but for one set after the other.) */
-__global__ void __launch_bounds__(64) weigh_sets(const LockSet* sets, CohortHead* heads, Images* pool)
+/* The weight table of a set: one lane walks the recurrence W[k+1] = RN(W[k] a),
+ * 64 absorptions at a time, and a second wave makes images of the 64 before.
+ * (The chain is a multiplication of 9 cycles an absorption, 4 ns, and the
+ * hand-over through LDS; on the host it is 1.3 ns, but for one set after the
+ * other.) */
+__global__ void __launch_bounds__(128) weigh_sets(const LockSet* sets, CohortHead* heads, Images* pool)
 {
+    __shared__ float4 weights[2][16];
+    __shared__ uint32_t valid[2]; /* weights of the block; 0: none, and none follows */
     const LockSet& s = sets[blockIdx.x];
     if (s.cuts == 0u)
         return;
     CohortHead& h = heads[s.head];
     Images* const entry = pool + s.entry;
-    const uint32_t lane = __lane_id();
     const float a = s.albedo;
     float w = 1.0f;
     uint32_t n = 0;
-    for (uint32_t k = 0; n < s.cuts && k < s.entries; k += 64u) {
-        float v = w, mine = w;
-        uint32_t me = lane;
-        asm volatile("" : "+v"(me)); /* (64 comparisons kept from one pass for the next would not fit) */
+    for (uint32_t k = 0, par = 0;; k += 64u, par ^= 1u) {
+        if (threadIdx.x == 0) {
+            const uint32_t room = n < s.cuts && k < s.entries ? (s.entries - k < 64u ? s.entries - k : 64u) : 0u;
+            float v = w;
 #pragma unroll
-        for (uint32_t i = 0; i < 64u; ++i) {
-            if (me == i)
-                mine = v;
-            v = v * a;
-        }
-        if (v < 0.001f) {
-            /* a roulette among them (the weight never grows between two) */
-            v = w;
-            for (uint32_t i = 0; i < 64u && n < s.cuts && k + i < s.entries; ++i) {
-                if (lane == i)
-                    mine = v;
-                v = v * a;
-                if (v < 0.001f) {
-                    v = v / 0.1f;
-                    if (lane == 0)
-                        h.cut[n] = k + i + 1u;
-                    ++n;
+            for (uint32_t i = 0; i < 16u; ++i) {
+                float4 q;
+                q.x = v;
+                q.y = q.x * a;
+                q.z = q.y * a;
+                q.w = q.z * a;
+                v = q.w * a;
+                weights[par][i] = q;
+            }
+            if (v < 0.001f) {
+                /* a roulette among them (the weight never grows between two) */
+                float* const out = (float*)weights[par];
+                v = w;
+                for (uint32_t i = 0; i < room && n < s.cuts; ++i) {
+                    out[i] = v;
+                    v = v * a;
+                    if (v < 0.001f) {
+                        v = v / 0.1f;
+                        h.cut[n++] = k + i + 1u;
+                    }
                 }
             }
+            if (room)
+                w = v;
+            valid[par] = room;
         }
-        w = v;
-        if (k + lane < s.entries)
-            entry[k + lane] = images_of(mine);
+        /* the block before, on the other side of the barrier */
+        const uint32_t lane = threadIdx.x - 64u;
+        if (k != 0u && lane < valid[par ^ 1u])
+            entry[k - 64u + lane] = images_of(((const float*)weights[par ^ 1u])[lane]);
+        __syncthreads();
+        if (valid[par] == 0u)
+            break;
     }
-    if (lane == 0) {
+    if (threadIdx.x == 0) {
         h.ncuts = n;
         h.w_end = w;
     }
@@ -925,7 +938,7 @@ hipError_t launch_cohort_sets(uint32_t math, const LockSetArgs& a, uint32_t grid
 
 hipError_t launch_weigh_sets(const LockSet* sets, uint32_t nsets, CohortHead* heads, void* entry, hipStream_t stream)
 {
-    hipLaunchKernelGGL(weigh_sets, dim3(nsets), dim3(64), 0, stream, sets, heads, (Images*)entry);
+    hipLaunchKernelGGL(weigh_sets, dim3(nsets), dim3(128), 0, stream, sets, heads, (Images*)entry);
     return hipGetLastError();
 }
 

@@ -91,7 +91,7 @@ uint32_t tmc::weight_sequence(const tmc_params* p, uint32_t room, uint32_t max_c
 
 /* Mean absorptions k1 + k2 p / (1 - p) with p the survival probability
  * 1677721 / 2^24 of the (0,1] uniform. */
-double tmc::expected_interactions(const tmc_params* p, uint64_t kcap)
+double tmc::expected_interactions(const tmc_params* p, uint64_t kcap, uint32_t* k1_out, uint32_t* k2_out)
 {
     const double pr = 1677721.0 / 16777216.0;
     uint32_t k1 = 0, k2 = 0;
@@ -104,7 +104,12 @@ double tmc::expected_interactions(const tmc_params* p, uint64_t kcap)
         const double a = (double)derived_albedo(p);
         c1 = std::log(0.001) / std::log(a);
         c2 = std::log(0.1) / std::log(a);
+        k1 = k2 = 0;
     }
+    if (k1_out)
+        *k1_out = k1;
+    if (k2_out)
+        *k2_out = k2;
     double mean = c1 + c2 * pr / (1.0 - pr);
     if (kcap && mean > (double)kcap)
         mean = (double)kcap;

@@ -52,7 +52,7 @@ uint32_t weight_sequence(const tmc_params* p, uint32_t room, uint32_t max_cuts, 
 
 /* Expected absorptions per photon of the FP32 weight cadence with the
  * roulette of photon.c:45-49, capped at kcap (scheduling estimate). */
-double expected_interactions(const tmc_params* p, uint64_t kcap);
+double expected_interactions(const tmc_params* p, uint64_t kcap, uint32_t* k1 = nullptr, uint32_t* k2 = nullptr);
 
 /* Launch shape of the cohort walk for a run. */
 struct CohortShape {
