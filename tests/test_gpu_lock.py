@@ -69,3 +69,28 @@ def test_alternating_runs(tmc, orc, hw_tables):
     for i, (phys, photons) in enumerate([(DEFAULT, 70000), (HIGHALB, 300), (LOWALB, 3000000), (DEFAULT, 50000),
                                          (DEFAULT, 20), (HIGHALB, 70000)]):
         check(tmc, orc, hw_tables, phys, photons, 160 + i)
+
+
+@pytest.mark.parametrize("math", [0, 1])
+@pytest.mark.parametrize("phys,photons,first,kmax", [
+    (DEFAULT, 49153, 0, 0), (DEFAULT, 400001, (1 << 32) - 1000, 0), (LOWALB, 524289, 0, 0), (HIGHALB, 60000, 7 << 33, 0),
+    (dict(DEFAULT, shells=450, microns_per_shell=9.0), 70000, 0, 0), (dict(DEFAULT, shells=451), 60000, 0, 0),
+    (dict(DEFAULT, shells=1), 50000, 3, 0), (dict(mu_a=100.0, mu_s=1e-30, shells=3, microns_per_shell=50.0), 60000, 0, 0),
+    (DEFAULT, 100003, 0, 1), (DEFAULT, 100003, 0, 74), (DEFAULT, 100003, 0, 99)])
+def test_rejection_sampler(tmc, phys, photons, first, kmax, math):
+    """The rejection sampler's groups of absorptions, whose later attempts are
+    gathered over the wave, against the lane-per-photon walk (block given)."""
+    print(f"lock rejection: {phys} photons={photons} first={first} kmax={kmax} math={math}", flush=True)
+    p = tmc.Params(photons=photons, **phys)
+    kw = dict(sampler=1, first_photon=first, math=math, max_interactions=kmax)
+    got, st = tmc.run_raw(p, (5 << 40) + photons, **kw)
+    want, ws = tmc.run_raw(p, (5 << 40) + photons, block=256, **kw)
+    np.testing.assert_array_equal(got, want)
+    assert (st.interactions, st.truncated) == (ws.interactions, ws.truncated)
+
+
+def test_rejection_sampler_against_the_oracle(tmc, orc, hw_tables):
+    tally, st = tmc.run_raw(tmc.Params(photons=50007, **DEFAULT), 12, sampler=1)
+    want, n = orc.mirror32(orc.params(**DEFAULT), 12, 50007, sampler=1, tables=hw_tables)
+    assert st.interactions == n
+    np.testing.assert_array_equal(tally, want)

@@ -300,7 +300,7 @@ int run_cohort(Context* c, const tmc_params* p, uint64_t seed, const tmc_options
                tmc_run_stats* st)
 {
     tmc::CohortShape shape;
-    const uint64_t most = o->sampler == TMC_SAMPLER_ANALYTIC ? TMC_COHORT_PHOTONS : TMC_COHORT_PHOTONS_REJECTION;
+    const uint64_t most = p->shells > TMC_LOCK_SHELLS ? TMC_COHORT_PHOTONS_WIDE : TMC_COHORT_PHOTONS;
     if (!tmc::cohort_shape(p->photons, most, first_cycle(p, kcap), p->shells, (uint32_t)c->compute_units, &shape))
         return TMC_E_UNSUPPORTED;
     tmc::CohortArgs a;
@@ -353,13 +353,15 @@ uint32_t list_cap(uint32_t which, uint32_t n) { return (which ? n / 64u : n / 8u
 int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* o, uint64_t kcap, uint64_t* tally,
              tmc_run_stats* st)
 {
-    /* (from 450 shells on, fewer than 5 waves' sums fit a SIMD's share of LDS) */
-    if (p->photons <= TMC_COHORT_PHOTONS || p->photons > (1ull << 40) || p->shells > 450)
+    if (p->photons <= TMC_COHORT_PHOTONS || p->photons > (1ull << 40) || p->shells > TMC_LOCK_SHELLS)
         return TMC_E_UNSUPPORTED;
     /* many photons of short walks: launching them 64 at a time and appending
      * the survivors costs what the step saves (albedo 0.5: 2^23 photons 951 us
-     * lane per photon, 306 us here; 2^27 2841 and 2897 us) */
-    if (p->photons > (1ull << 26) && first_cycle(p, kcap) < 32.0)
+     * lane per photon, 306 us here; 2^27 2841 and 2897 us; the rejection
+     * sampler's step is longer: 2^27 at albedo 0.5 4885 and 4696 us, at 1/6
+     * 2216 and 2306 us) */
+    const double shortest = o->sampler == TMC_SAMPLER_ANALYTIC ? 32.0 : 8.0;
+    if (p->photons > (1ull << 26) && first_cycle(p, kcap) < shortest)
         return TMC_E_UNSUPPORTED;
     const uint64_t slice = std::min<uint64_t>(p->photons, 1ull << tmc::kSliceLog);
     uint32_t levels = 1;
@@ -421,7 +423,7 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
     /* (the batches go round the resident waves, so a workgroup that had to wait
      * for another to end would double the launch's time) */
     int per_cu = 0;
-    if (tmc::lock_occupancy(o->math, block, p->shells, &per_cu) != hipSuccess || per_cu <= 0)
+    if (tmc::lock_occupancy(o->sampler, o->math, block, p->shells, &per_cu) != hipSuccess || per_cu <= 0)
         return TMC_E_HIP;
     const uint32_t grid_most = (uint32_t)per_cu * cus;
     tmc::CohortShape shape;
@@ -486,7 +488,7 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
                         l.cursor = count + levels * words;
                     }
                 }
-                if (tmc::launch_lock(o->math, l, grid, block, c->stream) != hipSuccess)
+                if (tmc::launch_lock(o->sampler, o->math, l, grid, block, c->stream) != hipSuccess)
                     return false;
             }
             a.finish = si + 1 == slices.size();
@@ -540,7 +542,7 @@ int tmc::run_walk(Context* c, const tmc_params* p, uint64_t seed, const tmc_opti
     if (work == c->d_work && o->precision == TMC_PRECISION_FP32 && !o->block && !o->grid && !o->chunk
         && !o->weight_table) {
         int rc = run_cohort(c, p, seed, o, kcap, tally, st);
-        if (rc == TMC_E_UNSUPPORTED && o->sampler == TMC_SAMPLER_ANALYTIC)
+        if (rc == TMC_E_UNSUPPORTED)
             rc = run_lock(c, p, seed, o, kcap, tally, st);
         if (rc == TMC_OK && st) {
             st->photons = p->photons;

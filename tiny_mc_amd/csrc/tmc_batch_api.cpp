@@ -262,15 +262,14 @@ uint32_t cuts_for(double n)
 
 /* Plans the lockstep launches of a batch; leaves p->lock off where they don't
  * apply: with the rejection sampler, with a cap on the absorptions, where the
- * caller chose a launch shape, where fewer than 5 waves' sums fit a SIMD's
- * share of LDS (tmc_api.cpp's line), and where the weight tables or a first
+ * caller chose a launch shape, with more than TMC_LOCK_SHELLS shells, and where the weight tables or a first
  * cycle are longer than is worth laying out.  TMC_OK, or TMC_E_HIP. */
 int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_batch_options* o, uint64_t kcap,
               const std::vector<tmc::BatchSet>& hs, const std::vector<Cadence>& cad, tmc_batch_plan* p)
 {
     LockPlan& l = p->lock;
     if (o->sampler != TMC_SAMPLER_ANALYTIC || o->block || o->waves_per_simd || o->copies || o->chunk_work
-        || kcap != 0xFFFFFFFFull || p->shells_max > 450u || p->photons == 0)
+        || kcap != 0xFFFFFFFFull || p->shells_max > TMC_LOCK_SHELLS || p->photons == 0)
         return TMC_OK;
 
     /* the sets' cadences and tables, and their parts */

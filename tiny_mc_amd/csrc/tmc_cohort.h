@@ -151,10 +151,10 @@ struct LockArgs {
     unsigned long long* work; /* as CohortArgs */
 };
 
-size_t lock_lds_bytes(uint32_t shells, uint32_t block);
+size_t lock_lds_bytes(uint32_t sampler, uint32_t shells, uint32_t block);
 /* Resident workgroups per CU of walk_lock. */
-hipError_t lock_occupancy(uint32_t math, uint32_t block, uint32_t shells, int* wg_per_cu);
-hipError_t launch_lock(uint32_t math, const LockArgs& a, uint32_t grid, uint32_t block, hipStream_t stream);
+hipError_t lock_occupancy(uint32_t sampler, uint32_t math, uint32_t block, uint32_t shells, int* wg_per_cu);
+hipError_t launch_lock(uint32_t sampler, uint32_t math, const LockArgs& a, uint32_t grid, uint32_t block, hipStream_t stream);
 
 /* The same for the sets of a batch: a level by lockstep waves (0 or 1), and
  * the survivors of a.level roulettes by cohorts, to their end.  Analytic

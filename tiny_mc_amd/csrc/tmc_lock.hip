@@ -20,7 +20,10 @@
  * walk_f32 -> this walk: 2^20 photons at default physics 425 -> 236 us,
  * 3,000,017 638 -> 500 us, 2^26 8.72 -> 7.87 ms; 2^20 at albedo 0.99 2.73 ->
  * 1.38 ms; 2^17 at albedo 0.9999 117 -> 22 ms; 2^23 at albedo 0.5 951 -> 306
- * us.
+ * us.  With the rejection sampler a step is 133 vector instructions, a third
+ * of them the second generator block of the quarter of the directions that
+ * are drawn again: 2^17 photons at default physics 304 -> 110 us, 2^24 4.23 ->
+ * 3.49 ms, 2^20 at albedo 0.99 5.0 -> 2.75 ms.
  *
  * Same words, same operations and the same integer sums as step(): results
  * are bit-identical.
@@ -46,7 +49,20 @@ __host__ __device__ __forceinline__ size_t lock_slot_words(uint32_t shells)
     return 2u * ((size_t)shells - 1u + TMC_LOCK_HOT);
 }
 
-size_t lock_lds_bytes(uint32_t shells, uint32_t block) { return (block / 64u) * lock_slot_words(shells) * 8u; }
+/* Absorptions the rejection sampler's waves walk at a time, and the LDS words
+ * of the directions they draw again. */
+#define TMC_LOCK_GROUP 4u
+#define TMC_LOCK_RETRIES (64u * TMC_LOCK_GROUP)
+
+__host__ __device__ __forceinline__ size_t lock_wave_words(uint32_t sampler, uint32_t shells)
+{
+    return lock_slot_words(shells) + (sampler ? TMC_LOCK_RETRIES : 0u);
+}
+
+size_t lock_lds_bytes(uint32_t sampler, uint32_t shells, uint32_t block)
+{
+    return (block / 64u) * lock_wave_words(sampler, shells) * 8u;
+}
 
 namespace {
 
@@ -196,6 +212,124 @@ __device__ __forceinline__ void lock_step2(LockPhoton& p, uint32_t k, uint32_t c
     lock_add(lt, (uint32_t)fb, e1);
 }
 
+/* Orders a wave's LDS accesses across its lanes (the LDS serves them in the
+ * order of the instructions). */
+__device__ __forceinline__ void wave_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+/* Absorptions k .. k + G - 1 with the rejection sampler (photon.c:34-43), as
+ * step_core makes its attempts: the first from words 1-2 of block (k, 0),
+ * attempts 2b and 2b + 1 from block (k, b).  Of 64 lanes some always reject
+ * (14 on average), so the (photon, absorption) pairs of G absorptions whose
+ * first attempt fails are gathered, through LDS, into as few passes over a
+ * further block as hold them: 55 pairs for G = 4, one pass with its lanes
+ * nearly full, and a second for the twentieth part that fails again.
+ * `images`: the table's entry of absorption k. */
+template <uint32_t MATH, uint32_t G>
+__device__ __forceinline__ void lock_group_rejection(LockPhoton& p, uint32_t k, uint32_t hi, uint32_t plo,
+                                                     const tmc_philox_photon& pp, const Physics& phys,
+                                                     const LaneTally& lt, const char* images, uint32_t zero,
+                                                     unsigned long long* retries)
+{
+    float t[G], a[G], b[G];
+    uint32_t at[G]; /* the lane's pair j among the gathered */
+    uint64_t again[G];
+    uint32_t n = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < G; ++j) {
+        const tmc_u32x4 r = block0_uniform(k + j, hi ^ phys.key1, pp, phys.keys);
+        t[j] = step_length<MATH>(r.x0);
+        a[j] = tmc_u11(r.x1);
+        b[j] = tmc_u11(r.x2);
+        if (j == G - 1u)
+            p.x3 = r.x3;
+        const float tt = __builtin_fmaf(b[j], b[j], a[j] * a[j]);
+        again[j] = lt.deposit & ~__ballot(tt <= 1.0f && tt > 0.0f);
+        at[j] = n + mask_rank(again[j]);
+        n += (uint32_t)__popcll(again[j]);
+        if (__builtin_amdgcn_inverse_ballot_w64(again[j]))
+            retries[at[j]] = __lane_id() | j << 6;
+    }
+    n = rfl32(n);
+    wave_order();
+    for (uint32_t first = 0; first < n; first += 64u) {
+        const uint32_t i = first + __lane_id();
+        bool open = i < n;
+        const uint32_t pair = open ? (uint32_t)retries[i] : 0u;
+        const uint32_t from = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((pair & 63u) << 2), (int)plo);
+        const tmc_philox_photon q = tmc_philox_photon_init(from, hi, phys.key0, phys.key1);
+        float x = 0.0f, y = 0.0f;
+        for (uint32_t block = 1u; __ballot(open) != 0; ++block) {
+            const tmc_u32x4 r = tmc_philox4x32_10_blockb(k + (pair >> 6), block, q, &phys.keys, phys.key0, phys.key1);
+            const float x0 = tmc_u11(r.x0), y0 = tmc_u11(r.x1), x1 = tmc_u11(r.x2), y1 = tmc_u11(r.x3);
+            const float t0 = __builtin_fmaf(y0, y0, x0 * x0), t1 = __builtin_fmaf(y1, y1, x1 * x1);
+            const bool ok0 = (t0 <= 1.0f && t0 > 0.0f) || block == 32u; /* (the 64th attempt is taken) */
+            if (open) {
+                x = ok0 ? x0 : x1;
+                y = ok0 ? y0 : y1;
+            }
+            open = open && !(ok0 || (t1 <= 1.0f && t1 > 0.0f));
+        }
+        if (i < n)
+            retries[i] = (uint64_t)__float_as_uint(y) << 32 | __float_as_uint(x);
+    }
+    wave_order();
+    Images e[G];
+#pragma unroll
+    for (uint32_t j = 0; j < G; ++j)
+        e[j] = *(const Images*)(images + 16u * j + zero);
+    float r2[G];
+#pragma unroll
+    for (uint32_t j = 0; j < G; ++j) {
+        if (__builtin_amdgcn_inverse_ballot_w64(again[j])) {
+            const uint64_t xy = retries[at[j]];
+            a[j] = __uint_as_float((uint32_t)xy);
+            b[j] = __uint_as_float((uint32_t)(xy >> 32));
+        }
+        const float tt = __builtin_fmaf(b[j], b[j], a[j] * a[j]);
+        Drawn d;
+        d.t = t[j];
+        d.u = __builtin_fmaf(2.0f, tt, -1.0f);
+        const float s = 2.0f * sqrt_cr_walk(1.0f - tt); /* 1 - tt: 0 or >= 2^-24 */
+        d.v = a[j] * s;
+        d.w = b[j] * s;
+        d.x3 = p.x3;
+        r2[j] = lock_move(p, d);
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < G; ++j)
+        lock_add(lt, shell_index(r2[j], phys, lt.fmax), e[j]);
+}
+
+/* lock_cycle with the rejection sampler. */
+template <uint32_t MATH, class Flush>
+__device__ __forceinline__ void lock_cycle_rejection(LockPhoton& p, uint32_t k0, uint32_t k1, const char* table,
+                                                     uint32_t zero, uint32_t hi, uint32_t plo,
+                                                     const tmc_philox_photon& pp, const Physics& phys,
+                                                     const LaneTally& lt, unsigned long long* retries, uint32_t& room,
+                                                     const Flush& flush)
+{
+    constexpr uint32_t G = TMC_LOCK_GROUP;
+    for (uint32_t k = k0; k != k1;) {
+        const uint32_t left = k1 - k, n = rfl32(left < room ? left : room);
+        room -= n;
+        const char* from = table + 16ull * k;
+        const uint32_t stop = k + n;
+        for (; k + G <= stop; k += G, from += 16u * G)
+            lock_group_rejection<MATH, G>(p, k, hi, plo, pp, phys, lt, from, zero, retries);
+        for (; k != stop; ++k, from += 16u)
+            lock_group_rejection<MATH, 1u>(p, k, hi, plo, pp, phys, lt, from, zero, retries);
+        if (room == 0u) {
+            flush();
+            room = TMC_LOCK_FLUSH_STEPS;
+        }
+    }
+}
+
 /* The wave's photons from absorption k0 to k1 (lanes without one walk a stale
  * one, their deposits masked).  `table`: the set's weight table; `room`: steps
  * to the next flush of the slot, which `flush` does. */
@@ -266,13 +400,13 @@ __device__ __forceinline__ bool lock_append(uint64_t S, uint32_t off, const Lock
 } // namespace
 
 /* (LockArgs must stay the only parameter: args_here) */
-template <uint32_t MATH>
-__global__ void __launch_bounds__(256) walk_lock(LockArgs a)
+template <uint32_t SAMPLER, uint32_t MATH>
+__global__ void __launch_bounds__(256, SAMPLER ? 6 : 8) walk_lock(LockArgs a)
 {
     extern __shared__ unsigned long long lds[];
     const uint32_t lane = __lane_id();
     const uint32_t wave = rfl32(threadIdx.x >> 6);
-    unsigned long long* const slot = lds + wave * lock_slot_words(a.shells);
+    unsigned long long* const slot = lds + wave * lock_wave_words(SAMPLER, a.shells);
     for (uint32_t i = lane; i < lock_slot_words(a.shells); i += 64u)
         slot[i] = 0;
 
@@ -338,18 +472,25 @@ __global__ void __launch_bounds__(256) walk_lock(LockArgs a)
         lt.deposit = in;
         LockPhoton p = { 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 1.0f, ~0u };
         tmc_philox_photon pp;
+        uint32_t plo; /* low index word */
         {
             const LockArgs& c = args_here<LockArgs>();
             uint32_t off = place + at + lane;
             if (c.level && __builtin_amdgcn_inverse_ballot_w64(in))
                 off = lock_load(p, c.in, off);
             const uint64_t photon = c.first_photon + off;
+            plo = (uint32_t)photon;
             pp = tmc_philox_photon_init((uint32_t)photon, (uint32_t)(photon >> 32), phys.key0, phys.key1);
         }
-        lock_cycle<MATH>(p, k0, k1, table, zero, c3k1, pp, phys, lt, room, [&]() {
+        const auto flush = [&]() {
             const LockArgs& c = args_here<LockArgs>();
             lock_flush(slot, lock_block(c, wave) + TMC_COHORT_COUNTERS, c.shells, lane);
-        });
+        };
+        if constexpr (SAMPLER == 1u)
+            lock_cycle_rejection<MATH>(p, k0, k1, table, zero, c3k1 ^ phys.key1, plo, pp, phys, lt,
+                                       slot + lock_slot_words(a.shells), room, flush);
+        else
+            lock_cycle<MATH>(p, k0, k1, table, zero, c3k1, pp, phys, lt, room, flush);
         interactions += (uint64_t)__popcll(in) * (k1 - k0);
         const LockArgs& c = args_here<LockArgs>();
         uint64_t S = c.cut_ends ? in & __ballot(p.x3 < TMC_ROULETTE_KILL_R) : in;
@@ -506,20 +647,26 @@ namespace {
 
 using LockKernel = void (*)(LockArgs);
 
-LockKernel lock_kernel(uint32_t math) { return math == TMC_MATH_OWN ? walk_lock<TMC_MATH_OWN> : walk_lock<TMC_MATH_HARDWARE>; }
+LockKernel lock_kernel(uint32_t sampler, uint32_t math)
+{
+    if (math == TMC_MATH_OWN)
+        return sampler ? walk_lock<1u, TMC_MATH_OWN> : walk_lock<0u, TMC_MATH_OWN>;
+    return sampler ? walk_lock<1u, TMC_MATH_HARDWARE> : walk_lock<0u, TMC_MATH_HARDWARE>;
+}
 
 } // namespace
 
-hipError_t launch_lock(uint32_t math, const LockArgs& a, uint32_t grid, uint32_t block, hipStream_t stream)
+hipError_t launch_lock(uint32_t sampler, uint32_t math, const LockArgs& a, uint32_t grid, uint32_t block, hipStream_t stream)
 {
-    hipLaunchKernelGGL(lock_kernel(math), dim3(grid), dim3(block), lock_lds_bytes(a.shells, block), stream, a);
+    hipLaunchKernelGGL(lock_kernel(sampler, math), dim3(grid), dim3(block), lock_lds_bytes(sampler, a.shells, block),
+                       stream, a);
     return hipGetLastError();
 }
 
-hipError_t lock_occupancy(uint32_t math, uint32_t block, uint32_t shells, int* wg_per_cu)
+hipError_t lock_occupancy(uint32_t sampler, uint32_t math, uint32_t block, uint32_t shells, int* wg_per_cu)
 {
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(wg_per_cu, lock_kernel(math), (int)block,
-                                                        lock_lds_bytes(shells, block));
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(wg_per_cu, lock_kernel(sampler, math), (int)block,
+                                                        lock_lds_bytes(sampler, shells, block));
 }
 
 namespace {
@@ -535,14 +682,14 @@ LockSetsKernel lock_sets_kernel(uint32_t math)
 
 hipError_t launch_lock_sets(uint32_t math, const LockSetArgs& a, uint32_t grid, uint32_t block, hipStream_t stream)
 {
-    hipLaunchKernelGGL(lock_sets_kernel(math), dim3(grid), dim3(block), lock_lds_bytes(a.shells_max, block), stream, a);
+    hipLaunchKernelGGL(lock_sets_kernel(math), dim3(grid), dim3(block), lock_lds_bytes(0u, a.shells_max, block), stream, a);
     return hipGetLastError();
 }
 
 hipError_t lock_sets_occupancy(uint32_t math, uint32_t block, uint32_t shells_max, int* wg_per_cu)
 {
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(wg_per_cu, lock_sets_kernel(math), (int)block,
-                                                        lock_lds_bytes(shells_max, block));
+                                                        lock_lds_bytes(0u, shells_max, block));
 }
 
 } // namespace tmc
