@@ -348,6 +348,59 @@ uint32_t list_photons(uint32_t photons, uint32_t stripes)
  * eighth of that for the second. */
 uint32_t list_cap(uint32_t which, uint32_t n) { return (which ? n / 64u : n / 8u) + 256u; }
 
+/* Constants of the precision variants (WalkArgs, PrecArgs): formed in FP64,
+ * each rounded once. */
+template <class Args>
+void precision_constants(const tmc_params* p, Args* a)
+{
+    const double mu_a = p->mu_a, mu_s = p->mu_s;
+    a->albedo_d = mu_s / (mu_s + mu_a);
+    a->spm_d = 1e4 / (double)p->microns_per_shell / (mu_a + mu_s);
+    const double l2a = std::log2(a->albedo_d), l2s = -std::log2((double)0.1f);
+    a->l2a_hi = (float)l2a;
+    a->l2a_lo = (float)(l2a - (double)a->l2a_hi);
+    a->l2s_hi = (float)l2s;
+    a->l2s_lo = (float)(l2s - (double)a->l2s_hi);
+    a->spm_w = (float)a->spm_d;
+}
+
+/* Room for lists of `bytes` bytes beside the start time and the counters of a
+ * large run, kept for the next one. */
+bool keep_lists(Context* c, size_t bytes)
+{
+    bytes += 4ull * tmc::kRunCounters + 8;
+    if (c->d_lists && c->lists_bytes >= bytes)
+        return true;
+    tmc::release_device(c->d_lists);
+    c->d_lists = nullptr;
+    if (hipMalloc(&c->d_lists, bytes) != hipSuccess) {
+        c->d_lists = nullptr;
+        return false;
+    }
+    c->lists_bytes = bytes;
+    return true;
+}
+
+/* Photons of a run in slices: at most `most` in each, none across a multiple of
+ * 2^32. */
+struct Slice {
+    uint64_t first;
+    uint32_t photons;
+};
+
+std::vector<Slice> slices_of(uint64_t first, uint64_t photons, uint64_t most)
+{
+    std::vector<Slice> slices;
+    for (uint64_t done = 0; done < photons;) {
+        const uint64_t at = first + done;
+        const uint64_t n = std::min<uint64_t>(std::min<uint64_t>(most, photons - done),
+                                              (1ull << 32) - (at & 0xFFFFFFFFull));
+        slices.push_back({ at, (uint32_t)n });
+        done += n;
+    }
+    return slices;
+}
+
 /* One large binary32 run by lockstep waves, level by level, and the cohort
  * walk for the last survivors.  TMC_E_UNSUPPORTED: not one for it. */
 int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* o, uint64_t kcap, uint64_t* tally,
@@ -373,22 +426,14 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
         return TMC_E_UNSUPPORTED;
     if (tmc::cohort_lds_bytes(p->shells, 0) > 160u * 1024u)
         return TMC_E_UNSUPPORTED;
-    /* the lists, counters and start time, kept for the next such run */
+    /* the lists, counters and start time */
     uint32_t log = 20;
     while ((1ull << log) < slice)
         ++log;
     const uint32_t most = list_photons(1u << log, tmc::kStripes);
     const size_t places[2] = { (size_t)tmc::kStripes * list_cap(0, most), (size_t)tmc::kStripes * list_cap(1, most) };
-    if (!c->d_lists || c->lists_log < log) {
-        tmc::release_device(c->d_lists);
-        c->d_lists = nullptr;
-        const size_t bytes = 28 * (places[0] + places[1]) + 4ull * tmc::kRunCounters + 8;
-        if (hipMalloc(&c->d_lists, bytes) != hipSuccess) {
-            c->d_lists = nullptr;
-            return TMC_E_UNSUPPORTED;
-        }
-        c->lists_log = log;
-    }
+    if (!keep_lists(c, 28 * (places[0] + places[1])))
+        return TMC_E_UNSUPPORTED;
     unsigned long long* const start = (unsigned long long*)c->d_lists;
     uint32_t* const counters = (uint32_t*)(start + 1);
     tmc::PhotonList lists[2];
@@ -401,19 +446,7 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
             at += places[w];
         }
     }
-    /* slices: at most `slice` photons, none across a multiple of 2^32 */
-    struct Slice {
-        uint64_t first;
-        uint32_t photons;
-    };
-    std::vector<Slice> slices;
-    for (uint64_t done = 0; done < p->photons;) {
-        const uint64_t first = o->first_photon + done;
-        const uint64_t n = std::min<uint64_t>(std::min<uint64_t>(slice, p->photons - done),
-                                              (1ull << 32) - (first & 0xFFFFFFFFull));
-        slices.push_back({ first, (uint32_t)n });
-        done += n;
-    }
+    const std::vector<Slice> slices = slices_of(o->first_photon, p->photons, slice);
     const uint32_t words = tmc::kStripes * TMC_LOCK_LINE; /* of a level's counts */
     const uint32_t per_slice = levels * words + TMC_LOCK_RANGES * TMC_LOCK_LINE;
     if (slices.size() * per_slice > tmc::kRunCounters)
@@ -513,6 +546,118 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
     return rc;
 }
 
+/* Photons from which on the survivors of a roulette are packed into full waves:
+ * a wave on each SIMD. */
+constexpr double kPackPhotons = 65536.0;
+
+/* One run with a precision variant's arithmetic by lockstep waves.
+ * TMC_E_UNSUPPORTED: not one for them. */
+int run_prec(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* o, uint64_t kcap, uint64_t* tally,
+             tmc_run_stats* st)
+{
+    if (p->photons == 0 || p->photons > (1ull << 36) || p->shells > TMC_LOCK_SHELLS || kcap != 0xFFFFFFFFull)
+        return TMC_E_UNSUPPORTED;
+    tmc::PrecArgs a;
+    std::memset(&a, 0, sizeof a);
+    precision_constants(p, &a);
+    if (!(a.albedo_d > 0.0 && a.albedo_d < 1.0))
+        return TMC_E_UNSUPPORTED;
+    a.seed = seed;
+    a.shell_max = (float)(p->shells - 1);
+    a.shells = p->shells;
+    const uint64_t slice = std::min<uint64_t>(p->photons, 1ull << tmc::kSliceLog);
+    /* the table: the cuts that the last survivors are expected to need, each
+     * cycle's length from its logarithm, and slack for the roundings on the way */
+    const double l = -std::log(a.albedo_d), first = std::log(1000.0) / l, later = std::log(10.0) / l;
+    a.cuts = cuts_for((double)slice);
+    const double room = 1.001 * (first + a.cuts * later) + 3.0 * a.cuts + 64.0;
+    if (room > (double)tmc::kTableEntries - 16.0)
+        return TMC_E_UNSUPPORTED;
+    a.entries = (uint32_t)room;
+    a.entry = c->d_table;
+
+    /* launches: through one roulette each, while the survivors fill the chip */
+    uint32_t packs = 0;
+    for (double rest = (double)slice; rest > kPackPhotons; rest *= 0.1)
+        ++packs;
+    const uint32_t most = list_photons((uint32_t)slice, tmc::kStripes);
+    const uint32_t planes = 1u + tmc::prec_words(o->precision);
+    const size_t places[2] = { packs > 0 ? (size_t)tmc::kStripes * list_cap(0, most) : 0,
+                               packs > 1 ? (size_t)tmc::kStripes * list_cap(1, most) : 0 };
+    if (!keep_lists(c, sizeof(tmc::PrecHead) + 4ull * planes * (places[0] + places[1])))
+        return TMC_E_UNSUPPORTED;
+    unsigned long long* const start = (unsigned long long*)c->d_lists;
+    uint32_t* const counters = (uint32_t*)(start + 1);
+    a.head = (tmc::PrecHead*)(counters + tmc::kRunCounters);
+    uint32_t* at = (uint32_t*)(a.head + 1);
+    tmc::PrecList lists[2];
+    for (uint32_t w = 0; w < 2; ++w) {
+        lists[w] = { at, at + places[w], (uint32_t)places[w] };
+        at += planes * places[w];
+    }
+    const std::vector<Slice> slices = slices_of(o->first_photon, p->photons, slice);
+    const uint32_t words = tmc::kStripes * TMC_LOCK_LINE; /* of a list's counts */
+    if (slices.size() * packs * words > tmc::kRunCounters)
+        return TMC_E_UNSUPPORTED;
+
+    const uint32_t block = 256, cus = (uint32_t)c->compute_units;
+    int per_cu = 0;
+    if (tmc::prec_occupancy(o->sampler, o->precision, block, p->shells, &per_cu) != hipSuccess || per_cu <= 0)
+        return TMC_E_HIP;
+    const uint32_t grid_most = (uint32_t)per_cu * cus;
+    a.copies = 8;
+    a.work = c->d_work;
+    tmc::CohortArgs f;
+    std::memset(&f, 0, sizeof f);
+    f.shells = p->shells;
+    f.copies = a.copies;
+    f.finish = 1;
+    f.list.photon = counters; /* (the sums are others', even with one workgroup) */
+    f.start = start;
+    f.token = ++c->token;
+    f.work = c->d_work;
+    f.out = c->d_out;
+    uint32_t grid0 = 0;
+    const int rc = finish_enqueued(c, f.token, p->shells, tally, st, [&]() {
+        if (tmc::launch_prec_table(o->precision, a, counters, (uint32_t)slices.size() * packs * words, start, c->stream)
+            != hipSuccess)
+            return false;
+        for (size_t si = 0; si < slices.size(); ++si) {
+            uint32_t* const count = counters + si * packs * words;
+            double n = (double)slices[si].photons;
+            const uint32_t wgs = (uint32_t)std::min<double>(grid_most, std::ceil(n / 256.0));
+            a.stripes = std::min(std::min(tmc::kStripes, cus), std::max(1u, wgs / 8u));
+            const uint32_t per = list_photons(slices[si].photons, a.stripes);
+            a.first_photon = slices[si].first;
+            a.photons = slices[si].photons;
+            for (uint32_t level = 0; level <= packs; ++level, n *= 0.1) {
+                a.level = level;
+                a.cycles = level < packs ? 1u : 0u;
+                a.in = lists[(level + 1) & 1u];
+                a.out = lists[level & 1u];
+                a.in_count = count + (level ? level - 1 : 0) * words;
+                a.in_cap = a.out_cap;
+                a.out_count = count + level * words;
+                a.out_cap = list_cap(level & 1u, per);
+                const uint32_t grid = std::max(a.stripes, (uint32_t)std::min<double>(grid_most, std::ceil(n / 256.0)));
+                if (level == 0)
+                    grid0 = grid;
+                if (tmc::launch_prec(o->sampler, o->precision, a, grid, block, c->stream) != hipSuccess)
+                    return false;
+            }
+        }
+        return tmc::launch_finish(f, c->stream) == hipSuccess;
+    });
+    if (rc == TMC_OK && c->h_out[2] >= TMC_LOCK_OVERFLOW)
+        return TMC_E_UNSUPPORTED;
+    if (rc == TMC_OK && st) {
+        st->grid = grid0;
+        st->block = block;
+        st->chunk = 64;
+    }
+    return rc;
+}
+
 } // namespace
 
 int tmc::run_walk(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* o, unsigned long long* work,
@@ -537,13 +682,17 @@ int tmc::run_walk(Context* c, const tmc_params* p, uint64_t seed, const tmc_opti
     if (o->reserved)
         return TMC_E_INVALID;
     const uint32_t table_k = tmc::weight_table_entries(p, o->precision, p->photons, o->weight_table);
-    /* the cohort and lockstep walks: binary32 runs of the allocating entry point
-     * with no launch shape or table asked for (cohort_shape has the sizes) */
-    if (work == c->d_work && o->precision == TMC_PRECISION_FP32 && !o->block && !o->grid && !o->chunk
-        && !o->weight_table) {
-        int rc = run_cohort(c, p, seed, o, kcap, tally, st);
-        if (rc == TMC_E_UNSUPPORTED)
-            rc = run_lock(c, p, seed, o, kcap, tally, st);
+    /* the cohort and lockstep walks: runs of the allocating entry point with no
+     * launch shape or table asked for (cohort_shape has the sizes) */
+    if (work == c->d_work && !o->block && !o->grid && !o->chunk && !o->weight_table) {
+        int rc;
+        if (o->precision == TMC_PRECISION_FP32) {
+            rc = run_cohort(c, p, seed, o, kcap, tally, st);
+            if (rc == TMC_E_UNSUPPORTED)
+                rc = run_lock(c, p, seed, o, kcap, tally, st);
+        } else {
+            rc = run_prec(c, p, seed, o, kcap, tally, st);
+        }
         if (rc == TMC_OK && st) {
             st->photons = p->photons;
             st->total_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -596,16 +745,7 @@ int tmc::run_walk(Context* c, const tmc_params* p, uint64_t seed, const tmc_opti
     a.shell_max = (float)(S - 1);
     a.shells = S;
     a.chunk = chunk;
-    /* precision variants: constants in FP64, each rounded once */
-    const double mu_a = p->mu_a, mu_s = p->mu_s;
-    a.albedo_d = mu_s / (mu_s + mu_a);
-    a.spm_d = 1e4 / (double)p->microns_per_shell / (mu_a + mu_s);
-    const double l2a = std::log2(a.albedo_d), l2s = -std::log2((double)0.1f);
-    a.l2a_hi = (float)l2a;
-    a.l2a_lo = (float)(l2a - (double)a.l2a_hi);
-    a.l2s_hi = (float)l2s;
-    a.l2s_lo = (float)(l2s - (double)a.l2s_hi);
-    a.spm_w = (float)a.spm_d;
+    precision_constants(p, &a);
     /* Each wave swaps the workgroup's LDS sums out at least every
      * flush_interval steps, so between two swaps of one entry at most
      * waves_per_wg * 64 * flush_interval deposits of at most 2^43 (heat2

@@ -165,6 +165,62 @@ hipError_t launch_cohort_sets(uint32_t math, const LockSetArgs& a, uint32_t grid
 /* Builds the weight tables of nsets sets. */
 hipError_t launch_weigh_sets(const LockSet* sets, uint32_t nsets, CohortHead* heads, void* entry, hipStream_t stream);
 
+/* ---- the precision variants (tmc_lock_prec.hip) ---- */
+
+/* Weight table of a precision variant: cuts as CohortArgs. */
+struct PrecHead {
+    uint32_t ncuts, pad;
+    double w_end;
+    uint32_t cut[TMC_COHORT_CUTS];
+};
+
+/* A list of photons between two roulettes: index in the slice, and the words of
+ * position and direction, word w of place i at state[w * places + i]. */
+struct PrecList {
+    uint32_t *photon, *state;
+    uint32_t places;
+};
+
+/* Words of a photon's position and direction. */
+__host__ __device__ constexpr uint32_t prec_words(uint32_t precision)
+{
+    return precision == 3u ? 12u : precision == 2u ? 9u : 6u;
+}
+
+/* One launch of a run with a precision variant's arithmetic: the photons of a
+ * slice, or of the list the launch before left, through `cycles` roulettes
+ * (0: to their end). */
+struct PrecArgs {
+    uint64_t seed; /* Philox key */
+    uint64_t first_photon; /* index of the slice's photon 0 */
+    double albedo_d, spm_d; /* as WalkArgs */
+    float l2a_hi, l2a_lo, l2s_hi, l2s_lo, spm_w, shell_max;
+    uint32_t shells;
+    uint32_t level, cycles; /* roulettes survived so far (0: the slice's photons), and to come */
+    uint32_t photons; /* of the slice (< 2^31) */
+    PrecHead* head;
+    void* entry; /* pairs of images, at least one entry beyond the last cut */
+    uint32_t entries, cuts; /* room of the table, and roulettes wanted */
+    uint32_t stripes; /* of the lists, as LockArgs */
+    PrecList in, out;
+    const uint32_t* in_count;
+    uint32_t* out_count;
+    uint32_t in_cap, out_cap;
+    uint32_t copies;
+    unsigned long long* work; /* as CohortArgs */
+};
+
+hipError_t prec_occupancy(uint32_t sampler, uint32_t precision, uint32_t block, uint32_t shells, int* wg_per_cu);
+/* Builds the weight table, zeroes `counters` 32-bit words at `counter` and
+ * notes the real time at *start. */
+hipError_t launch_prec_table(uint32_t precision, const PrecArgs& a, uint32_t* counter, uint32_t counters,
+                             unsigned long long* start, hipStream_t stream);
+hipError_t launch_prec(uint32_t sampler, uint32_t precision, const PrecArgs& a, uint32_t grid, uint32_t block,
+                       hipStream_t stream);
+/* Ends a run whose launches have left their sums in a.work (shells, copies,
+ * work, start, token and out of CohortArgs). */
+hipError_t launch_finish(const CohortArgs& a, hipStream_t stream);
+
 /* Converts n weights (host memory) to table entries of 16 bytes, zeroes
  * `counters` 32-bit words at `counter`, and notes the real time at *start
  * (null: neither). */

@@ -756,6 +756,17 @@ __global__ void __launch_bounds__(1024) walk_cohort(CohortArgs a)
     finish_run(a, l.tally, l.flag, wave == drawing && lane == 0, counts.interactions, counts.truncated, counts.flushed);
 }
 
+/* One workgroup: adds up the sums that other launches left in a.work, and
+ * hands the result over. */
+__global__ void __launch_bounds__(1024) finish_kernel(CohortArgs a)
+{
+    extern __shared__ unsigned long long lds_words[];
+    for (uint32_t i = threadIdx.x; i < cohort_tally_words(a.shells); i += blockDim.x)
+        lds_words[i] = 0;
+    uint32_t* const flag = (uint32_t*)(lds_words + cohort_tally_words(a.shells));
+    finish_run(a, lds_words, flag, false, 0, 0, true);
+}
+
 /* Waves that draw and that move in a workgroup of a batch: cohorts of 64. */
 #define TMC_COHORT_SETS_MOVING 3u
 #define TMC_COHORT_SETS_DRAWING 13u
@@ -925,6 +936,12 @@ hipError_t launch_cohort(uint32_t sampler, uint32_t math, const CohortArgs& a, u
 {
     hipLaunchKernelGGL(cohort_kernel(sampler, math), dim3(grid), dim3(block), cohort_lds_bytes_of(a.shells, a.build),
                        stream, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_finish(const CohortArgs& a, hipStream_t stream)
+{
+    hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(1024), cohort_tally_words(a.shells) * 8u + 16u, stream, a);
     return hipGetLastError();
 }
 

@@ -40,8 +40,8 @@ struct Context {
     unsigned long long* d_out = nullptr;
     float* h_weight = nullptr; /* weights of the run's table (host-coherent memory), and their device address */
     float* d_weight = nullptr;
-    void* d_lists = nullptr; /* survivor lists of large runs, for slices of 2^lists_log photons */
-    uint32_t lists_log = 0;
+    void* d_lists = nullptr; /* survivor lists and counters of large runs */
+    size_t lists_bytes = 0;
     uint64_t token = 0; /* of the last cohort walk */
     bool work_zero = false; /* d_work holds zeros */
     unsigned long long* d_work = nullptr; /* run_work_words(TMC_MAX_SHELLS) words, allocated at the first run */

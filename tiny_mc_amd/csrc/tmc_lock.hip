@@ -30,24 +30,12 @@
  */
 #include "tmc_cohort.h"
 #include "tmc_device.h"
+#include "tmc_lock_device.h"
 #include "tmc_math.h"
 #include "tmc_philox.h"
 #include "tmc_step.h"
 
 namespace tmc {
-
-/* Copies of the overflow shell's sums in a wave's slot (16: 1% slower). */
-#define TMC_LOCK_HOT 8u
-static_assert(TMC_LOCK_HOT <= TMC_CHECK_HOT, "the shell check covers every overflow copy");
-
-/* Steps between two flushes of a wave's slot: a word takes fewer than 2^20
- * deposits of at most 2^43 each, so it stays below 2^63. */
-#define TMC_LOCK_FLUSH_STEPS 16383u
-
-__host__ __device__ __forceinline__ size_t lock_slot_words(uint32_t shells)
-{
-    return 2u * ((size_t)shells - 1u + TMC_LOCK_HOT);
-}
 
 /* Absorptions the rejection sampler's waves walk at a time, and the LDS words
  * of the directions they draw again. */
@@ -65,75 +53,6 @@ size_t lock_lds_bytes(uint32_t sampler, uint32_t shells, uint32_t block)
 }
 
 namespace {
-
-typedef uint32_t Images __attribute__((ext_vector_type(4)));
-
-/* Philox block (k, 0) of photons with one high counter word and one k (both
- * wave-uniform): what rounds 1 and 2 make of k is scalar.  c3k1: the high
- * counter word ^ key1. */
-__device__ __forceinline__ tmc_u32x4 block0_uniform(uint32_t k, uint32_t c3k1, const tmc_philox_photon& pp,
-                                                    const tmc_philox_keys& ks)
-{
-    const uint64_t q0 = (uint64_t)k * TMC_PHILOX_M0;
-    const uint64_t p1 = (uint64_t)((uint32_t)(q0 >> 32) ^ c3k1) * TMC_PHILOX_M1;
-    uint32_t c0 = pp.c1r1 ^ ((uint32_t)(p1 >> 32) ^ ks.k0[1]), c2 = pp.c2r2k ^ (uint32_t)q0;
-    uint64_t a = (uint64_t)c0 * TMC_PHILOX_M0, b = (uint64_t)c2 * TMC_PHILOX_M1;
-    c0 = (uint32_t)(b >> 32) ^ ((uint32_t)p1 ^ ks.k0[2]);
-    c2 = tmc_xor3((uint32_t)(a >> 32), pp.c3r2, ks.k1[2]);
-    uint32_t c1 = (uint32_t)b, c3 = (uint32_t)a;
-#pragma unroll
-    for (int round = 3; round < 10; ++round) {
-        a = (uint64_t)c0 * TMC_PHILOX_M0;
-        b = (uint64_t)c2 * TMC_PHILOX_M1;
-        c0 = tmc_xor3((uint32_t)(b >> 32), c1, ks.k0[round]);
-        c2 = tmc_xor3((uint32_t)(a >> 32), c3, ks.k1[round]);
-        c1 = (uint32_t)b;
-        c3 = (uint32_t)a;
-    }
-    return tmc_u32x4{ c0, c1, c2, c3 };
-}
-
-/* Moves a wave's slot into its block of the global sums and zeroes it. */
-__device__ __forceinline__ void lock_flush(unsigned long long* slot, unsigned long long* g, uint32_t shells,
-                                           uint32_t lane)
-{
-    const uint32_t last = shells - 1u;
-    for (uint32_t q = lane; q < last + TMC_LOCK_HOT; q += 64u) {
-        const unsigned long long a = slot[2u * q], b = slot[2u * q + 1u];
-        slot[2u * q] = 0;
-        slot[2u * q + 1u] = 0;
-        const uint32_t s = q < last ? q : last;
-        unsigned long long oa = 0, ob = 0;
-        if (a)
-            oa = atomicAdd(g + 2u * s, a);
-        if (b)
-            ob = atomicAdd(g + 2u * shells + 2u * s, b);
-        if (oa + a < oa)
-            atomicAdd(g + 2u * s + 1u, 1ull);
-        if (ob + b < ob)
-            atomicAdd(g + 2u * shells + 2u * s + 1u, 1ull);
-    }
-}
-
-/* The block of global sums this wave flushes into. */
-__device__ __forceinline__ unsigned long long* lock_block(const LockArgs& a, uint32_t wave)
-{
-    return a.work
-        + (size_t)((blockIdx.x * (blockDim.x >> 6) + wave) % a.copies) * (TMC_COHORT_COUNTERS + 4u * a.shells);
-}
-
-/* The kernel's arguments where a path between two cycles uses them: read
- * through the argument block's pointer passed through an empty asm, so that
- * no load is hoisted into the step loop, whose scalar registers hold the
- * round keys. */
-template <class Args>
-__device__ __forceinline__ const Args& args_here()
-{
-    typedef const __attribute__((address_space(4))) Args* ConstArgs;
-    ConstArgs p = (ConstArgs)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(p));
-    return *(const Args*)p;
-}
 
 /* Photon state of a lane. */
 struct LockPhoton {
@@ -401,7 +320,7 @@ __device__ __forceinline__ bool lock_append(uint64_t S, uint32_t off, const Lock
 
 /* (LockArgs must stay the only parameter: args_here) */
 template <uint32_t SAMPLER, uint32_t MATH>
-__global__ void __launch_bounds__(256, SAMPLER ? 6 : 8) walk_lock(LockArgs a)
+__global__ void __launch_bounds__(256, SAMPLER ? 6 : 1) walk_lock(LockArgs a)
 {
     extern __shared__ unsigned long long lds[];
     const uint32_t lane = __lane_id();

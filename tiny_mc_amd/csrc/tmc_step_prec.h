@@ -108,12 +108,11 @@ __device__ __forceinline__ void compensated_move(float& x, float& xl, float t, f
     xl = lo - (x - s);
 }
 
-template <uint32_t SAMPLER, bool COMP>
-__device__ __forceinline__ bool step(PhotonW& p, const PhysicsW& ph, const LaneTally& lt)
+/* Moves p by the step of block (k, 0) (photon.c:21-24); returns the tally pair
+ * of where it is then (photon.c:26-29). */
+template <bool COMP>
+__device__ __forceinline__ uint32_t move(PhotonW& p, const tmc_u32x4& r, const PhysicsW& ph, const LaneTally& lt)
 {
-    const tmc_u32x4 r = tmc_philox4x32_10_block0(p.k, p.pp, ph.key0, ph.key1); /* block (k, 0) */
-
-    /* move (photon.c:21-24) */
     const float t = -log32_u24(tmc_u24(r.x0)); /* = -log32(tmc_u01(r.x0)) */
     if (COMP) {
         compensated_move(p.x, p.xl, t, p.u);
@@ -125,14 +124,16 @@ __device__ __forceinline__ bool step(PhotonW& p, const PhysicsW& ph, const LaneT
         p.z = __builtin_fmaf(t, p.w, p.z);
     }
 
-    /* absorb (photon.c:26-32) */
     const float r2 = __builtin_fmaf(p.z, p.z, __builtin_fmaf(p.y, p.y, p.x * p.x));
     const float f = sqrt_radius(r2) * ph.spm;
-    tally_add(lt, tally_pair(lt, f < ph.shell_max, (uint32_t)f), fx_heat(p.weight), fx_heat2(p.weight));
-    ++p.e;
-    p.weight = weight_from_counts(p.e, p.r, ph);
+    return tally_pair(lt, f < ph.shell_max, (uint32_t)f);
+}
 
-    /* new direction (photon.c:34-43), as the FP32 step */
+/* New direction of p from block (k, 0) and, where attempts are rejected,
+ * blocks (k, 1) and on (photon.c:34-43), as the FP32 step. */
+template <uint32_t SAMPLER>
+__device__ __forceinline__ void turn(PhotonW& p, const tmc_u32x4& r, const PhysicsW& ph)
+{
     if (SAMPLER == 1u) {
         uint32_t w0 = r.x1, w1 = r.x2;
         tmc_u32x4 blk = { 0u, 0u, 0u, 0u };
@@ -167,6 +168,18 @@ __device__ __forceinline__ bool step(PhotonW& p, const PhysicsW& ph, const LaneT
         p.v = s * cs;
         p.w = s * sn;
     }
+}
+
+template <uint32_t SAMPLER, bool COMP>
+__device__ __forceinline__ bool step(PhotonW& p, const PhysicsW& ph, const LaneTally& lt)
+{
+    const tmc_u32x4 r = tmc_philox4x32_10_block0(p.k, p.pp, ph.key0, ph.key1); /* block (k, 0) */
+
+    /* absorb (photon.c:21-32) */
+    tally_add(lt, move<COMP>(p, r, ph, lt), fx_heat(p.weight), fx_heat2(p.weight));
+    ++p.e;
+    p.weight = weight_from_counts(p.e, p.r, ph);
+    turn<SAMPLER>(p, r, ph);
     ++p.k;
 
     /* roulette (photon.c:45-49): a survival multiplies by 1/0.1f */
@@ -213,23 +226,21 @@ __device__ __forceinline__ void launch_photon(Photon64& p, uint64_t photon, uint
 __device__ __forceinline__ uint64_t fx_heat64(double w) { return (uint64_t)__double2ull_rn(w * 0x1p33); }
 __device__ __forceinline__ uint64_t fx_heat2_64(double w) { return (uint64_t)__double2ull_rn((w * w) * 0x1p43); }
 
-template <uint32_t SAMPLER>
-__device__ __forceinline__ bool step(Photon64& p, const Physics64& ph, const LaneTally& lt)
+/* As for PhotonW. */
+__device__ __forceinline__ uint32_t move(Photon64& p, const tmc_u32x4& r, const Physics64& ph, const LaneTally& lt)
 {
-    const tmc_u32x4 r = tmc_philox4x32_10_block0(p.k, p.pp, ph.key0, ph.key1); /* block (k, 0) */
-
-    /* move (photon.c:21-24) */
     const double t = -log((double)tmc_u01(r.x0));
     p.x += t * p.u;
     p.y += t * p.v;
     p.z += t * p.w;
 
-    /* absorb (photon.c:26-32) */
     const double f = sqrt(p.x * p.x + p.y * p.y + p.z * p.z) * ph.spm;
-    tally_add(lt, tally_pair(lt, f < ph.shell_max, (uint32_t)f), fx_heat64(p.weight), fx_heat2_64(p.weight));
-    p.weight *= ph.albedo;
+    return tally_pair(lt, f < ph.shell_max, (uint32_t)f);
+}
 
-    /* new direction (photon.c:34-43) */
+template <uint32_t SAMPLER>
+__device__ __forceinline__ void turn(Photon64& p, const tmc_u32x4& r, const Physics64& ph)
+{
     if (SAMPLER == 1u) {
         uint32_t w0 = r.x1, w1 = r.x2;
         tmc_u32x4 blk = { 0u, 0u, 0u, 0u };
@@ -263,6 +274,17 @@ __device__ __forceinline__ bool step(Photon64& p, const Physics64& ph, const Lan
         p.v = s * cs;
         p.w = s * sn;
     }
+}
+
+template <uint32_t SAMPLER>
+__device__ __forceinline__ bool step(Photon64& p, const Physics64& ph, const LaneTally& lt)
+{
+    const tmc_u32x4 r = tmc_philox4x32_10_block0(p.k, p.pp, ph.key0, ph.key1); /* block (k, 0) */
+
+    /* absorb (photon.c:21-32) */
+    tally_add(lt, move(p, r, ph, lt), fx_heat64(p.weight), fx_heat2_64(p.weight));
+    p.weight *= ph.albedo;
+    turn<SAMPLER>(p, r, ph);
     ++p.k;
 
     /* roulette (photon.c:45-49), the float literals widened as in C */
