@@ -94,3 +94,20 @@ def test_rejection_sampler_against_the_oracle(tmc, orc, hw_tables):
     want, n = orc.mirror32(orc.params(**DEFAULT), 12, 50007, sampler=1, tables=hw_tables)
     assert st.interactions == n
     np.testing.assert_array_equal(tally, want)
+
+
+@pytest.mark.parametrize("math", [0, 1])
+@pytest.mark.parametrize("phys,photons,first,kmax", [
+    (DEFAULT, (1 << 22) + 1001, (1 << 32) - (1 << 21), 0), (LOWALB, (1 << 25) + 77, 0, 0),
+    (DEFAULT, (1 << 23) + 5, 0, 50), (DEFAULT, (1 << 22) + 3, 0, 73), (dict(DEFAULT, shells=133), 5000001, 0, 0),
+    (dict(DEFAULT, shells=134), 5000001, 0, 0), (dict(DEFAULT, shells=1), 5000001, 0, 0)])
+def test_counted_first_cycles(tmc, phys, photons, first, kmax, math):
+    """First cycles of 3e8 absorptions and more, counted by absorption and shell
+    where the counts fit (at 73 absorptions up to 133 shells)."""
+    print(f"lock counted: {phys} photons={photons} first={first} kmax={kmax} math={math}", flush=True)
+    p = tmc.Params(photons=photons, **phys)
+    kw = dict(first_photon=first, math=math, max_interactions=kmax)
+    got, st = tmc.run_raw(p, 31, **kw)
+    want, ws = tmc.run_raw(p, 31, block=256, **kw)
+    np.testing.assert_array_equal(got, want)
+    assert (st.interactions, st.truncated) == (ws.interactions, ws.truncated)

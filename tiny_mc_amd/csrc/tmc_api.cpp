@@ -409,12 +409,11 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
     if (p->photons <= TMC_COHORT_PHOTONS || p->photons > (1ull << 40) || p->shells > TMC_LOCK_SHELLS)
         return TMC_E_UNSUPPORTED;
     /* many photons of short walks: launching them 64 at a time and appending
-     * the survivors costs what the step saves (albedo 0.5: 2^23 photons 951 us
-     * lane per photon, 306 us here; 2^27 2841 and 2897 us; the rejection
-     * sampler's step is longer: 2^27 at albedo 0.5 4885 and 4696 us, at 1/6
-     * 2216 and 2306 us) */
-    const double shortest = o->sampler == TMC_SAMPLER_ANALYTIC ? 32.0 : 8.0;
-    if (p->photons > (1ull << 26) && first_cycle(p, kcap) < shortest)
+     * the survivors costs what the step saves (2^27 photons, lane per photon
+     * and here: albedo 1/6 1548 and 1685 us, with the rejection sampler 2216
+     * and 2290 us; albedo 0.5 2849 and 2784 us, 4885 and 4696 us; 2^26 at 1/6
+     * 1049 and 850 us) */
+    if (p->photons > (1ull << 26) && first_cycle(p, kcap) < 8.0)
         return TMC_E_UNSUPPORTED;
     const uint64_t slice = std::min<uint64_t>(p->photons, 1ull << tmc::kSliceLog);
     uint32_t levels = 1;
@@ -456,9 +455,21 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
     /* (the batches go round the resident waves, so a workgroup that had to wait
      * for another to end would double the launch's time) */
     int per_cu = 0;
-    if (tmc::lock_occupancy(o->sampler, o->math, block, p->shells, &per_cu) != hipSuccess || per_cu <= 0)
+    if (tmc::lock_occupancy(o->sampler, o->math, 0u, block, p->shells, &per_cu) != hipSuccess || per_cu <= 0)
         return TMC_E_HIP;
     const uint32_t grid_most = (uint32_t)per_cu * cus;
+    /* the first cycle counted: where the counts of four workgroups fit a CU's
+     * LDS, and a slice has the work to make up for adding them up at the end
+     * (first cycles of 1.6e8 absorptions: 508 us summed, 536 counted; 2.2e8
+     * 528 and 528; 6e8 1231 and 1159; 4.8e9 7.93 and 7.75 ms) */
+    const uint32_t k_first = std::min(a.cut[0], a.kcap);
+    const bool counted = o->sampler == TMC_SAMPLER_ANALYTIC && (double)slice * (double)k_first >= 3e8
+        && tmc::lock_count_bytes(p->shells, k_first) <= 40u * 1024u;
+    int counted_cu = 0;
+    if (counted
+        && (tmc::lock_occupancy(o->sampler, o->math, k_first, TMC_LOCK_COUNTED_BLOCK, p->shells, &counted_cu) != hipSuccess
+            || counted_cu <= 0))
+        return TMC_E_HIP;
     tmc::CohortShape shape;
     tmc::cohort_shape((uint64_t)std::max(1.0, rest), kHandOver + 1u, first_cycle(p, kcap), p->shells, cus, &shape);
     use_shape(shape, &a);
@@ -510,18 +521,27 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
                 l.out_count = count + lv * words;
                 l.out_cap = list_cap(lv & 1u, per);
                 const double waves = std::ceil(n / 64.0);
-                const uint32_t grid = std::max(l.stripes, (uint32_t)std::min<double>(grid_most, std::ceil(waves / 4.0)));
+                const bool by_count = counted && lv == 0;
+                const uint32_t threads = by_count ? TMC_LOCK_COUNTED_BLOCK : block, per_wg = threads / 64u;
+                const uint32_t grid = std::max(
+                    l.stripes, (uint32_t)std::min<double>(by_count ? (uint32_t)counted_cu * cus : grid_most,
+                                                          std::ceil(waves / (double)per_wg)));
                 l.chunk = 0;
                 if (lv == 0) {
                     grid0 = grid;
-                    const uint64_t each = (uint64_t)waves / (4u * grid); /* batches a wave */
+                    const uint64_t each = (uint64_t)waves / (per_wg * grid); /* batches a wave */
                     if (each >= 8) {
-                        l.chunk = 64u * (uint32_t)std::min<uint64_t>(32, std::max<uint64_t>(1, each / 32));
+                        /* a wave's 32nd, but (short cycles) not less than 128
+                         * absorptions: a range's claims take 7 to 16 ns each,
+                         * one after the other (2^24 photons at albedo 0.5 854
+                         * and 509 us, at 1/6 878 and 406 us) */
+                        const uint64_t least = std::min<uint64_t>((127u + l.k1) / l.k1, each / 4);
+                        l.chunk = 64u * (uint32_t)std::min<uint64_t>(32, std::max<uint64_t>(least, each / 32));
                         l.range = (slices[si].photons / TMC_LOCK_RANGES + 64u) / 64u * 64u;
                         l.cursor = count + levels * words;
                     }
                 }
-                if (tmc::launch_lock(o->sampler, o->math, l, grid, block, c->stream) != hipSuccess)
+                if (tmc::launch_lock(o->sampler, o->math, by_count, l, grid, threads, c->stream) != hipSuccess)
                     return false;
             }
             a.finish = si + 1 == slices.size();

@@ -20,7 +20,16 @@
  * walk_f32 -> this walk: 2^20 photons at default physics 425 -> 236 us,
  * 3,000,017 638 -> 500 us, 2^26 8.72 -> 7.87 ms; 2^20 at albedo 0.99 2.73 ->
  * 1.38 ms; 2^17 at albedo 0.9999 117 -> 22 ms; 2^23 at albedo 0.5 951 -> 306
- * us.  With the rejection sampler a step is 133 vector instructions, a third
+ * us.
+ *
+ * Where a first cycle's counts fit LDS (absorptions times shells), a workgroup
+ * counts the photons of each (absorption, shell) instead of adding their images:
+ * one 32-bit addition for two of 64 bits, and no loads of the table, whose
+ * images come in once, when the counts are added up.  2% of a large run
+ * (2^30 photons at default physics 126.6 -> 123.9 ms): the LDS additions are
+ * not what a step waits for.
+ *
+ * With the rejection sampler a step is 133 vector instructions, a third
  * of them the second generator block of the quarter of the directions that
  * are drawn again: 2^17 photons at default physics 304 -> 110 us, 2^24 4.23 ->
  * 3.49 ms, 2^20 at albedo 0.99 5.0 -> 2.75 ms.
@@ -50,6 +59,11 @@ __host__ __device__ __forceinline__ size_t lock_wave_words(uint32_t sampler, uin
 size_t lock_lds_bytes(uint32_t sampler, uint32_t shells, uint32_t block)
 {
     return (block / 64u) * lock_wave_words(sampler, shells) * 8u;
+}
+
+size_t lock_count_bytes(uint32_t shells, uint32_t absorptions)
+{
+    return 4ull * absorptions * (shells - 1ull + TMC_LOCK_HOT);
 }
 
 namespace {
@@ -111,24 +125,89 @@ __device__ __forceinline__ void lock_step(LockPhoton& p, uint32_t k, uint32_t c3
     lock_add(lt, shell_index(r2, phys, lt.fmax), e);
 }
 
-/* Absorptions k and k + 1: both draws ahead of both moves, so that a wave has
- * four independent chains of products to issue from (with few waves on a
- * SIMD the products' latency is what a step costs). */
+/* Absorptions k and k + 1 up to the shells' pairs *qa and *qb: both draws ahead
+ * of both moves, so that a wave has four independent chains of products to
+ * issue from (with few waves on a SIMD the products' latency is what a step
+ * costs). */
+template <uint32_t MATH>
+__device__ __forceinline__ void lock_walk2(LockPhoton& p, uint32_t k, uint32_t c3k1, const tmc_philox_photon& pp,
+                                           const Physics& phys, float fmax, uint32_t* qa, uint32_t* qb)
+{
+    const Drawn a = lock_draw<MATH>(k, c3k1, pp, phys), b = lock_draw<MATH>(k + 1u, c3k1, pp, phys);
+    const float ra = lock_move(p, a), rb = lock_move(p, b);
+    bool sa, sb;
+    float fa = shell_coord_short(ra, phys, fmax, &sa), fb = shell_coord_short(rb, phys, fmax, &sb);
+    if (__builtin_expect(__ballot(!(sa && sb)) != 0, 0)) {
+        fa = (float)shell_index(ra, phys, fmax);
+        fb = (float)shell_index(rb, phys, fmax);
+    }
+    *qa = (uint32_t)fa;
+    *qb = (uint32_t)fb;
+}
+
 template <uint32_t MATH>
 __device__ __forceinline__ void lock_step2(LockPhoton& p, uint32_t k, uint32_t c3k1, const tmc_philox_photon& pp,
                                            const Physics& phys, const LaneTally& lt, const Images& e0,
                                            const Images& e1)
 {
-    const Drawn a = lock_draw<MATH>(k, c3k1, pp, phys), b = lock_draw<MATH>(k + 1u, c3k1, pp, phys);
-    const float ra = lock_move(p, a), rb = lock_move(p, b);
-    bool sa, sb;
-    float fa = shell_coord_short(ra, phys, lt.fmax, &sa), fb = shell_coord_short(rb, phys, lt.fmax, &sb);
-    if (__builtin_expect(__ballot(!(sa && sb)) != 0, 0)) {
-        fa = (float)shell_index(ra, phys, lt.fmax);
-        fb = (float)shell_index(rb, phys, lt.fmax);
+    uint32_t qa, qb;
+    lock_walk2<MATH>(p, k, c3k1, pp, phys, lt.fmax, &qa, &qb);
+    lock_add(lt, qa, e0);
+    lock_add(lt, qb, e1);
+}
+
+/* The wave's photons from their launch to absorption k1, counted: `row` holds
+ * a count for every pair and absorption, `pairs` to an absorption. */
+template <uint32_t MATH>
+__device__ __forceinline__ void lock_cycle_counted(LockPhoton& p, uint32_t k1, uint32_t c3k1,
+                                                   const tmc_philox_photon& pp, const Physics& phys,
+                                                   const LaneTally& lt, uint32_t* row, uint32_t pairs)
+{
+    uint32_t k = 0;
+    for (; k + 2u <= k1; k += 2u, row += 2u * pairs) {
+        uint32_t qa, qb;
+        lock_walk2<MATH>(p, k, c3k1, pp, phys, lt.fmax, &qa, &qb);
+        if (__builtin_amdgcn_inverse_ballot_w64(lt.deposit)) {
+            atomicAdd(row + qa, 1u);
+            atomicAdd(row + pairs + qb, 1u);
+        }
     }
-    lock_add(lt, (uint32_t)fa, e0);
-    lock_add(lt, (uint32_t)fb, e1);
+    if (k != k1) {
+        const float r2 = lock_move(p, lock_draw<MATH>(k, c3k1, pp, phys));
+        const uint32_t q = shell_index(r2, phys, lt.fmax);
+        if (__builtin_amdgcn_inverse_ballot_w64(lt.deposit))
+            atomicAdd(row + q, 1u);
+    }
+}
+
+/* Adds a workgroup's counts, each times its absorption's images, to a block of
+ * the global sums. */
+__device__ __forceinline__ void count_flush(const uint32_t* counts, const Images* entry, uint32_t k1,
+                                            unsigned long long* g, uint32_t shells)
+{
+    const uint32_t last = shells - 1u, pairs = last + TMC_LOCK_HOT;
+    const uint32_t parts = pairs < blockDim.x ? blockDim.x / pairs : 1u; /* threads to a pair */
+    for (uint32_t i = threadIdx.x; i < pairs * parts; i += blockDim.x) {
+        const uint32_t q = i % pairs;
+        unsigned __int128 h = 0, h2 = 0;
+        for (uint32_t k = i / pairs; k < k1; k += parts) {
+            const uint32_t n = counts[k * pairs + q];
+            const Images e = entry[k];
+            h += (unsigned __int128)(((uint64_t)e.y << 32) | e.x) * n;
+            h2 += (unsigned __int128)(((uint64_t)e.w << 32) | e.z) * n;
+        }
+        const uint32_t s = q < last ? q : last;
+        for (uint32_t w = 0; w < 2u; ++w) {
+            const unsigned __int128 v = w ? h2 : h;
+            if (v == 0)
+                continue;
+            unsigned long long* const at = g + 2u * (w * shells + s);
+            const unsigned long long lo = (unsigned long long)v, old = atomicAdd(at, lo);
+            const unsigned long long hi = (unsigned long long)(v >> 64) + (old + lo < old);
+            if (hi)
+                atomicAdd(at + 1, hi);
+        }
+    }
 }
 
 /* Orders a wave's LDS accesses across its lanes (the LDS serves them in the
@@ -319,15 +398,23 @@ __device__ __forceinline__ bool lock_append(uint64_t S, uint32_t off, const Lock
 } // namespace
 
 /* (LockArgs must stay the only parameter: args_here) */
-template <uint32_t SAMPLER, uint32_t MATH>
-__global__ void __launch_bounds__(256, SAMPLER ? 6 : 1) walk_lock(LockArgs a)
+template <uint32_t SAMPLER, uint32_t MATH, bool COUNTED = false>
+__global__ void __launch_bounds__(COUNTED ? TMC_LOCK_COUNTED_BLOCK : 256, SAMPLER ? 6 : 1) walk_lock(LockArgs a)
 {
     extern __shared__ unsigned long long lds[];
     const uint32_t lane = __lane_id();
     const uint32_t wave = rfl32(threadIdx.x >> 6);
-    unsigned long long* const slot = lds + wave * lock_wave_words(SAMPLER, a.shells);
-    for (uint32_t i = lane; i < lock_slot_words(a.shells); i += 64u)
-        slot[i] = 0;
+    unsigned long long* const slot = COUNTED ? lds : lds + wave * lock_wave_words(SAMPLER, a.shells);
+    uint32_t* const counts = (uint32_t*)lds;
+    const uint32_t pairs = a.shells - 1u + TMC_LOCK_HOT;
+    if constexpr (COUNTED) {
+        for (uint32_t i = threadIdx.x; i < a.k1 * pairs; i += blockDim.x)
+            counts[i] = 0u;
+        __syncthreads();
+    } else {
+        for (uint32_t i = lane; i < lock_slot_words(a.shells); i += 64u)
+            slot[i] = 0;
+    }
 
     Physics phys = {};
     phys.albedo = a.albedo;
@@ -405,7 +492,9 @@ __global__ void __launch_bounds__(256, SAMPLER ? 6 : 1) walk_lock(LockArgs a)
             const LockArgs& c = args_here<LockArgs>();
             lock_flush(slot, lock_block(c, wave) + TMC_COHORT_COUNTERS, c.shells, lane);
         };
-        if constexpr (SAMPLER == 1u)
+        if constexpr (COUNTED)
+            lock_cycle_counted<MATH>(p, k1, c3k1, pp, phys, lt, counts, pairs);
+        else if constexpr (SAMPLER == 1u)
             lock_cycle_rejection<MATH>(p, k0, k1, table, zero, c3k1 ^ phys.key1, plo, pp, phys, lt,
                                        slot + lock_slot_words(a.shells), room, flush);
         else
@@ -428,7 +517,12 @@ __global__ void __launch_bounds__(256, SAMPLER ? 6 : 1) walk_lock(LockArgs a)
     }
     const LockArgs& c = args_here<LockArgs>();
     unsigned long long* const block = lock_block(c, wave);
-    lock_flush(slot, block + TMC_COHORT_COUNTERS, c.shells, lane);
+    if constexpr (COUNTED) {
+        __syncthreads();
+        count_flush(counts, (const Images*)c.entry, c.k1, block + TMC_COHORT_COUNTERS, c.shells);
+    } else {
+        lock_flush(slot, block + TMC_COHORT_COUNTERS, c.shells, lane);
+    }
     if (lane == 0) {
         atomicAdd(block + 1, (unsigned long long)interactions);
         if (truncated)
@@ -566,8 +660,10 @@ namespace {
 
 using LockKernel = void (*)(LockArgs);
 
-LockKernel lock_kernel(uint32_t sampler, uint32_t math)
+LockKernel lock_kernel(uint32_t sampler, uint32_t math, bool counted)
 {
+    if (counted) /* (analytic sampler) */
+        return math == TMC_MATH_OWN ? walk_lock<0u, TMC_MATH_OWN, true> : walk_lock<0u, TMC_MATH_HARDWARE, true>;
     if (math == TMC_MATH_OWN)
         return sampler ? walk_lock<1u, TMC_MATH_OWN> : walk_lock<0u, TMC_MATH_OWN>;
     return sampler ? walk_lock<1u, TMC_MATH_HARDWARE> : walk_lock<0u, TMC_MATH_HARDWARE>;
@@ -575,17 +671,20 @@ LockKernel lock_kernel(uint32_t sampler, uint32_t math)
 
 } // namespace
 
-hipError_t launch_lock(uint32_t sampler, uint32_t math, const LockArgs& a, uint32_t grid, uint32_t block, hipStream_t stream)
+hipError_t launch_lock(uint32_t sampler, uint32_t math, bool counted, const LockArgs& a, uint32_t grid, uint32_t block,
+                       hipStream_t stream)
 {
-    hipLaunchKernelGGL(lock_kernel(sampler, math), dim3(grid), dim3(block), lock_lds_bytes(sampler, a.shells, block),
-                       stream, a);
+    const size_t lds = counted ? lock_count_bytes(a.shells, a.k1) : lock_lds_bytes(sampler, a.shells, block);
+    hipLaunchKernelGGL(lock_kernel(sampler, math, counted), dim3(grid), dim3(block), lds, stream, a);
     return hipGetLastError();
 }
 
-hipError_t lock_occupancy(uint32_t sampler, uint32_t math, uint32_t block, uint32_t shells, int* wg_per_cu)
+hipError_t lock_occupancy(uint32_t sampler, uint32_t math, uint32_t counted, uint32_t block, uint32_t shells,
+                          int* wg_per_cu)
 {
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(wg_per_cu, lock_kernel(sampler, math), (int)block,
-                                                        lock_lds_bytes(sampler, shells, block));
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        wg_per_cu, lock_kernel(sampler, math, counted), (int)block,
+        counted ? lock_count_bytes(shells, counted) : lock_lds_bytes(sampler, shells, block));
 }
 
 namespace {
