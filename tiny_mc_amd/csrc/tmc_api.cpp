@@ -451,11 +451,11 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
     if (slices.size() * per_slice > tmc::kRunCounters)
         return TMC_E_UNSUPPORTED;
 
-    const uint32_t block = 256, cus = (uint32_t)c->compute_units;
+    const uint32_t cus = (uint32_t)c->compute_units;
     /* (the batches go round the resident waves, so a workgroup that had to wait
      * for another to end would double the launch's time) */
     int per_cu = 0;
-    if (tmc::lock_occupancy(o->sampler, o->math, 0u, block, p->shells, &per_cu) != hipSuccess || per_cu <= 0)
+    if (tmc::lock_occupancy(o->sampler, o->math, 0u, p->shells, &per_cu) != hipSuccess || per_cu <= 0)
         return TMC_E_HIP;
     const uint32_t grid_most = (uint32_t)per_cu * cus;
     /* the first cycle counted: where the counts of four workgroups fit a CU's
@@ -467,7 +467,7 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
         && tmc::lock_count_bytes(p->shells, k_first) <= 40u * 1024u;
     int counted_cu = 0;
     if (counted
-        && (tmc::lock_occupancy(o->sampler, o->math, k_first, TMC_LOCK_COUNTED_BLOCK, p->shells, &counted_cu) != hipSuccess
+        && (tmc::lock_occupancy(o->sampler, o->math, k_first, p->shells, &counted_cu) != hipSuccess
             || counted_cu <= 0))
         return TMC_E_HIP;
     tmc::CohortShape shape;
@@ -501,7 +501,8 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
             uint32_t* const count = counters + si * per_slice; /* survivors by level */
             double n = (double)slices[si].photons;
             bool capped = false;
-            const uint32_t wgs = (uint32_t)std::min<double>(grid_most, std::ceil(n / 256.0));
+            constexpr uint32_t per_wg = TMC_LOCK_BLOCK / 64u;
+            const uint32_t wgs = (uint32_t)std::min<double>(grid_most, std::ceil(n / TMC_LOCK_BLOCK));
             /* at least eight workgroups a stripe, or one stripe */
             l.stripes = std::min(std::min(tmc::kStripes, cus), std::max(1u, wgs / 8u));
             const uint32_t per = list_photons(slices[si].photons, l.stripes);
@@ -522,7 +523,6 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
                 l.out_cap = list_cap(lv & 1u, per);
                 const double waves = std::ceil(n / 64.0);
                 const bool by_count = counted && lv == 0;
-                const uint32_t threads = by_count ? TMC_LOCK_COUNTED_BLOCK : block, per_wg = threads / 64u;
                 const uint32_t grid = std::max(
                     l.stripes, (uint32_t)std::min<double>(by_count ? (uint32_t)counted_cu * cus : grid_most,
                                                           std::ceil(waves / (double)per_wg)));
@@ -541,7 +541,7 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
                         l.cursor = count + levels * words;
                     }
                 }
-                if (tmc::launch_lock(o->sampler, o->math, by_count, l, grid, threads, c->stream) != hipSuccess)
+                if (tmc::launch_lock(o->sampler, o->math, by_count, l, grid, c->stream) != hipSuccess)
                     return false;
             }
             a.finish = si + 1 == slices.size();
@@ -560,7 +560,7 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
         return TMC_E_UNSUPPORTED;
     if (rc == TMC_OK && st) {
         st->grid = grid0;
-        st->block = block;
+        st->block = TMC_LOCK_BLOCK;
         st->chunk = 64;
     }
     return rc;

@@ -151,16 +151,15 @@ struct LockArgs {
     unsigned long long* work; /* as CohortArgs */
 };
 
-size_t lock_lds_bytes(uint32_t sampler, uint32_t shells, uint32_t block);
-/* LDS of a workgroup that counts the photons of each shell and absorption, and
- * its threads. */
+/* Threads of walk_lock's workgroups. */
+#define TMC_LOCK_BLOCK 512u
+size_t lock_lds_bytes(uint32_t sampler, uint32_t shells);
+/* LDS of a workgroup that counts the photons of each shell and absorption. */
 size_t lock_count_bytes(uint32_t shells, uint32_t absorptions);
-#define TMC_LOCK_COUNTED_BLOCK 512u
 /* Resident workgroups per CU of walk_lock (counted: the absorptions that are
  * counted by shell, 0: none). */
-hipError_t lock_occupancy(uint32_t sampler, uint32_t math, uint32_t counted, uint32_t block, uint32_t shells,
-                          int* wg_per_cu);
-hipError_t launch_lock(uint32_t sampler, uint32_t math, bool counted, const LockArgs& a, uint32_t grid, uint32_t block,
+hipError_t lock_occupancy(uint32_t sampler, uint32_t math, uint32_t counted, uint32_t shells, int* wg_per_cu);
+hipError_t launch_lock(uint32_t sampler, uint32_t math, bool counted, const LockArgs& a, uint32_t grid,
                        hipStream_t stream);
 
 /* The same for the sets of a batch: a level by lockstep waves (0 or 1), and

@@ -51,19 +51,16 @@ namespace tmc {
 #define TMC_LOCK_GROUP 4u
 #define TMC_LOCK_RETRIES (64u * TMC_LOCK_GROUP)
 
-__host__ __device__ __forceinline__ size_t lock_wave_words(uint32_t sampler, uint32_t shells)
+/* LDS of a workgroup: the sums, two totals, and the retries of each wave; or
+ * (lock_count_bytes) the totals and the counts. */
+size_t lock_lds_bytes(uint32_t sampler, uint32_t shells)
 {
-    return lock_slot_words(shells) + (sampler ? TMC_LOCK_RETRIES : 0u);
-}
-
-size_t lock_lds_bytes(uint32_t sampler, uint32_t shells, uint32_t block)
-{
-    return (block / 64u) * lock_wave_words(sampler, shells) * 8u;
+    return 8u * (lock_slot_words(shells) + 2u + (sampler ? TMC_LOCK_BLOCK / 64u * TMC_LOCK_RETRIES : 0u));
 }
 
 size_t lock_count_bytes(uint32_t shells, uint32_t absorptions)
 {
-    return 4ull * absorptions * (shells - 1ull + TMC_LOCK_HOT);
+    return 16u + 4ull * absorptions * (shells - 1ull + TMC_LOCK_HOT);
 }
 
 namespace {
@@ -309,7 +306,7 @@ __device__ __forceinline__ void lock_cycle_rejection(LockPhoton& p, uint32_t k0,
                                                      uint32_t zero, uint32_t hi, uint32_t plo,
                                                      const tmc_philox_photon& pp, const Physics& phys,
                                                      const LaneTally& lt, unsigned long long* retries, uint32_t& room,
-                                                     const Flush& flush)
+                                                     uint32_t every, const Flush& flush)
 {
     constexpr uint32_t G = TMC_LOCK_GROUP;
     for (uint32_t k = k0; k != k1;) {
@@ -323,18 +320,18 @@ __device__ __forceinline__ void lock_cycle_rejection(LockPhoton& p, uint32_t k0,
             lock_group_rejection<MATH, 1u>(p, k, hi, plo, pp, phys, lt, from, zero, retries);
         if (room == 0u) {
             flush();
-            room = TMC_LOCK_FLUSH_STEPS;
+            room = every;
         }
     }
 }
 
 /* The wave's photons from absorption k0 to k1 (lanes without one walk a stale
  * one, their deposits masked).  `table`: the set's weight table; `room`: steps
- * to the next flush of the slot, which `flush` does. */
+ * to the next flush of the slot, which `flush` does, `every` so many. */
 template <uint32_t MATH, class Flush>
 __device__ __forceinline__ void lock_cycle(LockPhoton& p, uint32_t k0, uint32_t k1, const char* table, uint32_t zero,
                                            uint32_t c3k1, const tmc_philox_photon& pp, const Physics& phys,
-                                           const LaneTally& lt, uint32_t& room, const Flush& flush)
+                                           const LaneTally& lt, uint32_t& room, uint32_t every, const Flush& flush)
 {
     for (uint32_t k = k0; k != k1;) {
         const uint32_t left = k1 - k, n = rfl32(left < room ? left : room);
@@ -354,7 +351,7 @@ __device__ __forceinline__ void lock_cycle(LockPhoton& p, uint32_t k0, uint32_t 
         }
         if (room == 0u) {
             flush();
-            room = TMC_LOCK_FLUSH_STEPS;
+            room = every;
         }
     }
 }
@@ -399,22 +396,19 @@ __device__ __forceinline__ bool lock_append(uint64_t S, uint32_t off, const Lock
 
 /* (LockArgs must stay the only parameter: args_here) */
 template <uint32_t SAMPLER, uint32_t MATH, bool COUNTED = false>
-__global__ void __launch_bounds__(COUNTED ? TMC_LOCK_COUNTED_BLOCK : 256, SAMPLER ? 6 : 1) walk_lock(LockArgs a)
+__global__ void __launch_bounds__(TMC_LOCK_BLOCK, SAMPLER ? 6 : 1) walk_lock(LockArgs a)
 {
     extern __shared__ unsigned long long lds[];
     const uint32_t lane = __lane_id();
     const uint32_t wave = rfl32(threadIdx.x >> 6);
-    unsigned long long* const slot = COUNTED ? lds : lds + wave * lock_wave_words(SAMPLER, a.shells);
-    uint32_t* const counts = (uint32_t*)lds;
+    unsigned long long *const totals = lds, *const slot = lds + 2;
+    uint32_t* const counts = (uint32_t*)slot;
     const uint32_t pairs = a.shells - 1u + TMC_LOCK_HOT;
-    if constexpr (COUNTED) {
-        for (uint32_t i = threadIdx.x; i < a.k1 * pairs; i += blockDim.x)
-            counts[i] = 0u;
-        __syncthreads();
-    } else {
-        for (uint32_t i = lane; i < lock_slot_words(a.shells); i += 64u)
-            slot[i] = 0;
-    }
+    for (uint32_t i = threadIdx.x; i < (COUNTED ? a.k1 * pairs : 4u * pairs); i += blockDim.x)
+        counts[i] = 0u; /* (a pair of sums is four words) */
+    if (threadIdx.x < 2u)
+        totals[threadIdx.x] = 0ull;
+    __syncthreads();
 
     Physics phys = {};
     phys.albedo = a.albedo;
@@ -453,7 +447,8 @@ __global__ void __launch_bounds__(COUNTED ? TMC_LOCK_COUNTED_BLOCK : 256, SAMPLE
         stride = 64u * waves_per_wg * ((gridDim.x - stripe + a.stripes - 1u) / a.stripes);
     }
     uint64_t interactions = 0, truncated = 0;
-    uint32_t room = TMC_LOCK_FLUSH_STEPS; /* steps to the next flush */
+    constexpr uint32_t every = lock_flush_steps(TMC_LOCK_BLOCK / 64u);
+    uint32_t room = every; /* steps to the next flush */
 
     if (claims) {
         /* range of this XCD's claims; `claimed`: where the current one ends */
@@ -490,15 +485,15 @@ __global__ void __launch_bounds__(COUNTED ? TMC_LOCK_COUNTED_BLOCK : 256, SAMPLE
         }
         const auto flush = [&]() {
             const LockArgs& c = args_here<LockArgs>();
-            lock_flush(slot, lock_block(c, wave) + TMC_COHORT_COUNTERS, c.shells, lane);
+            lock_flush<true>(slot, lock_block(c) + TMC_COHORT_COUNTERS, c.shells, lane, 64u);
         };
         if constexpr (COUNTED)
             lock_cycle_counted<MATH>(p, k1, c3k1, pp, phys, lt, counts, pairs);
         else if constexpr (SAMPLER == 1u)
             lock_cycle_rejection<MATH>(p, k0, k1, table, zero, c3k1 ^ phys.key1, plo, pp, phys, lt,
-                                       slot + lock_slot_words(a.shells), room, flush);
+                                       slot + lock_slot_words(a.shells) + wave * TMC_LOCK_RETRIES, room, every, flush);
         else
-            lock_cycle<MATH>(p, k0, k1, table, zero, c3k1, pp, phys, lt, room, flush);
+            lock_cycle<MATH>(p, k0, k1, table, zero, c3k1, pp, phys, lt, room, every, flush);
         interactions += (uint64_t)__popcll(in) * (k1 - k0);
         const LockArgs& c = args_here<LockArgs>();
         uint64_t S = c.cut_ends ? in & __ballot(p.x3 < TMC_ROULETTE_KILL_R) : in;
@@ -512,22 +507,13 @@ __global__ void __launch_bounds__(COUNTED ? TMC_LOCK_COUNTED_BLOCK : 256, SAMPLE
                 off = c.in.photon[off];
             if (!lock_append(S, off, p, c.out, c.out_count + stripe * TMC_LOCK_LINE, stripe * c.out_cap, c.out_cap, lane)
                 && lane == 0)
-                atomicOr(lock_block(c, wave) + 2, TMC_LOCK_OVERFLOW);
+                atomicOr(lock_block(c) + 2, TMC_LOCK_OVERFLOW);
         }
     }
     const LockArgs& c = args_here<LockArgs>();
-    unsigned long long* const block = lock_block(c, wave);
-    if constexpr (COUNTED) {
-        __syncthreads();
-        count_flush(counts, (const Images*)c.entry, c.k1, block + TMC_COHORT_COUNTERS, c.shells);
-    } else {
-        lock_flush(slot, block + TMC_COHORT_COUNTERS, c.shells, lane);
-    }
-    if (lane == 0) {
-        atomicAdd(block + 1, (unsigned long long)interactions);
-        if (truncated)
-            atomicAdd(block + 2, (unsigned long long)truncated);
-    }
+    lock_end(c, COUNTED ? nullptr : slot, totals, interactions, truncated);
+    if constexpr (COUNTED)
+        count_flush(counts, (const Images*)c.entry, c.k1, lock_block(c) + TMC_COHORT_COUNTERS, c.shells);
 }
 
 /* A level of a batch: each wave claims chunks of the queue, each a run of
@@ -546,9 +532,12 @@ __global__ void __launch_bounds__(256) walk_lock_sets(LockSetArgs a)
     extern __shared__ unsigned long long lds[];
     const uint32_t lane = __lane_id();
     const uint32_t wave = rfl32(threadIdx.x >> 6);
-    unsigned long long* const slot = lds + wave * lock_slot_words(a.shells_max);
+    unsigned long long *const totals = lds, *const slot = lds + 2u + wave * lock_slot_words(a.shells_max);
     for (uint32_t i = lane; i < lock_slot_words(a.shells_max); i += 64u)
         slot[i] = 0;
+    if (threadIdx.x < 2u)
+        totals[threadIdx.x] = 0ull;
+    __syncthreads();
     uint32_t zero = 0;
     asm volatile("" : "+v"(zero));
 
@@ -557,13 +546,14 @@ __global__ void __launch_bounds__(256) walk_lock_sets(LockSetArgs a)
     uint32_t set = ~0u, k0 = 0, k1 = 0, hi = 0;
     const char* table = nullptr;
     uint64_t interactions = 0, idle = 0;
-    uint32_t room = TMC_LOCK_FLUSH_STEPS;
+    constexpr uint32_t every = lock_flush_steps(1u);
+    uint32_t room = every;
     const uint32_t waves_per_wg = blockDim.x >> 6;
     bool begun = false;
     auto flush = [&]() {
         const LockSetArgs& c = args_here<LockSetArgs>();
         const LockSet& s = c.sets[set];
-        lock_flush(slot, c.tally + s.tally, s.shells, lane);
+        lock_flush<false>(slot, c.tally + s.tally, s.shells, lane, 64u);
     };
 
     for (;;) {
@@ -615,7 +605,7 @@ __global__ void __launch_bounds__(256) walk_lock_sets(LockSetArgs a)
                 k1 = rfl32(h.cut[c.level]);
                 hi = rfl32((uint32_t)(s.first_photon >> 32));
                 table = (const char*)c.entry + 16ull * rfl64(s.entry);
-                room = TMC_LOCK_FLUSH_STEPS;
+                room = every;
             }
         }
         for (uint32_t at = 0; at < count; at += 64u) {
@@ -632,7 +622,7 @@ __global__ void __launch_bounds__(256) walk_lock_sets(LockSetArgs a)
                 const uint64_t photon = s.first_photon + off;
                 pp = tmc_philox_photon_init((uint32_t)photon, hi, phys.key0, phys.key1);
             }
-            lock_cycle<MATH>(p, k0, k1, table, zero, hi ^ phys.key1, pp, phys, lt, room, flush);
+            lock_cycle<MATH>(p, k0, k1, table, zero, hi ^ phys.key1, pp, phys, lt, room, every, flush);
             const uint32_t n = (uint32_t)__popcll(in);
             interactions += (uint64_t)n * (k1 - k0);
             idle += (uint64_t)(64u - n) * (k1 - k0);
@@ -649,11 +639,14 @@ __global__ void __launch_bounds__(256) walk_lock_sets(LockSetArgs a)
     }
     if (set != ~0u)
         flush();
+    /* (one addition a workgroup to a word, as lock_end) */
     if (lane == 0) {
-        const LockSetArgs& c = args_here<LockSetArgs>();
-        atomicAdd(c.counters + 1, (unsigned long long)interactions);
-        atomicAdd(c.counters + 4, (unsigned long long)idle);
+        atomicAdd(totals, (unsigned long long)interactions);
+        atomicAdd(totals + 1, (unsigned long long)idle);
     }
+    __syncthreads();
+    if (threadIdx.x < 2u)
+        atomicAdd(args_here<LockSetArgs>().counters + 1u + 3u * threadIdx.x, totals[threadIdx.x]);
 }
 
 namespace {
@@ -671,25 +664,29 @@ LockKernel lock_kernel(uint32_t sampler, uint32_t math, bool counted)
 
 } // namespace
 
-hipError_t launch_lock(uint32_t sampler, uint32_t math, bool counted, const LockArgs& a, uint32_t grid, uint32_t block,
+hipError_t launch_lock(uint32_t sampler, uint32_t math, bool counted, const LockArgs& a, uint32_t grid,
                        hipStream_t stream)
 {
-    const size_t lds = counted ? lock_count_bytes(a.shells, a.k1) : lock_lds_bytes(sampler, a.shells, block);
-    hipLaunchKernelGGL(lock_kernel(sampler, math, counted), dim3(grid), dim3(block), lds, stream, a);
+    const size_t lds = counted ? lock_count_bytes(a.shells, a.k1) : lock_lds_bytes(sampler, a.shells);
+    hipLaunchKernelGGL(lock_kernel(sampler, math, counted), dim3(grid), dim3(TMC_LOCK_BLOCK), lds, stream, a);
     return hipGetLastError();
 }
 
-hipError_t lock_occupancy(uint32_t sampler, uint32_t math, uint32_t counted, uint32_t block, uint32_t shells,
-                          int* wg_per_cu)
+hipError_t lock_occupancy(uint32_t sampler, uint32_t math, uint32_t counted, uint32_t shells, int* wg_per_cu)
 {
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        wg_per_cu, lock_kernel(sampler, math, counted), (int)block,
-        counted ? lock_count_bytes(shells, counted) : lock_lds_bytes(sampler, shells, block));
+        wg_per_cu, lock_kernel(sampler, math, counted), (int)TMC_LOCK_BLOCK,
+        counted ? lock_count_bytes(shells, counted) : lock_lds_bytes(sampler, shells));
 }
 
 namespace {
 
 using LockSetsKernel = void (*)(LockSetArgs);
+
+size_t lock_sets_lds_bytes(uint32_t shells_max, uint32_t block)
+{
+    return 16u + (block / 64u) * lock_slot_words(shells_max) * 8u;
+}
 
 LockSetsKernel lock_sets_kernel(uint32_t math)
 {
@@ -700,14 +697,14 @@ LockSetsKernel lock_sets_kernel(uint32_t math)
 
 hipError_t launch_lock_sets(uint32_t math, const LockSetArgs& a, uint32_t grid, uint32_t block, hipStream_t stream)
 {
-    hipLaunchKernelGGL(lock_sets_kernel(math), dim3(grid), dim3(block), lock_lds_bytes(0u, a.shells_max, block), stream, a);
+    hipLaunchKernelGGL(lock_sets_kernel(math), dim3(grid), dim3(block), lock_sets_lds_bytes(a.shells_max, block), stream, a);
     return hipGetLastError();
 }
 
 hipError_t lock_sets_occupancy(uint32_t math, uint32_t block, uint32_t shells_max, int* wg_per_cu)
 {
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(wg_per_cu, lock_sets_kernel(math), (int)block,
-                                                        lock_lds_bytes(0u, shells_max, block));
+                                                        lock_sets_lds_bytes(shells_max, block));
 }
 
 } // namespace tmc

@@ -11,13 +11,14 @@
 
 namespace tmc {
 
-/* Copies of the overflow shell's sums in a wave's slot (16: 1% slower). */
+/* Copies of the overflow shell's sums in a slot (16: 1% slower). */
 #define TMC_LOCK_HOT 8u
 static_assert(TMC_LOCK_HOT <= TMC_CHECK_HOT, "the shell check covers every overflow copy");
 
-/* Steps between two flushes of a wave's slot: a word takes fewer than 2^20
- * deposits of at most 2^43 each, so it stays below 2^63. */
-#define TMC_LOCK_FLUSH_STEPS 16383u
+/* Steps of a wave between two flushes of its slot by it: with `waves` waves to
+ * the slot a word takes fewer than 2^20 deposits of at most 2^43 each from one
+ * flush to the next, so it stays below 2^63. */
+__host__ __device__ constexpr uint32_t lock_flush_steps(uint32_t waves) { return (1u << 14) / waves - 1u; }
 
 __host__ __device__ __forceinline__ size_t lock_slot_words(uint32_t shells)
 {
@@ -51,15 +52,24 @@ __device__ __forceinline__ tmc_u32x4 block0_uniform(uint32_t k, uint32_t c3k1, c
     return tmc_u32x4{ c0, c1, c2, c3 };
 }
 
-/* Moves a wave's slot into its block of the global sums and zeroes it. */
+/* Moves a slot into a block of the global sums and zeroes it: pairs first,
+ * first + stride, ...  SHARED: by atomic swaps, safe while other waves add. */
+template <bool SHARED>
 __device__ __forceinline__ void lock_flush(unsigned long long* slot, unsigned long long* g, uint32_t shells,
-                                           uint32_t lane)
+                                           uint32_t first, uint32_t stride)
 {
     const uint32_t last = shells - 1u;
-    for (uint32_t q = lane; q < last + TMC_LOCK_HOT; q += 64u) {
-        const unsigned long long a = slot[2u * q], b = slot[2u * q + 1u];
-        slot[2u * q] = 0;
-        slot[2u * q + 1u] = 0;
+    for (uint32_t q = first; q < last + TMC_LOCK_HOT; q += stride) {
+        unsigned long long a, b;
+        if (SHARED) {
+            a = atomicExch(slot + 2u * q, 0ull);
+            b = atomicExch(slot + 2u * q + 1u, 0ull);
+        } else {
+            a = slot[2u * q];
+            b = slot[2u * q + 1u];
+            slot[2u * q] = 0;
+            slot[2u * q + 1u] = 0;
+        }
         const uint32_t s = q < last ? q : last;
         unsigned long long oa = 0, ob = 0;
         if (a)
@@ -73,12 +83,34 @@ __device__ __forceinline__ void lock_flush(unsigned long long* slot, unsigned lo
     }
 }
 
-/* The block of global sums this wave flushes into (LockArgs, PrecArgs). */
+/* The block of global sums this workgroup flushes into (LockArgs, PrecArgs). */
 template <class Args>
-__device__ __forceinline__ unsigned long long* lock_block(const Args& a, uint32_t wave)
+__device__ __forceinline__ unsigned long long* lock_block(const Args& a)
 {
-    return a.work
-        + (size_t)((blockIdx.x * (blockDim.x >> 6) + wave) % a.copies) * (TMC_COHORT_COUNTERS + 4u * a.shells);
+    return a.work + (size_t)(blockIdx.x % a.copies) * (TMC_COHORT_COUNTERS + 4u * a.shells);
+}
+
+/* The end of a lockstep workgroup, called by all its threads: its sums and
+ * counts go to its block, by one addition to a word.  (Additions to one word
+ * take 7 to 16 ns each, whoever makes them: with a slot and counts a wave, 3e6
+ * photons at default physics took 415 us to their first roulette and 76 to the
+ * second, with one for eight waves 396 and 28.  Four waves: 2^26 photons 7.69
+ * for 7.63 ms; sixteen, whose waves wait for one another at both ends: 7.79.)  `totals`: two zeroed words of LDS. */
+template <class Args>
+__device__ __forceinline__ void lock_end(const Args& a, unsigned long long* slot, unsigned long long* totals,
+                                         uint64_t interactions, uint64_t truncated)
+{
+    if (__lane_id() == 0u) {
+        atomicAdd(totals, (unsigned long long)interactions);
+        if (truncated)
+            atomicAdd(totals + 1, (unsigned long long)truncated);
+    }
+    __syncthreads();
+    unsigned long long* const block = lock_block(a);
+    if (slot)
+        lock_flush<false>(slot, block + TMC_COHORT_COUNTERS, a.shells, threadIdx.x, blockDim.x);
+    if (threadIdx.x < 2u && totals[threadIdx.x])
+        atomicAdd(block + 1u + threadIdx.x, totals[threadIdx.x]);
 }
 
 /* The kernel's arguments where a path between two cycles uses them: read

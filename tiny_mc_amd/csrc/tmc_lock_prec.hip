@@ -22,7 +22,7 @@
 
 namespace tmc {
 
-static size_t prec_lds_bytes(uint32_t shells, uint32_t block) { return (block / 64u) * lock_slot_words(shells) * 8u; }
+static size_t prec_lds_bytes(uint32_t shells) { return (lock_slot_words(shells) + 2u) * 8u; }
 
 namespace {
 
@@ -207,9 +207,10 @@ __global__ void __launch_bounds__(256) walk_lock_prec(PrecArgs a)
     extern __shared__ unsigned long long lds[];
     const uint32_t lane = __lane_id();
     const uint32_t wave = rfl32(threadIdx.x >> 6);
-    unsigned long long* const slot = lds + wave * lock_slot_words(a.shells);
-    for (uint32_t i = lane; i < lock_slot_words(a.shells); i += 64u)
-        slot[i] = 0;
+    unsigned long long *const totals = lds, *const slot = lds + 2;
+    for (uint32_t i = threadIdx.x; i < lock_slot_words(a.shells) + 2u; i += blockDim.x)
+        lds[i] = 0;
+    __syncthreads();
 
     using PhotonT = typename Variant<PREC>::PhotonT;
     const auto phys = physics_of<PREC>(a);
@@ -234,7 +235,8 @@ __global__ void __launch_bounds__(256) walk_lock_prec(PrecArgs a)
     const uint32_t ncuts = rfl32(a.head->ncuts);
     bool failed = ncuts < a.cuts; /* (the table has room for them: never seen) */
     uint64_t interactions = 0;
-    uint32_t room = TMC_LOCK_FLUSH_STEPS;
+    const uint32_t every = lock_flush_steps(waves_per_wg);
+    uint32_t room = every;
     for (; at < photons && !failed; at += stride) {
         uint64_t in = photons - at >= 64u ? ~0ull : (1ull << (photons - at)) - 1ull;
         PhotonT p;
@@ -283,8 +285,8 @@ __global__ void __launch_bounds__(256) walk_lock_prec(PrecArgs a)
                 }
                 if (room == 0u) {
                     const PrecArgs& c = args_here<PrecArgs>();
-                    lock_flush(slot, lock_block(c, wave) + TMC_COHORT_COUNTERS, c.shells, lane);
-                    room = TMC_LOCK_FLUSH_STEPS;
+                    lock_flush<true>(slot, lock_block(c) + TMC_COHORT_COUNTERS, c.shells, lane, 64u);
+                    room = every;
                 }
             }
             in &= __ballot(x3 < TMC_ROULETTE_KILL_R);
@@ -320,23 +322,18 @@ __global__ void __launch_bounds__(256) walk_lock_prec(PrecArgs a)
                 interactions += (uint64_t)__popcll(__ballot(live));
                 if (live)
                     live = step_of<SAMPLER, PREC>(p, phys, lt);
-                if (steps % TMC_LOCK_FLUSH_STEPS == TMC_LOCK_FLUSH_STEPS - 1u) {
+                if (steps % every == every - 1u) {
                     const PrecArgs& c = args_here<PrecArgs>();
-                    lock_flush(slot, lock_block(c, wave) + TMC_COHORT_COUNTERS, c.shells, lane);
+                    lock_flush<true>(slot, lock_block(c) + TMC_COHORT_COUNTERS, c.shells, lane, 64u);
                 }
             }
             /* (the slot has taken at most two intervals' deposits, below 2^64) */
         }
     }
     const PrecArgs& c = args_here<PrecArgs>();
-    unsigned long long* const block = lock_block(c, wave);
-    lock_flush(slot, block + TMC_COHORT_COUNTERS, c.shells, lane);
-    if (lane == 0) {
-        if (interactions)
-            atomicAdd(block + 1, (unsigned long long)interactions);
-        if (failed)
-            atomicOr(block + 2, TMC_LOCK_OVERFLOW);
-    }
+    if (failed && lane == 0)
+        atomicOr(lock_block(c) + 2, TMC_LOCK_OVERFLOW);
+    lock_end(c, slot, totals, interactions, 0);
 }
 
 namespace {
@@ -358,7 +355,7 @@ PrecKernel prec_kernel(uint32_t sampler, uint32_t precision)
 hipError_t prec_occupancy(uint32_t sampler, uint32_t precision, uint32_t block, uint32_t shells, int* wg_per_cu)
 {
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(wg_per_cu, prec_kernel(sampler, precision), (int)block,
-                                                        prec_lds_bytes(shells, block));
+                                                        prec_lds_bytes(shells));
 }
 
 hipError_t launch_prec_table(uint32_t precision, const PrecArgs& a, uint32_t* counter, uint32_t counters,
@@ -375,7 +372,7 @@ hipError_t launch_prec_table(uint32_t precision, const PrecArgs& a, uint32_t* co
 hipError_t launch_prec(uint32_t sampler, uint32_t precision, const PrecArgs& a, uint32_t grid, uint32_t block,
                        hipStream_t stream)
 {
-    hipLaunchKernelGGL(prec_kernel(sampler, precision), dim3(grid), dim3(block), prec_lds_bytes(a.shells, block), stream,
+    hipLaunchKernelGGL(prec_kernel(sampler, precision), dim3(grid), dim3(block), prec_lds_bytes(a.shells), stream,
                        a);
     return hipGetLastError();
 }
