@@ -30,7 +30,7 @@ struct Physics {
     float spm; /* shells per mean free path (photon.c:9) */
     float shell_max; /* (float)(shells - 1), the overflow shell */
     uint32_t key0, key1; /* Philox key = 64-bit seed */
-    float clear_half; /* 0.5 - eps, set by set_derived */
+    float eps, clear; /* shell_index's eps and 2 eps, set by set_derived */
     tmc_philox_keys keys; /* round keys of (key0, key1), set by set_derived */
 };
 
@@ -57,9 +57,9 @@ __device__ __forceinline__ void set_derived(Physics& ph)
         }
     }
     const int e = __builtin_amdgcn_frexp_expf(ph.shell_max + 2.0f); /* shell_max + 2 < 2^e */
+    ph.eps = __builtin_ldexpf(1.0f, e - 21);
     /* wave-uniform: keep the bound in a scalar register */
-    ph.clear_half =
-        __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(0.5f - __builtin_ldexpf(1.0f, e - 21))));
+    ph.clear = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(2.0f * ph.eps)));
 }
 
 /* LDS words one lane deposits into.  Each pair of adjacent words holds a
@@ -108,15 +108,17 @@ __device__ __forceinline__ uint32_t tally_pair(const LaneTally& lt, bool inner, 
     return inner ? s : (uint32_t)lt.fmax;
 }
 
-/* The clamped short shell coordinate fc = min(RN(v_sqrt(r2) * spm), fmax)
- * and whether its floor is certainly the pair of the exact coordinate. */
+/* The clamped short shell coordinate fc = min(RN(v_sqrt(r2) * spm + eps), fmax)
+ * and whether its floor is certainly the pair of the exact coordinate (less
+ * than eps and more than zero below it: a fraction of at least 2 eps). */
 __device__ __forceinline__ float shell_coord_short(float r2, const Physics& ph, float fmax, bool* sure)
 {
     /* both operands are non-negative floats, ordered as their bit patterns:
      * one integer min, where fminf would first quiet a signalling fmax */
     const float fc = __uint_as_float(
-        __builtin_elementwise_min(__float_as_uint(__builtin_amdgcn_sqrtf(r2) * ph.spm), __float_as_uint(fmax)));
-    *sure = __builtin_fabsf(__builtin_amdgcn_fractf(fc) - 0.5f) < ph.clear_half;
+        __builtin_elementwise_min(__float_as_uint(__builtin_fmaf(__builtin_amdgcn_sqrtf(r2), ph.spm, ph.eps)),
+                                  __float_as_uint(fmax)));
+    *sure = __builtin_amdgcn_fractf(fc) >= ph.clear;
     return fc;
 }
 
@@ -124,11 +126,11 @@ __device__ __forceinline__ float shell_coord_short(float r2, const Physics& ph, 
  * f = RN(RN(sqrt(r2)) * spm), floor(f) if f < shell_max, else one of the
  * overflow shell's copies.  The hardware square root is within one ulp of
  * the correctly rounded one (the one-ulp correction of sqrt_cr_walk is exact
- * on every float), so f' = RN(v_sqrt(r2) * spm) is within 3 ulp of f.  The
- * clamped fc = min(f', fmax) has the right pair when it is clear of every
- * integer by eps: below shell_max + 1, floor(f') = floor(f) and both lie on
- * the same side of shell_max; from shell_max + 1 on (fmax included, whose
- * fraction is 1/2), f' and f are both overflows and any copy will do
+ * on every float), so f' = RN(v_sqrt(r2) * spm + eps) is within 4 ulp of
+ * f + eps, eps = 8 ulp.  The clamped fc = min(f', fmax) has the right pair when
+ * its fraction is 2 eps or more: below shell_max + 1, floor(f') = floor(f) and
+ * both lie on the same side of shell_max; from shell_max + 1 on (fmax included,
+ * whose fraction is 1/2), f' and f are both overflows and any copy will do
  * (checked on every float r2 and every copy by tiny_mc_gpu_check_shell_index).
  * Otherwise, for a lane near a shell boundary (a few per ten thousand at 101
  * shells, including radii within eps / spm of the origin), the whole wave
