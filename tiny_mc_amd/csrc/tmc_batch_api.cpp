@@ -27,8 +27,9 @@
  * walked to the second roulette the same way, and workgroups carry what is
  * left to its end as cohorts.  Measured on MI355X, walk_multi -> this:
  * 64 sets, 1.1e6 photons, planned, run and released 11.1 -> 3.1 ms; a kept
- * plan of 512 sets, 5.6e7 photons 232 -> 144 ms (its lanes idle 1% of the
- * steps, 24% before).
+ * plan of 512 sets, 5.6e7 photons 232 -> 140 ms, of 4096 sets, 4.1e9 photons
+ * 11.9 -> 9.9 s (its lanes idle 0.02% of the steps, 1.1% before; making it 16
+ * -> 141 ms).
  */
 #include <hip/hip_runtime.h>
 
@@ -281,7 +282,6 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
     std::vector<Part> parts;
     l.cycles = 0.1 * (double)p->photons >= kSecondCycle ? 2u : 1u;
     uint64_t entries = 0;
-    double steps = 0.0; /* of 64 photons, in the first cycles */
     for (uint32_t i = 0; i < nsets; ++i) {
         const uint64_t n = sets[i].params.photons;
         if (n == 0)
@@ -315,7 +315,6 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
             ls.push_back(s);
             s.cuts = 0; /* the first part builds the table */
             done += count;
-            steps += (double)cad[i].k1 * std::ceil((double)count / 64.0);
         }
     }
     if (parts.size() > 1u << 20)
@@ -331,8 +330,9 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
     l.cus = (uint32_t)c->compute_units;
     l.grid = (uint32_t)per_cu * l.cus;
 
-    /* slices, places and queues: chunks of a wave's 32nd of the work, longest first */
-    const double target = std::max(kChunkSteps, steps / ((double)l.grid * (kLockBlock / 64u)) / 32.0);
+    /* slices, places and queues: chunks of a wave's 32nd of a launch's work,
+     * longest first */
+    const double waves = (double)l.grid * (kLockBlock / 64u);
     struct Run { /* chunks of a part, of one length */
         double steps;
         uint32_t part, first, each, chunks;
@@ -351,6 +351,8 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
             if (rest)
                 runs[level].push_back({ cycle * std::ceil((double)rest / 64.0), part, (uint32_t)(n - rest), rest, 1u });
         };
+        const size_t begin = i;
+        double steps[2] = { 0.0, 0.0 }; /* of 64 photons, in the first and the second cycles */
         for (; i < parts.size(); ++i) {
             /* places for an eighth of the photons and a slack, where a tenth
              * survive, and for a 64th after the second roulette */
@@ -358,16 +360,21 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
             const uint32_t cap[2] = { (uint32_t)(n / 8u + 64u), (uint32_t)(n / 64u + 64u) };
             if (used[0] && used[0] + cap[0] > kSlicePlaces)
                 break;
-            const Cadence& k = cad[parts[i].set];
             for (uint32_t w = 0; w < 2u; ++w) {
                 ls[i].place[w] = (uint32_t)used[w];
                 ls[i].cap[w] = cap[w];
                 used[w] += cap[w];
             }
-            cut(0, (uint32_t)i, n, (double)k.k1, target);
+            const Cadence& k = cad[parts[i].set];
+            steps[0] += (double)k.k1 * std::ceil((double)n / 64.0);
+            steps[1] += (double)k.k2 * std::ceil((double)n / 640.0);
+        }
+        for (size_t j = begin; j < i; ++j) {
+            const Cadence& k = cad[parts[j].set];
+            cut(0, (uint32_t)j, parts[j].count, (double)k.k1, std::max(kChunkSteps, steps[0] / waves / 32.0));
             if (l.cycles > 1u)
-                cut(1, (uint32_t)i, cap[0], (double)k.k2, target);
-            cut(2, (uint32_t)i, cap[l.cycles - 1u], (double)k.k2, 1.0);
+                cut(1, (uint32_t)j, ls[j].cap[0], (double)k.k2, std::max(kChunkSteps, steps[1] / waves / 32.0));
+            cut(2, (uint32_t)j, ls[j].cap[l.cycles - 1u], (double)k.k2, 1.0);
         }
         for (uint32_t level = 0; level < 3u; ++level) {
             std::stable_sort(runs[level].begin(), runs[level].end(),
