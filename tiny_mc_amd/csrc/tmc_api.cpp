@@ -595,6 +595,32 @@ int run_prec(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
         return TMC_E_UNSUPPORTED;
     a.entries = (uint32_t)room;
     a.entry = c->d_table;
+    if (o->precision == TMC_PRECISION_FP64) {
+        /* the weights and cuts themselves, in the memory that holds a binary32
+         * run's weights: its products, one after the other, as the walk's */
+        constexpr size_t kHead = 32; /* of its doubles */
+        static_assert(sizeof(tmc::PrecHead) <= 8 * kHead, "head");
+        const uint32_t most = (uint32_t)(tmc::kTableEntries / 2 - kHead);
+        double* const weight = (double*)c->h_weight;
+        tmc::PrecHead* const head = (tmc::PrecHead*)(weight + most);
+        head->ncuts = head->pad = 0;
+        uint32_t k = 0;
+        double w = 1.0;
+        while (head->ncuts < a.cuts && k < most) {
+            weight[k++] = w;
+            w *= a.albedo_d;
+            if (w < (double)0.001f) {
+                w /= (double)0.1f;
+                head->cut[head->ncuts++] = k;
+            }
+        }
+        if (head->ncuts < a.cuts)
+            return TMC_E_UNSUPPORTED;
+        head->w_end = w;
+        a.entries = k;
+        a.weight = (const double*)c->d_weight;
+        a.host_head = (const tmc::PrecHead*)(a.weight + most);
+    }
 
     /* launches: through one roulette each, while the survivors fill the chip */
     uint32_t packs = 0;

@@ -206,7 +206,9 @@ struct PrecArgs {
     uint32_t photons; /* of the slice (< 2^31) */
     PrecHead* head;
     void* entry; /* pairs of images, at least one entry beyond the last cut */
-    uint32_t entries, cuts; /* room of the table, and roulettes wanted */
+    uint32_t entries, cuts; /* room of the table (binary64: its weights), and roulettes wanted */
+    const double* weight; /* binary64: host memory, the weights and the table's head */
+    const PrecHead* host_head;
     uint32_t stripes; /* of the lists, as LockArgs */
     PrecList in, out;
     const uint32_t* in_count;

@@ -846,57 +846,64 @@ __global__ void __launch_bounds__(1024) walk_cohort_sets(LockSetArgs a)
 }
 
 /* The weight table of a set: one lane walks the recurrence W[k+1] = RN(W[k] a),
- * 64 absorptions at a time, and a second wave makes images of the 64 before.
- * (The chain is a multiplication of 9 cycles an absorption, 4 ns, and the
- * hand-over through LDS; on the host it is 1.3 ns, but for one set after the
- * other.) */
-__global__ void __launch_bounds__(128) weigh_sets(const LockSet* sets, CohortHead* heads, Images* pool)
+ * 64 absorptions at a time, and four waves make images of the 256 before.
+ * (The chain is a multiplication of 9 cycles an absorption, 4 ns; handing 64 at
+ * a time over cost 6 ns an absorption more.  On the host it is 1.3 ns, but for
+ * one set after the other.) */
+#define TMC_WEIGH_BLOCK 256u
+
+__global__ void __launch_bounds__(64u + TMC_WEIGH_BLOCK) weigh_sets(const LockSet* sets, CohortHead* heads,
+                                                                    Images* pool)
 {
-    __shared__ float4 weights[2][16];
-    __shared__ uint32_t valid[2]; /* weights of the block; 0: none, and none follows */
+    __shared__ float4 weights[2][TMC_WEIGH_BLOCK / 4u];
+    __shared__ uint32_t valid[2]; /* weights of the block; fewer than it holds: none follow */
     const LockSet& s = sets[blockIdx.x];
     if (s.cuts == 0u)
         return;
     CohortHead& h = heads[s.head];
     Images* const entry = pool + s.entry;
     const float a = s.albedo;
+    const uint32_t cuts = s.cuts, entries = s.entries;
     float w = 1.0f;
     uint32_t n = 0;
-    for (uint32_t k = 0, par = 0;; k += 64u, par ^= 1u) {
+    for (uint32_t k = 0, par = 0;; k += TMC_WEIGH_BLOCK, par ^= 1u) {
         if (threadIdx.x == 0) {
-            const uint32_t room = n < s.cuts && k < s.entries ? (s.entries - k < 64u ? s.entries - k : 64u) : 0u;
-            float v = w;
+            uint32_t done = 0;
+            while (done < TMC_WEIGH_BLOCK && n < cuts && k + done < entries) {
+                const uint32_t left = entries - k - done, room = left < 64u ? left : 64u;
+                float4* const out = weights[par] + done / 4u;
+                float v = w;
 #pragma unroll
-            for (uint32_t i = 0; i < 16u; ++i) {
-                float4 q;
-                q.x = v;
-                q.y = q.x * a;
-                q.z = q.y * a;
-                q.w = q.z * a;
-                v = q.w * a;
-                weights[par][i] = q;
-            }
-            if (v < 0.001f) {
-                /* a roulette among them (the weight never grows between two) */
-                float* const out = (float*)weights[par];
-                v = w;
-                for (uint32_t i = 0; i < room && n < s.cuts; ++i) {
-                    out[i] = v;
-                    v = v * a;
-                    if (v < 0.001f) {
-                        v = v / 0.1f;
-                        h.cut[n++] = k + i + 1u;
+                for (uint32_t i = 0; i < 16u; ++i) {
+                    float4 q;
+                    q.x = v;
+                    q.y = q.x * a;
+                    q.z = q.y * a;
+                    q.w = q.z * a;
+                    v = q.w * a;
+                    out[i] = q;
+                }
+                if (v < 0.001f) {
+                    /* a roulette among them (the weight never grows between two) */
+                    v = w;
+                    for (uint32_t i = 0; i < room && n < cuts; ++i) {
+                        ((float*)out)[i] = v;
+                        v = v * a;
+                        if (v < 0.001f) {
+                            v = v / 0.1f;
+                            h.cut[n++] = k + done + i + 1u;
+                        }
                     }
                 }
-            }
-            if (room)
                 w = v;
-            valid[par] = room;
+                done += room;
+            }
+            valid[par] = done;
         }
         /* the block before, on the other side of the barrier */
-        const uint32_t lane = threadIdx.x - 64u;
-        if (k != 0u && lane < valid[par ^ 1u])
-            entry[k - 64u + lane] = images_of(((const float*)weights[par ^ 1u])[lane]);
+        const uint32_t i = threadIdx.x - 64u;
+        if (k != 0u && threadIdx.x >= 64u && i < valid[par ^ 1u])
+            entry[k - TMC_WEIGH_BLOCK + i] = images_of(((const float*)weights[par ^ 1u])[i]);
         __syncthreads();
         if (valid[par] == 0u)
             break;
@@ -955,7 +962,7 @@ hipError_t launch_cohort_sets(uint32_t math, const LockSetArgs& a, uint32_t grid
 
 hipError_t launch_weigh_sets(const LockSet* sets, uint32_t nsets, CohortHead* heads, void* entry, hipStream_t stream)
 {
-    hipLaunchKernelGGL(weigh_sets, dim3(nsets), dim3(128), 0, stream, sets, heads, (Images*)entry);
+    hipLaunchKernelGGL(weigh_sets, dim3(nsets), dim3(64u + TMC_WEIGH_BLOCK), 0, stream, sets, heads, (Images*)entry);
     return hipGetLastError();
 }
 

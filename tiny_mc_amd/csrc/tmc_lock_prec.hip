@@ -118,51 +118,37 @@ __device__ __forceinline__ bool step_of(PhotonT& p, const PhysicsT& ph, const La
 
 } // namespace
 
-/* The weight table (one workgroup), and what a run starts from. */
+/* The weight table, and what a run starts from: workgroup 0 builds the table,
+ * the others clear the counters. */
 #define TMC_PREC_BLOCK 1024u
 
 template <uint32_t PREC>
 __global__ void __launch_bounds__(TMC_PREC_BLOCK) prec_table(PrecArgs a, uint32_t* counter, uint32_t counters,
                                                              unsigned long long* start)
 {
-    __shared__ double weights[PREC == 3u ? TMC_PREC_BLOCK : 1u];
     __shared__ uint32_t first;
     const uint32_t i = threadIdx.x;
-    if (blockIdx.x != 0u) {
-        for (uint32_t j = (blockIdx.x - 1u) * TMC_PREC_BLOCK + i; j < counters; j += (gridDim.x - 1u) * TMC_PREC_BLOCK)
-            counter[j] = 0u;
-        return;
-    }
-    if (i == 0u)
-        *start = __builtin_amdgcn_s_memrealtime();
-    const auto phys = physics_of<PREC>(a);
     Images* const entry = (Images*)a.entry;
-    uint32_t n = 0; /* cuts so far */
-    double w = 1.0;
+    const uint32_t at = blockIdx.x * TMC_PREC_BLOCK + i;
+    if (at < counters)
+        counter[at] = 0u;
+    if (at == 0u)
+        *start = __builtin_amdgcn_s_memrealtime();
     if constexpr (PREC == 3u) {
-        /* one thread walks the products, the others make images of them */
-        for (uint32_t k = 0; k < a.entries; k += TMC_PREC_BLOCK) {
-            __syncthreads();
-            if (i == 0u) {
-                uint32_t j = 0;
-                for (; j < TMC_PREC_BLOCK && k + j < a.entries && n < a.cuts; ++j) {
-                    weights[j] = w;
-                    w *= phys.albedo;
-                    if (w < (double)0.001f) {
-                        a.head->cut[n++] = k + j + 1u;
-                        w /= (double)0.1f;
-                    }
-                }
-                first = j | (n == a.cuts ? 0x80000000u : 0u);
-            }
-            __syncthreads();
-            const uint32_t f = first;
-            if (i < (f & 0x7FFFFFFFu))
-                entry[k + i] = pair_of(fx_heat64(weights[i]), fx_heat2_64(weights[i]));
-            if (f >> 31)
-                break;
+        /* the host has walked the products (on the device 93 ns an absorption
+         * for a lane with its comparisons) */
+        if (at < a.entries) {
+            const double w = a.weight[at];
+            entry[at] = pair_of(fx_heat64(w), fx_heat2_64(w));
         }
+        if (at < sizeof(PrecHead) / 4u)
+            ((uint32_t*)a.head)[at] = ((const uint32_t*)a.host_head)[at];
     } else {
+        if (blockIdx.x != 0u)
+            return;
+        const auto phys = physics_of<PREC>(a);
+        uint32_t n = 0; /* cuts so far */
+        float w = 1.0f;
         /* 1024 absorptions of a cycle at a time, up to the first that ends it */
         if (i == 0u)
             entry[0] = pair_of(fx_heat(1.0f), fx_heat2(1.0f));
@@ -187,16 +173,15 @@ __global__ void __launch_bounds__(TMC_PREC_BLOCK) prec_table(PrecArgs a, uint32_
             if (i == 0u)
                 a.head->cut[n] = f;
             ++n;
-            const float next = weight_from_counts(f, n, phys);
-            w = next;
+            w = weight_from_counts(f, n, phys);
             if (i == 0u)
-                entry[f] = pair_of(fx_heat(next), fx_heat2(next));
+                entry[f] = pair_of(fx_heat(w), fx_heat2(w));
             k = f + 1u;
         }
-    }
-    if (i == 0u) {
-        a.head->ncuts = n;
-        a.head->w_end = w;
+        if (i == 0u) {
+            a.head->ncuts = n;
+            a.head->w_end = w;
+        }
     }
 }
 
@@ -361,7 +346,8 @@ hipError_t prec_occupancy(uint32_t sampler, uint32_t precision, uint32_t block, 
 hipError_t launch_prec_table(uint32_t precision, const PrecArgs& a, uint32_t* counter, uint32_t counters,
                              unsigned long long* start, hipStream_t stream)
 {
-    const uint32_t grid = 1u + (counters + TMC_PREC_BLOCK - 1u) / TMC_PREC_BLOCK;
+    const uint32_t most = precision == 3u && a.entries > counters ? a.entries : counters;
+    const uint32_t grid = 1u + most / TMC_PREC_BLOCK;
     if (precision == 3u)
         hipLaunchKernelGGL(prec_table<3u>, dim3(grid), dim3(TMC_PREC_BLOCK), 0, stream, a, counter, counters, start);
     else
