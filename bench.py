@@ -1,15 +1,16 @@
 """Benchmark of the MI355X photon-transport path (one GPU).
 
-A step is one launch of the walk over 2^30 photons at default physics
+A step is one run of the walk over 2^30 photons at default physics
 (mu_a = 2/cm, mu_s = 20/cm, 101 shells of 50 um, weight cutoff 0.001,
-roulette 0.1), through the C ABI call tiny_mc_gpu_run_ex: clear the tallies,
-run the persistent kernel, copy the 128-bit tallies back.  There is no input
+roulette 0.1), through the C ABI call tiny_mc_gpu_run_ex: build the weight
+table, walk the photons in lockstep through their roulettes, hand the 128-bit
+tallies back.  There is no input
 data: photons are generated from (seed, photon index) on the device.
 
 Prints one JSON line: whole-job photons/s, the roofline of the walk kernel
 (algorithmic FP32 FLOPs of the reference algorithm, 40.5 per absorption
-event counted from photon.c:21-48, over the kernel's average duration
-measured with HIP events on the library's stream), the same walk with the
+event counted from photon.c:21-48, over the run's average time on the
+device, from its first launch to its result), the same walk with the
 reference's own rejection sampler (photon.c:34-43), and the reference CPU
 loop timed on this machine's host cores.
 
@@ -53,7 +54,7 @@ FLOP_PER_INTERACTION = 40.5
 # 1 - mu^2 (2), sqrt (1), the angle (1), sin and cos (2), v and w (2).
 FLOP_PER_INTERACTION_ANALYTIC = 40.5 - 19.46 + 10.0
 PEAK_FP32_TFLOPS = 157.3  # MI355X published FP32 vector peak
-TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "walk_f32_default_2e30_traffic.txt")
+TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "walk_lock_default_2e30_traffic.txt")
 REF_BENCH = os.path.join(ROOT, "oracle", "_ref", "tiny_mc_bench")
 REF_SHIPPED = os.path.join(ROOT, "oracle", "_ref", "tiny_mc_shipped")
 
@@ -465,7 +466,7 @@ def main():
             "unit": "TFLOP/s",
             "frac": achieved / PEAK_FP32_TFLOPS,
             "traffic": read_traffic(),
-            "kernel": "walk_f32",
+            "kernel": "walk_lock",
             "flop_per_launch": flop_per_launch,
             "flop_per_absorption": FLOP_PER_INTERACTION,
         },

@@ -108,8 +108,8 @@ typedef struct tmc_run_stats {
     uint64_t photons; /* photons walked */
     uint64_t interactions; /* absorption events (iterations of photon.c:20) */
     uint64_t truncated; /* photons stopped by max_interactions */
-    double kernel_ms; /* walk kernel time: HIP events on the library stream, or, for small runs, the device's
-                         real-time counter */
+    double kernel_ms; /* time on the device: by its real-time counter from the first launch to the result, or (runs
+                         with a launch shape of their own and the others of the lane-per-photon walk) HIP events */
     double total_ms; /* whole call: clears, kernel, copies back */
     uint32_t grid, block, chunk; /* launch shape used */
     uint32_t sampler;
@@ -230,8 +230,11 @@ int tiny_mc_gpu_check_shell_index(const tmc_params* p, uint32_t first_bits, uint
                                   uint32_t* first_violation, uint64_t* unsure);
 
 /* ------------------------------------------------------------------------
- * Batched sweep: many parameter sets in one persistent launch (one per
- * LDS size class of the sets, up to three, back to back).
+ * Batched sweep: many parameter sets in a few launches back to back.  With
+ * the analytic sampler and every launch option automatic, waves walk 64
+ * photons of a set in lockstep and survivors of a roulette go through lists
+ * that the plan holds; otherwise one persistent launch (one per LDS size
+ * class of the sets, up to three).  Same results.
  *
  * No counterpart in the reference (it has one compile-time parameter set);
  * this is the loop of tiny_mc.c:47-49 run for many params.h configurations
@@ -272,8 +275,9 @@ typedef struct tmc_batch_stats {
     uint64_t idle_lane_steps; /* lanes without a photon while their wave stepped
                                  (drains at set switches and the end of the queue):
                                  lane utilisation = interactions / (interactions + idle) */
-    uint32_t passes; /* launches, one per LDS size class of the sets (grid, block,
-                        waves_per_simd, chunk_work above: the pass with the most work) */
+    uint32_t passes; /* persistent launches, one per LDS size class of the sets (chunks, grid, block,
+                        waves_per_simd, chunk_work above: the pass with the most work; with automatic
+                        options the shape they would have) */
     uint32_t reserved;
 } tmc_batch_stats;
 

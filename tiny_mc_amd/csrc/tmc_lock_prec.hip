@@ -11,8 +11,11 @@
  *
  * What bounds it: the binary64 logarithm, square roots, sine and cosine (200
  * binary64 instructions of an absorption's 300, 4 cycles and more each), and
- * with few photons a lane's chain through them.
- * @@
+ * with few photons a lane's chain through them.  Measured on MI355X, whole
+ * calls at default physics, lane per photon -> this walk: binary64 4096 photons
+ * 327 -> 107 us, 2^20 1176 -> 754 us, 2^22 2.85 -> 2.56 ms (1.2e11
+ * absorptions/s; the shape does not matter: 4 to 6 waves a SIMD 9.7 to 10.2 ms
+ * at 2^24); weight from counts 242 -> 93, 543 -> 368 us and 1.30 -> 1.08 ms.
  *
  * Same words, same operations and the same integer sums as step(): results
  * are bit-identical.
