@@ -401,6 +401,21 @@ std::vector<Slice> slices_of(uint64_t first, uint64_t photons, uint64_t most)
     return slices;
 }
 
+/* Threads of a lockstep launch's workgroups for `waves` waves of work: half of
+ * TMC_LOCK_BLOCK where that leaves fewer waves on the fullest compute unit, if
+ * the waves are all resident (albedo 0.99: 50,000 photons, 98 workgroups of
+ * eight waves or 196 of four, 237 and 198 us; 180,000 421 and 352 us), else
+ * TMC_LOCK_BLOCK, with half as many sums to add up (2^17 photons at default
+ * physics 58 and 61 us), which is what a cycle of fewer than 64 steps takes. */
+uint32_t lock_block_for(double waves, uint32_t steps, uint32_t grid_most, uint32_t cus)
+{
+    const auto fullest = [=](double per_wg) { return per_wg * std::ceil(std::ceil(waves / per_wg) / (double)cus); };
+    constexpr double per_wg = TMC_LOCK_BLOCK / 64u;
+    return steps >= 64u && waves <= per_wg * (double)grid_most && fullest(per_wg / 2.0) < fullest(per_wg)
+        ? TMC_LOCK_BLOCK / 2u
+        : TMC_LOCK_BLOCK;
+}
+
 /* One large binary32 run by lockstep waves, level by level, and the cohort
  * walk for the last survivors.  TMC_E_UNSUPPORTED: not one for it. */
 int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* o, uint64_t kcap, uint64_t* tally,
@@ -490,7 +505,7 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
     l.entry = c->d_table;
     l.work = c->d_work;
     l.copies = a.copies;
-    uint32_t grid0 = 0;
+    uint32_t grid0 = 0, block0 = 0;
     auto launches = [&]() {
         /* two more entries than the steps read ahead of the last cut */
         if (tmc::launch_cohort_table(a.weight, a.entries, c->d_table, counters, (uint32_t)slices.size() * per_slice,
@@ -501,7 +516,6 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
             uint32_t* const count = counters + si * per_slice; /* survivors by level */
             double n = (double)slices[si].photons;
             bool capped = false;
-            constexpr uint32_t per_wg = TMC_LOCK_BLOCK / 64u;
             const uint32_t wgs = (uint32_t)std::min<double>(grid_most, std::ceil(n / TMC_LOCK_BLOCK));
             /* at least eight workgroups a stripe, or one stripe */
             l.stripes = std::min(std::min(tmc::kStripes, cus), std::max(1u, wgs / 8u));
@@ -523,12 +537,15 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
                 l.out_cap = list_cap(lv & 1u, per);
                 const double waves = std::ceil(n / 64.0);
                 const bool by_count = counted && lv == 0;
+                const uint32_t block = by_count ? TMC_LOCK_BLOCK : lock_block_for(waves, l.k1 - l.k0, grid_most, cus);
+                const uint32_t per_wg = block / 64u;
                 const uint32_t grid = std::max(
                     l.stripes, (uint32_t)std::min<double>(by_count ? (uint32_t)counted_cu * cus : grid_most,
                                                           std::ceil(waves / (double)per_wg)));
                 l.chunk = 0;
                 if (lv == 0) {
                     grid0 = grid;
+                    block0 = block;
                     const uint64_t each = (uint64_t)waves / (per_wg * grid); /* batches a wave */
                     if (each >= 8) {
                         /* a wave's 32nd, but (short cycles) not less than 128
@@ -541,7 +558,7 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
                         l.cursor = count + levels * words;
                     }
                 }
-                if (tmc::launch_lock(o->sampler, o->math, by_count, l, grid, c->stream) != hipSuccess)
+                if (tmc::launch_lock(o->sampler, o->math, by_count, l, grid, block, c->stream) != hipSuccess)
                     return false;
             }
             a.finish = si + 1 == slices.size();
@@ -560,7 +577,7 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
         return TMC_E_UNSUPPORTED;
     if (rc == TMC_OK && st) {
         st->grid = grid0;
-        st->block = TMC_LOCK_BLOCK;
+        st->block = block0;
         st->chunk = 64;
     }
     return rc;

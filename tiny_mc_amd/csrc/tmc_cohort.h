@@ -151,15 +151,15 @@ struct LockArgs {
     unsigned long long* work; /* as CohortArgs */
 };
 
-/* Threads of walk_lock's workgroups. */
+/* Threads of walk_lock's workgroups, at most. */
 #define TMC_LOCK_BLOCK 512u
-size_t lock_lds_bytes(uint32_t sampler, uint32_t shells);
+size_t lock_lds_bytes(uint32_t sampler, uint32_t shells, uint32_t block);
 /* LDS of a workgroup that counts the photons of each shell and absorption. */
 size_t lock_count_bytes(uint32_t shells, uint32_t absorptions);
-/* Resident workgroups per CU of walk_lock (counted: the absorptions that are
+/* Resident workgroups of TMC_LOCK_BLOCK threads per CU of walk_lock (counted: the absorptions that are
  * counted by shell, 0: none). */
 hipError_t lock_occupancy(uint32_t sampler, uint32_t math, uint32_t counted, uint32_t shells, int* wg_per_cu);
-hipError_t launch_lock(uint32_t sampler, uint32_t math, bool counted, const LockArgs& a, uint32_t grid,
+hipError_t launch_lock(uint32_t sampler, uint32_t math, bool counted, const LockArgs& a, uint32_t grid, uint32_t block,
                        hipStream_t stream);
 
 /* The same for the sets of a batch: a level by lockstep waves (0 or 1), and

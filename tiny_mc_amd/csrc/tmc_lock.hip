@@ -53,9 +53,9 @@ namespace tmc {
 
 /* LDS of a workgroup: the sums, two totals, and the retries of each wave; or
  * (lock_count_bytes) the totals and the counts. */
-size_t lock_lds_bytes(uint32_t sampler, uint32_t shells)
+size_t lock_lds_bytes(uint32_t sampler, uint32_t shells, uint32_t block)
 {
-    return 8u * (lock_slot_words(shells) + 2u + (sampler ? TMC_LOCK_BLOCK / 64u * TMC_LOCK_RETRIES : 0u));
+    return 8u * (lock_slot_words(shells) + 2u + (sampler ? block / 64u * TMC_LOCK_RETRIES : 0u));
 }
 
 size_t lock_count_bytes(uint32_t shells, uint32_t absorptions)
@@ -664,11 +664,11 @@ LockKernel lock_kernel(uint32_t sampler, uint32_t math, bool counted)
 
 } // namespace
 
-hipError_t launch_lock(uint32_t sampler, uint32_t math, bool counted, const LockArgs& a, uint32_t grid,
+hipError_t launch_lock(uint32_t sampler, uint32_t math, bool counted, const LockArgs& a, uint32_t grid, uint32_t block,
                        hipStream_t stream)
 {
-    const size_t lds = counted ? lock_count_bytes(a.shells, a.k1) : lock_lds_bytes(sampler, a.shells);
-    hipLaunchKernelGGL(lock_kernel(sampler, math, counted), dim3(grid), dim3(TMC_LOCK_BLOCK), lds, stream, a);
+    const size_t lds = counted ? lock_count_bytes(a.shells, a.k1) : lock_lds_bytes(sampler, a.shells, block);
+    hipLaunchKernelGGL(lock_kernel(sampler, math, counted), dim3(grid), dim3(block), lds, stream, a);
     return hipGetLastError();
 }
 
@@ -676,7 +676,7 @@ hipError_t lock_occupancy(uint32_t sampler, uint32_t math, uint32_t counted, uin
 {
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(
         wg_per_cu, lock_kernel(sampler, math, counted), (int)TMC_LOCK_BLOCK,
-        counted ? lock_count_bytes(shells, counted) : lock_lds_bytes(sampler, shells));
+        counted ? lock_count_bytes(shells, counted) : lock_lds_bytes(sampler, shells, TMC_LOCK_BLOCK));
 }
 
 namespace {
