@@ -111,3 +111,17 @@ def test_counted_first_cycles(tmc, phys, photons, first, kmax, math):
     want, ws = tmc.run_raw(p, 31, block=256, **kw)
     np.testing.assert_array_equal(got, want)
     assert (st.interactions, st.truncated) == (ws.interactions, ws.truncated)
+
+
+@pytest.mark.parametrize("photons,first,kw", [
+    ((1 << 27) + 12345, 0, {}), ((1 << 27) + 99, (1 << 32) - (1 << 26) - 5, {}), ((1 << 27) + 1, 0, dict(sampler=1)),
+    ((1 << 27) + 77, 0, dict(precision=1))])
+def test_slices(tmc, photons, first, kw):
+    """Runs of more than one slice (2^27 photons), against the lane-per-photon
+    walk (block given); the precision variants' slices are the same."""
+    print(f"lock slices: photons={photons} first={first} {kw}", flush=True)
+    p = tmc.Params(photons=photons, **LOWALB)
+    got, st = tmc.run_raw(p, 8, first_photon=first, **kw)
+    want, ws = tmc.run_raw(p, 8, first_photon=first, block=256, **kw)
+    np.testing.assert_array_equal(got, want)
+    assert st.interactions == ws.interactions

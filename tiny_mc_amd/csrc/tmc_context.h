@@ -24,8 +24,11 @@ constexpr size_t run_work_words(uint32_t shells) { return kRunCounterWords + 4 *
 /* Entries of the cohort walk's weight table (16 bytes each). */
 constexpr size_t kTableEntries = 1u << 20;
 
-/* Photons of a slice of a large run (log2), and the counters of all its slices. */
-constexpr uint32_t kSliceLog = 26;
+/* Photons of a slice of a large run (log2), and the counters of all its slices.
+ * (A slice's last launches leave the chip idle for 70 us: 2^27 photons at
+ * albedo 0.5 in slices of 2^26 2658 us, in one of 2^27 2497; the lists of 2^27
+ * take 0.6 GB.) */
+constexpr uint32_t kSliceLog = 27;
 constexpr uint32_t kRunCounters = 1u << 21;
 constexpr uint32_t kStripes = 64; /* parts of a slice and of the survivor lists */
 

@@ -17,9 +17,9 @@
  * SIMD, the 15 three-input XORs, conversions and compares 4.1, the five
  * transcendentals 8, and the additions and multiplications of three vector
  * registers 2.2 (4 with a scalar operand).  Measured on MI355X, whole calls,
- * walk_f32 -> this walk: 2^20 photons at default physics 425 -> 236 us,
- * 3,000,017 638 -> 500 us, 2^26 8.72 -> 7.87 ms; 2^20 at albedo 0.99 2.73 ->
- * 1.38 ms; 2^17 at albedo 0.9999 117 -> 22 ms; 2^23 at albedo 0.5 951 -> 306
+ * walk_f32 -> this walk: 2^20 photons at default physics 425 -> 190 us,
+ * 3,000,017 638 -> 436 us, 2^26 8.72 -> 7.63 ms; 2^17 at albedo 0.99 1218 -> 257
+ * us, at 0.9999 117 -> 22 ms; at albedo 0.5 2^23 951 -> 260, 2^27 2842 -> 2497
  * us.
  *
  * Where a first cycle's counts fit LDS (absorptions times shells), a workgroup
