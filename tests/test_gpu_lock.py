@@ -1,5 +1,5 @@
-"""The lockstep walk of large binary32 runs (more than 49,152 photons, analytic
-sampler) against the oracle's mirror: ragged sizes on either side of its
+"""The lockstep walk of large binary32 runs (more than 32,768 photons with the
+analytic sampler, 49,152 with the other) against the oracle's mirror: ragged sizes on either side of its
 levels, photon indices across a multiple of 2^32, caps at and beside a
 roulette, several slices, and the walk of the same photons in two runs (GPU
 tests, bit-exact)."""
@@ -125,3 +125,11 @@ def test_slices(tmc, photons, first, kw):
     want, ws = tmc.run_raw(p, 8, first_photon=first, block=256, **kw)
     np.testing.assert_array_equal(got, want)
     assert st.interactions == ws.interactions
+
+
+@pytest.mark.parametrize("sampler,photons", [(0, 32768), (0, 32769), (0, 49152), (1, 49152), (1, 49153)])
+def test_line_to_the_cohort_walk(tmc, orc, hw_tables, sampler, photons):
+    tally, st = tmc.run_raw(tmc.Params(photons=photons, **DEFAULT), 3, sampler=sampler)
+    want, n = orc.mirror32(orc.params(**DEFAULT), 3, photons, sampler=sampler, tables=hw_tables)
+    assert st.interactions == n
+    np.testing.assert_array_equal(tally, want)

@@ -295,12 +295,20 @@ int finish_enqueued(Context* c, uint64_t token, uint32_t shells, uint64_t* tally
     return TMC_OK;
 }
 
+/* Photons of the largest run for the cohort walk. */
+uint64_t cohort_most(const tmc_params* p, const tmc_options* o)
+{
+    if (p->shells > TMC_LOCK_SHELLS)
+        return TMC_COHORT_PHOTONS_WIDE;
+    return o->sampler == TMC_SAMPLER_ANALYTIC ? TMC_COHORT_PHOTONS : TMC_COHORT_PHOTONS_REJECTION;
+}
+
 /* One binary32 run by the cohort walk.  TMC_E_UNSUPPORTED: not one for it. */
 int run_cohort(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* o, uint64_t kcap, uint64_t* tally,
                tmc_run_stats* st)
 {
     tmc::CohortShape shape;
-    const uint64_t most = p->shells > TMC_LOCK_SHELLS ? TMC_COHORT_PHOTONS_WIDE : TMC_COHORT_PHOTONS;
+    const uint64_t most = cohort_most(p, o);
     if (!tmc::cohort_shape(p->photons, most, first_cycle(p, kcap), p->shells, (uint32_t)c->compute_units, &shape))
         return TMC_E_UNSUPPORTED;
     tmc::CohortArgs a;
@@ -421,7 +429,7 @@ uint32_t lock_block_for(double waves, uint32_t steps, uint32_t grid_most, uint32
 int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* o, uint64_t kcap, uint64_t* tally,
              tmc_run_stats* st)
 {
-    if (p->photons <= TMC_COHORT_PHOTONS || p->photons > (1ull << 40) || p->shells > TMC_LOCK_SHELLS)
+    if (p->photons <= cohort_most(p, o) || p->photons > (1ull << 40) || p->shells > TMC_LOCK_SHELLS)
         return TMC_E_UNSUPPORTED;
     /* many photons of short walks: launching them 64 at a time and appending
      * the survivors costs what the step saves (2^27 photons, lane per photon

@@ -19,8 +19,7 @@
  * registers 2.2 (4 with a scalar operand).  Measured on MI355X, whole calls,
  * walk_f32 -> this walk: 2^20 photons at default physics 425 -> 190 us,
  * 3,000,017 638 -> 436 us, 2^26 8.72 -> 7.63 ms; 2^17 at albedo 0.99 1218 -> 257
- * us, at 0.9999 117 -> 22 ms; at albedo 0.5 2^23 951 -> 260, 2^27 2842 -> 2497
- * us.
+ * us, at 0.9999 117 -> 22 ms; 2^27 at albedo 0.5 2842 -> 2497 us.
  *
  * Where a first cycle's counts fit LDS (absorptions times shells), a workgroup
  * counts the photons of each (absorption, shell) instead of adding their images:
@@ -31,8 +30,8 @@
  *
  * With the rejection sampler a step is 133 vector instructions, a third
  * of them the second generator block of the quarter of the directions that
- * are drawn again: 2^17 photons at default physics 304 -> 110 us, 2^24 4.23 ->
- * 3.49 ms, 2^20 at albedo 0.99 5.0 -> 2.75 ms.
+ * are drawn again: 2^17 photons at default physics 304 -> 94 us, 2^24 4.24 ->
+ * 3.43 ms, 2^20 at albedo 0.99 4.97 -> 2.43 ms.
  *
  * Same words, same operations and the same integer sums as step(): results
  * are bit-identical.

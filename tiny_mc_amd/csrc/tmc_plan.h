@@ -61,19 +61,20 @@ struct CohortShape {
     uint32_t grid, copies; /* workgroups, and blocks of sums they flush into */
 };
 
-/* Largest run of the cohort walk, and where the lockstep waves' sums do not
- * fit (more than TMC_LOCK_SHELLS shells).  It walks 0.9 to 1.9e11 absorptions/s (default physics to
- * albedo 0.99), a third of a full chip's rate, which the other walks only come
- * near with several photons a lane: all take time in proportion to a photon's
- * absorptions, so the lines are numbers of photons.  Measured, cohort walk
- * against lockstep waves (walk_lock): 2^15 photons 48 / 59 us at default
- * physics, 154 / 185 us at albedo 0.99; 49,152 62 / 66 us and 227 / 203 us;
- * 2^16 71 / 71 us and 275 / 205 us; 2^17 119 / 89 us and 526 / 287 us
- * (rejection sampler: 50,000 97 / 87 and 416 / 391 us; 2^17 173 / 110 and 836 /
- * 504 us).  Against lane per photon (walk_f32): 2^17 121 / 185
- * us and 544 / 1218 us; 2^18 208 / 213 us and 1008 / 1484 us; 2^19 381 / 304 us
- * and 1963 / 1880 us. */
-#define TMC_COHORT_PHOTONS 49152ull
+/* Largest run of the cohort walk with the analytic and with the rejection
+ * sampler, and where the lockstep waves' sums do not fit (more than
+ * TMC_LOCK_SHELLS shells).  It walks 0.9 to 1.9e11 absorptions/s (default
+ * physics to albedo 0.99), a third of a full chip's rate, which the other walks
+ * only come near with several photons a lane: all take time in proportion to a
+ * photon's absorptions, so the lines are numbers of photons (256 workgroups of
+ * two cohorts of 64 photons, and of three).  Measured, cohort walk against
+ * lockstep waves (walk_lock), default physics and albedo 0.99: 32,768 photons
+ * 43 / 49 and 151 / 183 us, 40,960 54 / 51 and 210 / 188 us; rejection sampler
+ * 49,152 75 / 75 and 316 / 386 us, 2^16 100 / 76 and 442 / 402 us.  Against lane
+ * per photon (walk_f32): 2^17 121 / 185 us and 544 / 1218 us; 2^18 208 / 213 us
+ * and 1008 / 1484 us; 2^19 381 / 304 us and 1963 / 1880 us. */
+#define TMC_COHORT_PHOTONS 32768ull
+#define TMC_COHORT_PHOTONS_REJECTION 49152ull
 #define TMC_COHORT_PHOTONS_WIDE (1ull << 17)
 
 /* Shells up to which at least 5 lockstep waves' sums fit a SIMD's share of LDS. */
