@@ -383,6 +383,7 @@ bool keep_lists(Context* c, size_t bytes)
     c->d_lists = nullptr;
     if (hipMalloc(&c->d_lists, bytes) != hipSuccess) {
         c->d_lists = nullptr;
+        (void)hipGetLastError(); /* (the launches of the other walk look at it) */
         return false;
     }
     c->lists_bytes = bytes;
