@@ -590,7 +590,12 @@ int plan_create_locked(tmc::Context* c, const tmc_set* sets, uint32_t nsets, con
         a.done = p->d_done;
     }
 
-    const int lrc = plan_lock(c, sets, nsets, o, kcap, hs, cad, p);
+    int lrc = TMC_OK;
+    try {
+        lrc = plan_lock(c, sets, nsets, o, kcap, hs, cad, p);
+    } catch (const std::bad_alloc&) {
+        p->lock.on = false; /* (its queue is the largest of the host's tables) */
+    }
     if (lrc != TMC_OK) {
         plan_free(p);
         return lrc;
