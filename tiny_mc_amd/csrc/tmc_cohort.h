@@ -15,12 +15,6 @@ namespace tmc {
 #define TMC_COHORT_BUILD 512u
 /* Counter words of a block of sums, and of the result. */
 #define TMC_COHORT_COUNTERS 4u
-/* Rows of 64 items a drawing wave takes of a round, and the rows a round holds
- * at most. */
-#ifndef TMC_COHORT_WAVE_ROWS
-#define TMC_COHORT_WAVE_ROWS 2u
-#endif
-#define TMC_COHORT_ROWS (16u * TMC_COHORT_WAVE_ROWS)
 
 /* Photons between two roulettes: index in the slice, position and direction. */
 struct PhotonList {

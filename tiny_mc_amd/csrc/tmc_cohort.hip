@@ -17,8 +17,10 @@
  *   tally   (photon, k) -> shell, and the weight's images added to the LDS
  *           sums; spread over the drawing waves again.
  * The stages of three successive rounds run at once, with one barrier per
- * round.  At a roulette the survivors (a tenth) are packed into the low lanes
- * and go on as a smaller cohort, whose rows then hold several k per wave.
+ * round, and a second where the round to be drawn lays its items out otherwise
+ * than the one to be tallied, whose buffer it takes.  At a roulette the
+ * survivors (a tenth) are packed into the low lanes and go on as a smaller
+ * cohort, whose rows then hold several k per wave.
  *
  * What bounds it: the movers' chain, 23 cycles an absorption (a lane that does
  * a whole step by itself takes 740), plus 900 cycles a round to schedule it;
@@ -33,6 +35,7 @@
  * are bit-identical.
  */
 #include "tmc_cohort.h"
+#include "tmc_cohort_rows.h"
 #include "tmc_device.h"
 #include "tmc_internal.h"
 #include "tmc_math.h"
@@ -50,15 +53,6 @@ __host__ __device__ __forceinline__ size_t cohort_tally_words(uint32_t shells)
     return 2u * ((size_t)shells - 1u + TMC_COHORT_HOT);
 }
 
-/* A round's items in LDS: four arrays (step length, then direction x, y, z,
- * which the movers overwrite with the position), in each a row of absorptions
- * per photon, so that a mover reads and writes four absorptions at a time.
- * Rows are padded by four floats: 16 lanes' rows then start in 16 different
- * groups of banks. */
-#define TMC_COHORT_ARRAY (64u * (TMC_COHORT_ROWS + 4u))
-#define TMC_COHORT_ROUND (4u * TMC_COHORT_ARRAY)
-/* Floats of a photon's row in a round of 2^lg photons. */
-__device__ __forceinline__ constexpr uint32_t row_floats(uint32_t lg) { return (TMC_COHORT_ROWS << (6u - lg)) + 4u; }
 /* Floats of a hand-over of the movers' state at a roulette: position and
  * direction, three coordinates of 64 photons. */
 #define TMC_COHORT_STATE (2u * 3u * 64u)
@@ -130,13 +124,6 @@ enum : uint32_t {
 
 /* Smallest lg with 2^lg >= p (1 <= p <= 64). */
 __device__ __forceinline__ uint32_t ceil_log2(uint32_t p) { return p <= 1u ? 0u : 32u - (uint32_t)__builtin_clz(p - 1u); }
-
-/* Place of lane `lane` of row `row` in a round's arrays: absorption
- * row (64 >> lg) + (lane >> lg) of photon lane & (2^lg - 1). */
-__device__ __forceinline__ uint32_t item_of(uint32_t row, uint32_t lane, uint32_t lg)
-{
-    return (lane & ((1u << lg) - 1u)) * row_floats(lg) + (row << (6u - lg)) + (lane >> lg);
-}
 
 /* Step length and direction of one absorption from its Philox words. */
 template <uint32_t MATH>
@@ -568,6 +555,10 @@ __device__ __forceinline__ void walk_cohorts(const CohortArgs& a, const PhotonLi
         }
         if (!((next.flags | cur.flags | prev.flags) & R_VALID))
             break;
+        /* (at a roulette and where a cohort of another size starts: two rounds
+         * of a cycle) */
+        if ((prev.flags & next.flags & R_VALID) && draws_wait(prev.lg, next.lg))
+            __syncthreads();
 
         if (wave < drawing) {
             /* ---- the images of the current round's items ---- */
