@@ -210,7 +210,8 @@ __device__ __forceinline__ void store_agent(unsigned long long* p, unsigned long
  * the host's memory, its token last: the host reads the result as soon as it
  * sees the token, with no copy queued behind the kernel.  A lone workgroup
  * writes its result as it is.  `flag`: a word of LDS; `flushed`: the
- * workgroup has moved sums into the block before. */
+ * workgroup has moved sums into the block before (the same in every thread:
+ * there are barriers on either side of the branch). */
 __device__ __forceinline__ void finish_run(const CohortArgs& a, unsigned long long* lds, uint32_t* flag, bool counts,
                                            uint64_t interactions, uint64_t truncated, bool flushed)
 {
@@ -410,7 +411,7 @@ struct CohortTask {
 struct CohortCounts {
     uint64_t interactions, truncated;
     uint64_t idle; /* lanes of the rows without an absorption (batches) */
-    bool flushed; /* sums have been moved to `tally` */
+    bool flushed; /* sums have been moved to `tally` (in every wave alike) */
 };
 
 /* Walks a task's cohorts.  a.cut is in LDS (l.cuts); a.build: the weigher's
@@ -484,7 +485,7 @@ __device__ __forceinline__ void walk_cohorts(const CohortArgs& a, const PhotonLi
         /* ---- schedule the next round ---- */
         uint64_t S = 0; /* photons of cur that outlive its end */
         const uint32_t pid_cur = pid;
-        next.flags = 0;
+        next.flags = next.T = 0;
         bool changed = false;
         if (cur.flags & (R_CUT | R_CAP)) {
             const uint64_t all = cur.P == 64u ? ~0ull : (1ull << cur.P) - 1ull;
@@ -560,6 +561,15 @@ __device__ __forceinline__ void walk_cohorts(const CohortArgs& a, const PhotonLi
         if ((prev.flags & next.flags & R_VALID) && draws_wait(prev.lg, next.lg))
             __syncthreads();
 
+        /* whether the drawing waves flush the sums in this round: counted by
+         * every wave, since all of finish_run's threads go by counts.flushed */
+        since_flush = rfl32(since_flush + prev.P * prev.T);
+        const bool flush = since_flush >= TMC_COHORT_FLUSH - 64u * TMC_COHORT_ROWS;
+        if (flush) {
+            since_flush = 0;
+            counts.flushed = true;
+        }
+
         if (wave < drawing) {
             /* ---- the images of the current round's items ---- */
             if (cur.flags & R_VALID) {
@@ -584,12 +594,8 @@ __device__ __forceinline__ void walk_cohorts(const CohortArgs& a, const PhotonLi
                                          ((uint64_t)image[j].w << 32) | image[j].z);
                     }
                 }
-                since_flush = rfl32(since_flush + prev.P * prev.T);
-                if (since_flush >= TMC_COHORT_FLUSH - 64u * TMC_COHORT_ROWS) {
+                if (flush)
                     cohort_flush(lds, tally, a.shells, wave * 64u + lane, drawing * 64u);
-                    since_flush = 0;
-                    counts.flushed = true;
-                }
             }
             /* ---- draw the next round (lanes past its items draw unused ones) ---- */
             if (next.flags & R_VALID) {
