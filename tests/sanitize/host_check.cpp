@@ -1,0 +1,114 @@
+// The library's host code (tmc_api.cpp, tmc_batch_api.cpp, tmc_serve_api.cpp)
+// over the fake device, with AddressSanitizer and UndefinedBehaviorSanitizer:
+// failed allocations, calls beside servers, repeats after a full list.  The
+// argument names the check to run.  Test infrastructure; prints "<name>: ok".
+#include <chrono>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <thread>
+#include <vector>
+
+#include "../../include/tiny_mc_gpu.h"
+#include "fake_device.h"
+
+#define CHECK(c)                                                                  \
+    do {                                                                          \
+        if (!(c)) {                                                               \
+            std::fprintf(stderr, "host_check: %s:%d: %s\n", __FILE__, __LINE__, #c); \
+            std::_Exit(1);                                                        \
+        }                                                                         \
+    } while (0)
+
+namespace {
+
+tmc_params params(uint64_t photons, float mu_a = 2.0f, float mu_s = 20.0f, uint32_t shells = 101)
+{
+    tmc_params p;
+    std::memset(&p, 0, sizeof p);
+    p.mu_a = mu_a;
+    p.mu_s = mu_s;
+    p.shells = shells;
+    p.microns_per_shell = 50.0f;
+    p.photons = photons;
+    return p;
+}
+
+int run(const tmc_params& p, uint32_t precision = TMC_PRECISION_FP32, uint32_t block = 0,
+        uint64_t max_interactions = 0, tmc_run_stats* stats = nullptr)
+{
+    tmc_options o;
+    tmc_options_default(&o);
+    o.precision = precision;
+    o.block = block;
+    o.max_interactions = max_interactions;
+    std::vector<uint64_t> tally(4 * (size_t)p.shells);
+    tmc_run_stats st;
+    std::memset(&st, 0, sizeof st);
+    const int rc = tiny_mc_gpu_run_ex(&p, 1, &o, tally.data(), &st);
+    if (stats)
+        *stats = st;
+    return rc;
+}
+
+struct Form {
+    uint64_t photons;
+    uint32_t precision;
+    int fake::Launches::*kernel;
+};
+const Form kForms[] = { { 3000, TMC_PRECISION_FP32, &fake::Launches::cohort },
+                        { 300000, TMC_PRECISION_FP32, &fake::Launches::lock },
+                        { 3000, TMC_PRECISION_FP32_WEIGHT, &fake::Launches::prec },
+                        { 300000, TMC_PRECISION_FP64, &fake::Launches::prec } };
+
+// Each allocation of a first run fails in turn: that call is refused or takes
+// the lane-per-photon walk, and the next one, with the memory there, is an
+// ordinary one.
+void failed_allocations()
+{
+    for (const Form& f : kForms)
+        for (long n = 0; n < 6; ++n) {
+            fake::reset();
+            fake::fail_alloc = n;
+            const int first = run(params(f.photons), f.precision);
+            CHECK(first == TMC_OK || (first == TMC_E_NOMEM && n == 0));
+            fake::fail_alloc = -1;
+            fake::reset();
+            CHECK(run(params(f.photons), f.precision) == TMC_OK);
+            CHECK(fake::launched().*f.kernel > 0 && fake::launched().walk == 0);
+            tiny_mc_gpu_shutdown();
+            CHECK(fake::live_bytes() == 0);
+        }
+    // 256 KiB are all that the lane-per-photon walk needs
+    for (uint32_t block : { 0u, 256u }) {
+        fake::reset();
+        fake::alloc_limit = 1u << 19;
+        for (int i = 0; i < 2; ++i)
+            CHECK(run(params(3000), TMC_PRECISION_FP32, block) == TMC_OK);
+        CHECK(fake::launched().walk == 2 && fake::launched().cohort == 0);
+        fake::alloc_limit = SIZE_MAX;
+        CHECK(run(params(3000)) == TMC_OK && fake::launched().cohort == 1);
+        tiny_mc_gpu_shutdown();
+    }
+}
+
+const struct {
+    const char* name;
+    void (*check)();
+} kChecks[] = {
+    { "failed_allocations", failed_allocations },
+};
+
+} // namespace
+
+int main(int argc, char** argv)
+{
+    for (const auto& c : kChecks)
+        if (argc == 2 && !std::strcmp(argv[1], c.name)) {
+            c.check();
+            std::printf("%s: ok\n", c.name);
+            return 0;
+        }
+    std::fprintf(stderr, "host_check: no such check\n");
+    return 2;
+}

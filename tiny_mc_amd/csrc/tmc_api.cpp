@@ -111,29 +111,60 @@ int tmc::acquire_context(Context** out)
 
 namespace {
 
+/* An allocation that failed: its error must not meet the next launch, which
+ * returns the last one. */
+bool no_memory()
+{
+    (void)hipGetLastError();
+    return false;
+}
+
 /* The single-run words at the largest shell count, once per context. */
 int ensure_work(Context* c)
 {
-    if (c->d_work)
-        return TMC_OK;
-    if (hipMalloc((void**)&c->d_work, tmc::run_work_words(TMC_MAX_SHELLS) * sizeof(unsigned long long)) != hipSuccess) {
+    if (!c->d_work
+        && hipMalloc((void**)&c->d_work, tmc::run_work_words(TMC_MAX_SHELLS) * sizeof(unsigned long long))
+            != hipSuccess) {
         c->d_work = nullptr;
-        return TMC_E_NOMEM;
-    }
-    if (hipHostMalloc((void**)&c->h_out, tmc::run_work_words(TMC_MAX_SHELLS) * sizeof(unsigned long long),
-                      hipHostMallocCoherent)
-            != hipSuccess
-        || hipHostGetDevicePointer((void**)&c->d_out, c->h_out, 0) != hipSuccess
-        || hipHostMalloc((void**)&c->h_weight, tmc::kTableEntries * sizeof(float), hipHostMallocCoherent)
-            != hipSuccess
-        || hipHostGetDevicePointer((void**)&c->d_weight, c->h_weight, 0) != hipSuccess)
-        return TMC_E_NOMEM;
-    std::memset(c->h_out, 0, 8);
-    if (hipMalloc(&c->d_table, 16ull * tmc::kTableEntries) != hipSuccess) {
-        c->d_table = nullptr;
+        no_memory();
         return TMC_E_NOMEM;
     }
     return TMC_OK;
+}
+
+/* n values of host-coherent memory, the first of them zero, and their device
+ * address, once. */
+template <class T>
+bool host_values(T** host, T** device, size_t n)
+{
+    if (*host)
+        return true;
+    T *h = nullptr, *d = nullptr;
+    if (hipHostMalloc((void**)&h, n * sizeof(T), hipHostMallocCoherent) != hipSuccess)
+        return no_memory();
+    if (hipHostGetDevicePointer((void**)&d, h, 0) != hipSuccess) {
+        tmc::release_host(h);
+        return no_memory();
+    }
+    h[0] = 0;
+    *host = h;
+    *device = d;
+    return true;
+}
+
+/* What the cohort and lockstep walks need beside those words (20 MB): each
+ * piece is allocated once, and without one of them the run is lane per
+ * photon. */
+bool ensure_lockstep(Context* c)
+{
+    if (!host_values(&c->h_out, &c->d_out, tmc::run_work_words(TMC_MAX_SHELLS))
+        || !host_values(&c->h_weight, &c->d_weight, tmc::kTableEntries))
+        return false;
+    if (!c->d_table && hipMalloc(&c->d_table, 16ull * tmc::kTableEntries) != hipSuccess) {
+        c->d_table = nullptr;
+        return no_memory();
+    }
+    return true;
 }
 
 /* Releases made while a serving kernel is resident (tmc_context.h). */
@@ -383,8 +414,7 @@ bool keep_lists(Context* c, size_t bytes)
     c->d_lists = nullptr;
     if (hipMalloc(&c->d_lists, bytes) != hipSuccess) {
         c->d_lists = nullptr;
-        (void)hipGetLastError(); /* (the launches of the other walk look at it) */
-        return false;
+        return no_memory();
     }
     c->lists_bytes = bytes;
     return true;
@@ -756,7 +786,8 @@ int tmc::run_walk(Context* c, const tmc_params* p, uint64_t seed, const tmc_opti
     const uint32_t table_k = tmc::weight_table_entries(p, o->precision, p->photons, o->weight_table);
     /* the cohort and lockstep walks: runs of the allocating entry point with no
      * launch shape or table asked for (cohort_shape has the sizes) */
-    if (work == c->d_work && !o->block && !o->grid && !o->chunk && !o->weight_table) {
+    if (work == c->d_work && !o->block && !o->grid && !o->chunk && !o->weight_table && p->photons
+        && ensure_lockstep(c)) {
         int rc;
         if (o->precision == TMC_PRECISION_FP32) {
             rc = run_cohort(c, p, seed, o, kcap, tally, st);
