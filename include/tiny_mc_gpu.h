@@ -334,7 +334,9 @@ int tmc_batch_autotune(const tmc_set* sets, uint32_t nsets, const tmc_batch_opti
  * device (single runs, batches, another server's) get the workgroups of
  * their launch spread over every compute unit, so with the default of none
  * reserved they wait until the server has been idle for idle_ms and its
- * kernel has left; with 2 per compute unit they run beside it.
+ * kernel has left; with 2 per compute unit they run beside it.  A single run
+ * or a batch of this library that is on the device when an idle server's next
+ * request arrives is finished before the server's kernel is launched.
  * ------------------------------------------------------------------------ */
 
 #define TMC_PENDING 1 /* positive status: the request has not finished */

@@ -92,11 +92,89 @@ void failed_allocations()
     }
 }
 
+tmc_server* open_server()
+{
+    tmc_serve_options o;
+    tmc_serve_options_default(&o);
+    o.max_requests = 8;
+    o.ring_chunks = 1u << 12;
+    o.idle_ms = 60000; // the kernel stays
+    tmc_server* s = nullptr;
+    CHECK(tmc_serve_open(&o, &s) == TMC_OK);
+    return s;
+}
+
+uint64_t submit(tmc_server* s, uint64_t photons)
+{
+    tmc_set q;
+    std::memset(&q, 0, sizeof q);
+    q.params = params(photons);
+    uint64_t id = 0;
+    CHECK(tmc_serve_submit(s, &q, &id) == TMC_OK);
+    return id;
+}
+
+int batch(uint64_t photons, tmc_batch_stats* stats = nullptr)
+{
+    std::vector<tmc_set> sets(3);
+    for (tmc_set& q : sets) {
+        std::memset(&q, 0, sizeof q);
+        q.params = params(photons);
+    }
+    std::vector<uint64_t> tally(tmc_batch_tally_words(sets.data(), 3));
+    tmc_batch_stats st;
+    return tmc_batch_run(sets.data(), 3, nullptr, tally.data(), stats ? stats : &st);
+}
+
+// A request that arrives while a run's launches are queued: the serving kernel
+// is not launched before the last of them has ended, the server's callers do
+// not wait for it, and the next run does not take the device again.
+void server_during_run()
+{
+    constexpr size_t forms = sizeof kForms / sizeof kForms[0];
+    for (size_t i = 0; i <= forms; ++i) {
+        const bool sets = i == forms;
+        int fake::Launches::*const kernel = sets ? &fake::Launches::cohort_sets
+            : kForms[i].precision               ? &fake::Launches::prec
+                                                : &fake::Launches::cohort;
+        auto once = [&]() { return sets ? batch(50000) : run(params(kForms[i].photons), kForms[i].precision); };
+        fake::reset();
+        tmc_server* s = open_server();
+        fake::hold(true);
+        int first = 1, second = 1;
+        std::thread caller([&]() {
+            first = once();
+            second = once();
+        });
+        while (!(fake::launched().*kernel))
+            std::this_thread::sleep_for(std::chrono::milliseconds(1));
+        const uint64_t id = submit(s, 1000);
+        std::this_thread::sleep_for(std::chrono::milliseconds(50));
+        const int launched = fake::launched().*kernel;
+        CHECK(fake::launched().serve == 0);
+        CHECK(tmc_serve_poll(s, id, nullptr, nullptr) == TMC_PENDING);
+        fake::hold(false);
+        caller.join();
+        CHECK(first == TMC_OK && second == TMC_OK);
+        CHECK(fake::launched().*kernel == launched);
+        CHECK((sets ? fake::launched().batch : fake::launched().walk) > 0);
+        std::vector<uint64_t> tally(4 * 101);
+        CHECK(tmc_serve_wait(s, id, 60.0, tally.data(), nullptr) == TMC_OK);
+        CHECK(fake::launched().serve == 1);
+        tmc_serve_close(s);
+        // without the server the runs are in lockstep again
+        CHECK(once() == TMC_OK && fake::launched().*kernel > launched);
+        tiny_mc_gpu_shutdown();
+        CHECK(fake::live_bytes() == 0);
+    }
+}
+
 const struct {
     const char* name;
     void (*check)();
 } kChecks[] = {
     { "failed_allocations", failed_allocations },
+    { "server_during_run", server_during_run },
 };
 
 } // namespace

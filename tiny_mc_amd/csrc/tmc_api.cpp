@@ -169,7 +169,7 @@ bool ensure_lockstep(Context* c)
 
 /* Releases made while a serving kernel is resident (tmc_context.h). */
 std::mutex g_release_mutex;
-int g_serving_kernels = 0;
+int g_serving_kernels = 0, g_serving_waiting = 0, g_lockstep_runs = 0;
 std::vector<std::function<void()>> g_deferred;
 
 } // namespace
@@ -195,19 +195,34 @@ void tmc::release_host(void* p)
         release([p]() { (void)hipHostFree(p); });
 }
 
-bool tmc::unless_serving(const std::function<void()>& fn)
+tmc::LockstepRun::LockstepRun()
 {
     std::lock_guard<std::mutex> lock(g_release_mutex);
-    if (g_serving_kernels > 0)
-        return false;
-    fn();
-    return true;
+    on_ = g_serving_kernels == 0 && g_serving_waiting == 0;
+    g_lockstep_runs += on_;
 }
 
-void tmc::serving_kernel_started()
+tmc::LockstepRun::~LockstepRun()
 {
     std::lock_guard<std::mutex> lock(g_release_mutex);
-    ++g_serving_kernels;
+    g_lockstep_runs -= on_;
+}
+
+bool tmc::serving_kernel_started(bool* waiting)
+{
+    std::lock_guard<std::mutex> lock(g_release_mutex);
+    const bool wait = g_lockstep_runs > 0;
+    g_serving_waiting += (int)wait - (int)*waiting;
+    *waiting = wait;
+    g_serving_kernels += !wait;
+    return !wait;
+}
+
+void tmc::serving_kernel_waived(bool* waiting)
+{
+    std::lock_guard<std::mutex> lock(g_release_mutex);
+    g_serving_waiting -= *waiting;
+    *waiting = false;
 }
 
 void tmc::serving_kernel_left()
@@ -290,23 +305,19 @@ void use_shape(const tmc::CohortShape& s, tmc::CohortArgs* a)
 }
 
 /* Enqueues a run by `launches` behind what clears the device words, unless a
- * serving kernel is resident (TMC_E_UNSUPPORTED), and waits for its result. */
+ * server has the device (TMC_E_UNSUPPORTED), and waits for its result. */
 int finish_enqueued(Context* c, uint64_t token, uint32_t shells, uint64_t* tally, tmc_run_stats* st,
                     const std::function<bool()>& launches)
 {
-    int rc = TMC_OK;
-    const bool launched = tmc::unless_serving([&]() {
-        const bool zero = c->work_zero;
-        c->work_zero = false;
-        if ((!zero && tmc::launch_clear(c->d_work, tmc::run_work_words(TMC_MAX_SHELLS), c->stream) != hipSuccess)
-            || !launches())
-            rc = TMC_E_HIP;
-    });
-    if (!launched)
+    const tmc::LockstepRun run;
+    if (!run)
         return TMC_E_UNSUPPORTED;
-    if (rc != TMC_OK) {
+    const bool zero = c->work_zero;
+    c->work_zero = false;
+    if ((!zero && tmc::launch_clear(c->d_work, tmc::run_work_words(TMC_MAX_SHELLS), c->stream) != hipSuccess)
+        || !launches()) {
         (void)hipStreamSynchronize(c->stream); /* h_weight may still be read */
-        return rc;
+        return TMC_E_HIP;
     }
     const auto t0 = std::chrono::steady_clock::now();
     while (__atomic_load_n(&c->h_out[0], __ATOMIC_ACQUIRE) != token) {

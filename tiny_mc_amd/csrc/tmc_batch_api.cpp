@@ -442,10 +442,10 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
     hipError_t e = hipMemcpyAsync(d, stage.data(), written, hipMemcpyHostToDevice, c->stream);
     /* (beside a resident serving kernel a plan is made without waiting for it,
      * and keeps to walk_multi) */
-    if (e == hipSuccess)
-        l.on = tmc::unless_serving([&]() {
-            e = tmc::launch_weigh_sets(a.sets, l.parts, (tmc::CohortHead*)(d + at_heads), d + at_entries, c->stream);
-        });
+    const tmc::LockstepRun run;
+    l.on = (bool)run;
+    if (e == hipSuccess && l.on)
+        e = tmc::launch_weigh_sets(a.sets, l.parts, (tmc::CohortHead*)(d + at_heads), d + at_entries, c->stream);
     if (e != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess)
         return TMC_E_HIP;
     return TMC_OK;
@@ -638,20 +638,23 @@ int plan_launch(tmc::Context* c, tmc_batch_plan* p, bool lock)
 int plan_run_locked(tmc::Context* c, tmc_batch_plan* p, uint64_t* tallies, tmc_batch_stats* st)
 {
     const auto t0 = std::chrono::steady_clock::now();
-    int rc = TMC_OK;
-    /* (the cohorts' workgroups need whole compute units, and would wait for a
-     * resident serving kernel) */
-    bool lock = p->lock.on && tmc::unless_serving([&]() { rc = plan_launch(c, p, true); });
-    for (;;) {
-        if (!lock)
-            rc = plan_launch(c, p, false);
+    bool walked = false;
+    if (p->lock.on) {
+        /* (the cohorts' workgroups need whole compute units) */
+        const tmc::LockstepRun run;
+        if (run) {
+            const int rc = plan_launch(c, p, true);
+            if (hipStreamSynchronize(c->stream) != hipSuccess || rc != TMC_OK)
+                return TMC_E_HIP;
+            walked = p->h_counters[2] < TMC_LOCK_OVERFLOW; /* else a list had no room for a survivor */
+        }
+    }
+    if (!walked) {
+        const int rc = plan_launch(c, p, false);
         if (rc != TMC_OK)
             return rc;
         if (hipStreamSynchronize(c->stream) != hipSuccess)
             return TMC_E_HIP;
-        if (!lock || p->h_counters[2] < TMC_LOCK_OVERFLOW)
-            break;
-        lock = false; /* a list had no room for a survivor */
     }
     float ms = 0.0f;
     if (hipEventElapsedTime(&ms, c->ev_start, c->ev_stop) != hipSuccess)

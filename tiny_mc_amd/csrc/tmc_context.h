@@ -80,12 +80,29 @@ int scratch_setup(int device);
 void release(std::function<void()> fn);
 void release_device(void* p); /* hipFree */
 void release_host(void* p); /* hipHostFree */
-/* Runs fn, which enqueues a kernel that needs whole compute units, unless a
- * serving kernel is resident (false): the kernel would wait for it, where one
- * of small workgroups finds room beside a server that reserves some. */
-bool unless_serving(const std::function<void()>& fn);
-void serving_kernel_started();
+/* Launches that need whole compute units, from before the first of them is
+ * enqueued until the last has ended.  Beside a resident serving kernel they
+ * would wait for it, where a kernel of small workgroups finds room beside a
+ * server that reserves some: false, for the whole life of the object, if one is
+ * resident or waits to be launched.  While one of these objects is true, no
+ * serving kernel is launched. */
+class LockstepRun {
+public:
+    LockstepRun();
+    ~LockstepRun();
+    LockstepRun(const LockstepRun&) = delete;
+    LockstepRun& operator=(const LockstepRun&) = delete;
+    explicit operator bool() const { return on_; }
+
+private:
+    bool on_;
+};
+/* False while a LockstepRun is on: the caller asks again later, *waiting (false
+ * at first) is set, and from then on every new LockstepRun is off. */
+bool serving_kernel_started(bool* waiting);
 void serving_kernel_left();
+/* A server that ends without its kernel. */
+void serving_kernel_waived(bool* waiting);
 
 } // namespace tmc
 

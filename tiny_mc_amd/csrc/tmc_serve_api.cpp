@@ -164,6 +164,7 @@ struct tmc_server {
     uint64_t launch_id = 0;
     bool kernel_running = false;
     bool stopping = false; /* the running kernel was asked to stop */
+    bool waiting = false; /* a kernel is to be launched, and a lockstep run has the device */
     double last_busy = 0; /* last time the server held a request */
     tmc_serve_stats st;
 
@@ -409,11 +410,12 @@ void serve_step(tmc_server* s)
         s->st.chunks_published = s->published;
     }
 
-    /* keep a kernel running while published work waits */
-    if (!s->kernel_running && s->published > s->base) {
+    /* keep a kernel running while published work waits (not ahead of what is
+     * still queued of a run whose workgroups need whole compute units: those
+     * would wait until the server is idle, and so would the run's caller) */
+    if (!s->kernel_running && s->published > s->base && tmc::serving_kernel_started(&s->waiting)) {
         s->args.ticket_base = s->base;
         s->args.launch_id = ++s->launch_id;
-        tmc::serving_kernel_started();
         if (tmc::launch_serve(s->opt.sampler, s->opt.math, s->args, s->grid, s->block, s->kstream) != hipSuccess) {
             tmc::serving_kernel_left();
             s->error = TMC_E_HIP;
@@ -499,6 +501,7 @@ void serve_loop(tmc_server* s)
         }
         kernel_left(s, q);
     }
+    tmc::serving_kernel_waived(&s->waiting);
     s->worker_done = true;
     s->cv_done.notify_all();
 }
