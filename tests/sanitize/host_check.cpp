@@ -169,12 +169,40 @@ void server_during_run()
     }
 }
 
+// Runs and plans beside a resident serving kernel take no memory for the walks
+// that they cannot use there.
+void memory_beside_server()
+{
+    fake::reset();
+    tmc_server* s = open_server();
+    const uint64_t id = submit(s, 1000);
+    std::vector<uint64_t> tally(4 * 101);
+    CHECK(tmc_serve_wait(s, id, 60.0, tally.data(), nullptr) == TMC_OK && fake::launched().serve == 1);
+    const size_t before = fake::live_bytes();
+    for (const Form& f : kForms)
+        CHECK(run(params(f.photons), f.precision) == TMC_OK);
+    CHECK(fake::launched().walk == 4 && fake::live_bytes() - before < 1u << 20);
+    tmc_set q;
+    std::memset(&q, 0, sizeof q);
+    q.params = params(1u << 24);
+    tmc_batch_plan* plan = nullptr;
+    CHECK(tmc_batch_plan_create(&q, 1, nullptr, &plan) == TMC_OK);
+    CHECK(fake::live_bytes() - before < 2u << 20);
+    CHECK(tmc_batch_plan_run(plan, tally.data(), nullptr) == TMC_OK && fake::launched().batch == 1);
+    tmc_batch_plan_destroy(plan);
+    tmc_serve_close(s);
+    CHECK(fake::launched().lock + fake::launched().lock_sets + fake::launched().cohort + fake::launched().prec == 0);
+    tiny_mc_gpu_shutdown();
+    CHECK(fake::live_bytes() == 0);
+}
+
 const struct {
     const char* name;
     void (*check)();
 } kChecks[] = {
     { "failed_allocations", failed_allocations },
     { "server_during_run", server_during_run },
+    { "memory_beside_server", memory_beside_server },
 };
 
 } // namespace

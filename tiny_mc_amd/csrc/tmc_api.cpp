@@ -208,6 +208,12 @@ tmc::LockstepRun::~LockstepRun()
     g_lockstep_runs -= on_;
 }
 
+bool tmc::serving()
+{
+    std::lock_guard<std::mutex> lock(g_release_mutex);
+    return g_serving_kernels > 0 || g_serving_waiting > 0;
+}
+
 bool tmc::serving_kernel_started(bool* waiting)
 {
     std::lock_guard<std::mutex> lock(g_release_mutex);
@@ -796,8 +802,9 @@ int tmc::run_walk(Context* c, const tmc_params* p, uint64_t seed, const tmc_opti
         return TMC_E_INVALID;
     const uint32_t table_k = tmc::weight_table_entries(p, o->precision, p->photons, o->weight_table);
     /* the cohort and lockstep walks: runs of the allocating entry point with no
-     * launch shape or table asked for (cohort_shape has the sizes) */
-    if (work == c->d_work && !o->block && !o->grid && !o->chunk && !o->weight_table && p->photons
+     * launch shape or table asked for (cohort_shape has the sizes), unless a
+     * server has the device */
+    if (work == c->d_work && !o->block && !o->grid && !o->chunk && !o->weight_table && p->photons && !tmc::serving()
         && ensure_lockstep(c)) {
         int rc;
         if (o->precision == TMC_PRECISION_FP32) {

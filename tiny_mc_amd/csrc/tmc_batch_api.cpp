@@ -263,14 +263,14 @@ uint32_t cuts_for(double n)
 
 /* Plans the lockstep launches of a batch; leaves p->lock off where they don't
  * apply: with the rejection sampler, with a cap on the absorptions, where the
- * caller chose a launch shape, with more than TMC_LOCK_SHELLS shells, and where the weight tables or a first
- * cycle are longer than is worth laying out.  TMC_OK, or TMC_E_HIP. */
+ * caller chose a launch shape, with more than TMC_LOCK_SHELLS shells, where the weight tables or a first
+ * cycle are longer than is worth laying out, and beside a server that has the device.  TMC_OK, or TMC_E_HIP. */
 int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_batch_options* o, uint64_t kcap,
               const std::vector<tmc::BatchSet>& hs, const std::vector<Cadence>& cad, tmc_batch_plan* p)
 {
     LockPlan& l = p->lock;
     if (o->sampler != TMC_SAMPLER_ANALYTIC || o->block || o->waves_per_simd || o->copies || o->chunk_work
-        || kcap != 0xFFFFFFFFull || p->shells_max > TMC_LOCK_SHELLS || p->photons == 0)
+        || kcap != 0xFFFFFFFFull || p->shells_max > TMC_LOCK_SHELLS || p->photons == 0 || tmc::serving())
         return TMC_OK;
 
     /* the sets' cadences and tables, and their parts */
@@ -440,8 +440,8 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
     a.tally = p->d_tally;
     a.counters = p->d_counters;
     hipError_t e = hipMemcpyAsync(d, stage.data(), written, hipMemcpyHostToDevice, c->stream);
-    /* (beside a resident serving kernel a plan is made without waiting for it,
-     * and keeps to walk_multi) */
+    /* (a server may have taken the device since: the plan is made without
+     * waiting for it, and keeps to walk_multi) */
     const tmc::LockstepRun run;
     l.on = (bool)run;
     if (e == hipSuccess && l.on)
@@ -595,6 +595,10 @@ int plan_create_locked(tmc::Context* c, const tmc_set* sets, uint32_t nsets, con
         lrc = plan_lock(c, sets, nsets, o, kcap, hs, cad, p);
     } catch (const std::bad_alloc&) {
         p->lock.on = false; /* (its queue is the largest of the host's tables) */
+    }
+    if (!p->lock.on) {
+        tmc::release_device(p->lock.d);
+        p->lock = LockPlan();
     }
     if (lrc != TMC_OK) {
         plan_free(p);

@@ -97,6 +97,8 @@ public:
 private:
     bool on_;
 };
+/* Whether a LockstepRun would be off: nothing need be prepared for it. */
+bool serving();
 /* False while a LockstepRun is on: the caller asks again later, *waiting (false
  * at first) is set, and from then on every new LockstepRun is off. */
 bool serving_kernel_started(bool* waiting);
