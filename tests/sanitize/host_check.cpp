@@ -6,6 +6,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -19,6 +20,20 @@
             std::_Exit(1);                                                        \
         }                                                                         \
     } while (0)
+
+static size_t g_largest = 0; // of the host's allocations
+
+void* operator new(size_t n)
+{
+    if (n > g_largest)
+        g_largest = n;
+    if (void* p = std::malloc(n ? n : 1))
+        return p;
+    throw std::bad_alloc();
+}
+void* operator new(size_t n, const std::nothrow_t&) noexcept { return std::malloc(n ? n : 1); }
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 namespace {
 
@@ -196,6 +211,23 @@ void memory_beside_server()
     CHECK(fake::live_bytes() == 0);
 }
 
+// A set with more photons than a plan's lockstep launches are laid out for: it
+// is planned, and what the host lays out before it leaves them is bounded.
+void enormous_set()
+{
+    fake::reset();
+    tmc_set q;
+    std::memset(&q, 0, sizeof q);
+    q.params = params(1ull << 48);
+    tmc_batch_plan* plan = nullptr;
+    g_largest = 0;
+    CHECK(tmc_batch_plan_create(&q, 1, nullptr, &plan) == TMC_OK);
+    tmc_batch_plan_destroy(plan);
+    CHECK(g_largest <= 100u << 20);
+    tiny_mc_gpu_shutdown();
+    CHECK(fake::live_bytes() == 0);
+}
+
 const struct {
     const char* name;
     void (*check)();
@@ -203,6 +235,7 @@ const struct {
     { "failed_allocations", failed_allocations },
     { "server_during_run", server_during_run },
     { "memory_beside_server", memory_beside_server },
+    { "enormous_set", enormous_set },
 };
 
 } // namespace

@@ -82,6 +82,8 @@ struct LockPlan {
 
 /* Photons of a part (its survivors' places fit a slice). */
 constexpr uint64_t kPart = 1ull << 26;
+/* Parts of a batch: 100 MB in the host's memory (a set may have 2^63 photons). */
+constexpr size_t kParts = 1u << 20;
 /* Places of a slice's first list: 0.9 GB. */
 constexpr uint64_t kSlicePlaces = 1ull << 25;
 /* Entries of the weight tables of a batch: 1 GB. */
@@ -311,14 +313,14 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
             s.first_photon = hs[i].first_photon + done;
             const uint64_t count =
                 std::min<uint64_t>(std::min<uint64_t>(kPart, n - done), (1ull << 32) - (s.first_photon & 0xFFFFFFFFull));
+            if (parts.size() == kParts)
+                return TMC_OK;
             parts.push_back({ i, done, count });
             ls.push_back(s);
             s.cuts = 0; /* the first part builds the table */
             done += count;
         }
     }
-    if (parts.size() > 1u << 20)
-        return TMC_OK;
     l.parts = (uint32_t)parts.size();
 
     /* launch shape */
