@@ -228,6 +228,21 @@ void enormous_set()
     CHECK(fake::live_bytes() == 0);
 }
 
+// A run stopped after a few absorptions takes no longer weight table than that,
+// whatever the albedo, and a table of its own for one that would not fit.
+void capped_runs()
+{
+    for (const float mu_a : { 2.0f, 2e-3f, 2e-5f })
+        for (const uint64_t cap : { 1ull, 7ull, 1000ull, 50000ull })
+            for (const Form& f : { kForms[0], kForms[1] }) {
+                fake::reset();
+                CHECK(run(params(f.photons, mu_a), f.precision, 0, cap) == TMC_OK);
+                CHECK(fake::launched().*f.kernel > 0 && fake::launched().walk == 0);
+                CHECK(fake::table_entries <= cap);
+            }
+    tiny_mc_gpu_shutdown();
+}
+
 const struct {
     const char* name;
     void (*check)();
@@ -236,6 +251,7 @@ const struct {
     { "server_during_run", server_during_run },
     { "memory_beside_server", memory_beside_server },
     { "enormous_set", enormous_set },
+    { "capped_runs", capped_runs },
 };
 
 } // namespace

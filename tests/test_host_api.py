@@ -8,7 +8,8 @@ import pytest
 from test_sanitize import BUILD, SAN_ENV, built  # noqa: F401  (built: the fixture)
 
 
-@pytest.mark.parametrize("name", ["failed_allocations", "server_during_run", "memory_beside_server", "enormous_set"])
+@pytest.mark.parametrize("name", ["failed_allocations", "server_during_run", "memory_beside_server", "enormous_set",
+                                  "capped_runs"])
 def test_host(built, name):  # noqa: F811
     r = subprocess.run([os.path.join(BUILD, "host_check"), name], capture_output=True, text=True, timeout=120,
                        env=SAN_ENV)

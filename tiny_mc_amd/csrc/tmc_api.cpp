@@ -261,14 +261,20 @@ namespace {
 constexpr std::chrono::microseconds kSpin(500);
 
 /* The weight table of a run and the arguments its launches share.  `cuts`:
- * roulettes the table is to span.  False if it does not fit. */
+ * roulettes the table is to span.  False if it does not fit.  A capped run's
+ * table ends with the cap, and its roulettes with ones that are never reached
+ * (100 photons stopped after 100 absorptions, the whole table and this: albedo
+ * 0.9999 161 and 25 us; 1 - 1e-6, which does not fit, 1376 and 22 us). */
 bool weigh(Context* c, const tmc_params* p, uint64_t seed, uint64_t kcap, uint32_t cuts, tmc::CohortArgs* a)
 {
     std::memset(a, 0, sizeof *a);
-    a->ncuts = tmc::weight_sequence(p, (uint32_t)tmc::kTableEntries - 2u, cuts, c->h_weight, a->cut, &a->w_end);
-    if (a->ncuts < cuts)
+    constexpr uint32_t room = (uint32_t)tmc::kTableEntries - 2u;
+    a->ncuts = tmc::weight_sequence(p, (uint32_t)std::min<uint64_t>(room, kcap), cuts, c->h_weight, a->cut, &a->w_end);
+    if (a->ncuts < cuts && kcap > room)
         return false;
-    a->entries = a->cut[a->ncuts - 1];
+    a->entries = a->ncuts < cuts ? (uint32_t)kcap : a->cut[a->ncuts - 1];
+    while (a->ncuts < cuts)
+        a->cut[a->ncuts++] = ~0u;
     a->weight = c->d_weight;
     a->entry = c->d_table;
     a->seed = seed;

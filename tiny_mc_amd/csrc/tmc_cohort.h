@@ -85,7 +85,8 @@ struct CohortArgs {
     uint32_t entries; /* weights of the table */
     const float* weight; /* host memory: the weight deposited at absorption k < entries */
     const void* entry; /* device memory: the same as pairs of images, where build is 0 */
-    uint32_t ncuts; /* roulettes the table spans: the i-th follows absorption cut[i] - 1, and cut[ncuts - 1] = entries */
+    uint32_t ncuts; /* roulettes the table spans: the i-th follows absorption cut[i] - 1, and cut[ncuts - 1] = entries
+                       (past the cap: ~0u, and entries = kcap) */
     uint32_t cut[TMC_COHORT_CUTS];
     float w_end; /* the weight with which a survivor of the last one goes on */
     uint32_t copies; /* copies of the sums the workgroups flush into */
