@@ -2,6 +2,7 @@
 // over the fake device, with AddressSanitizer and UndefinedBehaviorSanitizer:
 // failed allocations, calls beside servers, repeats after a full list.  The
 // argument names the check to run.  Test infrastructure; prints "<name>: ok".
+#include <algorithm>
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
@@ -50,20 +51,17 @@ tmc_params params(uint64_t photons, float mu_a = 2.0f, float mu_s = 20.0f, uint3
 }
 
 int run(const tmc_params& p, uint32_t precision = TMC_PRECISION_FP32, uint32_t block = 0,
-        uint64_t max_interactions = 0, tmc_run_stats* stats = nullptr)
+        uint64_t max_interactions = 0, uint32_t sampler = TMC_SAMPLER_ANALYTIC)
 {
     tmc_options o;
     tmc_options_default(&o);
     o.precision = precision;
     o.block = block;
     o.max_interactions = max_interactions;
+    o.sampler = sampler;
     std::vector<uint64_t> tally(4 * (size_t)p.shells);
     tmc_run_stats st;
-    std::memset(&st, 0, sizeof st);
-    const int rc = tiny_mc_gpu_run_ex(&p, 1, &o, tally.data(), &st);
-    if (stats)
-        *stats = st;
-    return rc;
+    return tiny_mc_gpu_run_ex(&p, 1, &o, tally.data(), &st);
 }
 
 struct Form {
@@ -243,6 +241,20 @@ void capped_runs()
     tiny_mc_gpu_shutdown();
 }
 
+// Lockstep waves of the rejection sampler in long cycles: where they fit the
+// chip, in workgroups of either size, every one of them is launched.
+void all_waves_at_once()
+{
+    for (uint64_t n = 50000; n <= 400000; n += 9973) { // one level
+        fake::reset();
+        CHECK(run(params(n, 0.5f, 50.0f), TMC_PRECISION_FP32, 0, 0, TMC_SAMPLER_REJECTION) == TMC_OK);
+        CHECK(fake::launched().lock == 1);
+        const uint64_t waves = (n + 63) / 64; // fake: four workgroups of eight a CU
+        CHECK((uint64_t)fake::lock_grid * fake::lock_block / 64 >= std::min<uint64_t>(waves, 8192));
+    }
+    tiny_mc_gpu_shutdown();
+}
+
 const struct {
     const char* name;
     void (*check)();
@@ -252,6 +264,7 @@ const struct {
     { "memory_beside_server", memory_beside_server },
     { "enormous_set", enormous_set },
     { "capped_runs", capped_runs },
+    { "all_waves_at_once", all_waves_at_once },
 };
 
 } // namespace

@@ -465,7 +465,8 @@ std::vector<Slice> slices_of(uint64_t first, uint64_t photons, uint64_t most)
 
 /* Threads of a lockstep launch's workgroups for `waves` waves of work: half of
  * TMC_LOCK_BLOCK where that leaves fewer waves on the fullest compute unit, if
- * the waves are all resident (albedo 0.99: 50,000 photons, 98 workgroups of
+ * the waves are all resident (half as large, at least twice as many workgroups
+ * are: 8 of them take 60 KB of LDS, with the rejection sampler 6 take 90) (albedo 0.99: 50,000 photons, 98 workgroups of
  * eight waves or 196 of four, 237 and 198 us; 180,000 421 and 352 us), else
  * TMC_LOCK_BLOCK, with half as many sums to add up (2^17 photons at default
  * physics 58 and 61 us), which is what a cycle of fewer than 64 steps takes. */
@@ -601,9 +602,17 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
                 const bool by_count = counted && lv == 0;
                 const uint32_t block = by_count ? TMC_LOCK_BLOCK : lock_block_for(waves, l.k1 - l.k0, grid_most, cus);
                 const uint32_t per_wg = block / 64u;
-                const uint32_t grid = std::max(
-                    l.stripes, (uint32_t)std::min<double>(by_count ? (uint32_t)counted_cu * cus : grid_most,
-                                                          std::ceil(waves / (double)per_wg)));
+                /* (of half the size twice as many, with the rejection sampler:
+                 * its waves' passes over retries differ, and one that takes a
+                 * second batch ends late.  262,145 to 327,680 photons, albedo
+                 * 0.99, capped as the large ones and all at once: 826 and 765
+                 * to 957 and 888 us; analytic 490 and 495 at 300,000, default
+                 * physics 93 and 96 us, for the sums) */
+                const uint32_t most = by_count ? (uint32_t)counted_cu * cus
+                    : o->sampler == TMC_SAMPLER_REJECTION ? grid_most * (TMC_LOCK_BLOCK / block)
+                                                          : grid_most;
+                const uint32_t grid =
+                    std::max(l.stripes, (uint32_t)std::min<double>(most, std::ceil(waves / (double)per_wg)));
                 l.chunk = 0;
                 if (lv == 0) {
                     grid0 = grid;
