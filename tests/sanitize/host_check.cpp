@@ -127,16 +127,23 @@ uint64_t submit(tmc_server* s, uint64_t photons)
     return id;
 }
 
-int batch(uint64_t photons, tmc_batch_stats* stats = nullptr)
+int batch(uint64_t photons, uint32_t nsets = 3, float mu_a = 2.0f, bool keep = false)
 {
-    std::vector<tmc_set> sets(3);
+    std::vector<tmc_set> sets(nsets);
     for (tmc_set& q : sets) {
         std::memset(&q, 0, sizeof q);
-        q.params = params(photons);
+        q.params = params(photons, mu_a);
     }
-    std::vector<uint64_t> tally(tmc_batch_tally_words(sets.data(), 3));
+    std::vector<uint64_t> tally(tmc_batch_tally_words(sets.data(), nsets));
     tmc_batch_stats st;
-    return tmc_batch_run(sets.data(), 3, nullptr, tally.data(), stats ? stats : &st);
+    if (!keep)
+        return tmc_batch_run(sets.data(), nsets, nullptr, tally.data(), &st);
+    tmc_batch_plan* plan = nullptr;
+    int rc = tmc_batch_plan_create(sets.data(), nsets, nullptr, &plan);
+    if (rc == TMC_OK)
+        rc = tmc_batch_plan_run(plan, tally.data(), &st);
+    tmc_batch_plan_destroy(plan);
+    return rc;
 }
 
 // A request that arrives while a run's launches are queued: the serving kernel
@@ -197,7 +204,7 @@ void memory_beside_server()
     CHECK(fake::launched().walk == 4 && fake::live_bytes() - before < 1u << 20);
     tmc_set q;
     std::memset(&q, 0, sizeof q);
-    q.params = params(1u << 24);
+    q.params = params(1u << 24, 0.2f);
     tmc_batch_plan* plan = nullptr;
     CHECK(tmc_batch_plan_create(&q, 1, nullptr, &plan) == TMC_OK);
     CHECK(fake::live_bytes() - before < 2u << 20);
@@ -216,7 +223,7 @@ void enormous_set()
     fake::reset();
     tmc_set q;
     std::memset(&q, 0, sizeof q);
-    q.params = params(1ull << 48);
+    q.params = params(1ull << 48, 0.2f);
     tmc_batch_plan* plan = nullptr;
     g_largest = 0;
     CHECK(tmc_batch_plan_create(&q, 1, nullptr, &plan) == TMC_OK);
@@ -255,6 +262,28 @@ void all_waves_at_once()
     tiny_mc_gpu_shutdown();
 }
 
+// Batches of short cycles, and one-off batches of many small sets, by the
+// lane-per-photon walk; others in lockstep.
+void batch_walks()
+{
+    const struct {
+        uint32_t nsets;
+        uint64_t photons;
+        float mu_a;
+        bool keep, lock;
+    } forms[] = { { 3, 50000, 2.0f, false, true },  { 2000, 64, 2.0f, false, false }, { 2000, 64, 2.0f, true, true },
+                  { 64, 1 << 18, 2000.0f, true, false }, { 64, 1 << 18, 20.0f, true, false },
+                  { 64, 1 << 14, 20.0f, true, true }, { 2, 1 << 22, 2.0f, true, false },
+                  { 2, 1 << 22, 0.2f, false, true } };
+    for (const auto& f : forms) {
+        fake::reset();
+        CHECK(batch(f.photons, f.nsets, f.mu_a, f.keep) == TMC_OK);
+        CHECK((fake::launched().lock_sets > 0) == f.lock && (fake::launched().batch > 0) == !f.lock);
+    }
+    tiny_mc_gpu_shutdown();
+    CHECK(fake::live_bytes() == 0);
+}
+
 const struct {
     const char* name;
     void (*check)();
@@ -265,6 +294,7 @@ const struct {
     { "enormous_set", enormous_set },
     { "capped_runs", capped_runs },
     { "all_waves_at_once", all_waves_at_once },
+    { "batch_walks", batch_walks },
 };
 
 } // namespace

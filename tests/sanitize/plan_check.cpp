@@ -50,6 +50,36 @@ tmc_params params(float mu_a, float mu_s, uint32_t shells, float mps, uint64_t p
     return p;
 }
 
+// Which batches are walked in lockstep: long cycles; short ones only where there
+// are few photons; and not where all waves would append to one set's count, or
+// a plan for one run costs more than it gains.
+void check_lockstep_batch()
+{
+    using tmc::LockLoad;
+    constexpr double waves = 6144.0;
+    auto equal = [](size_t n, double photons, double k1) { return std::vector<LockLoad>(n, LockLoad{ photons, k1 }); };
+    for (const bool once : { false, true }) {
+        CHECK(!tmc::lockstep_batch({}, waves, once));
+        for (const double n : { 1.0, 1000.0, 1e6, 4e9, 0x1p63 }) {
+            CHECK(tmc::lockstep_batch(equal(8, n, 7946.0), waves, once));
+            CHECK(!tmc::lockstep_batch(equal(8, n, 1.0), waves, once));
+            CHECK(!tmc::lockstep_batch(equal(300, n, 5.0), waves, once));
+        }
+        CHECK(tmc::lockstep_batch(equal(64, 16384, 10.0), waves, once));
+        CHECK(!tmc::lockstep_batch(equal(64, 1 << 20, 10.0), waves, once));
+        CHECK(!tmc::lockstep_batch(equal(8, 1 << 22, 31.0), waves, once));
+        CHECK(!tmc::lockstep_batch(equal(8, 1 << 22, 73.0), waves, once));
+        CHECK(tmc::lockstep_batch(equal(2000, 64, 73.0), waves, once) == !once);
+        CHECK(tmc::lockstep_batch(equal(300, 65536, 73.0), waves, once) == !once);
+        // a large set of short cycles among others that take most of the time
+        std::vector<LockLoad> mix = equal(64, 16384, 5000.0);
+        mix.push_back({ 1 << 22, 30.0 });
+        CHECK(tmc::lockstep_batch(mix, waves, once));
+        mix[64].photons *= 64.0;
+        CHECK(!tmc::lockstep_batch(mix, waves, once));
+    }
+}
+
 void check_params_and_cadence()
 {
     const float inf = std::numeric_limits<float>::infinity(), nan = std::numeric_limits<float>::quiet_NaN();
@@ -332,6 +362,7 @@ void check_chunk_scale()
 int main()
 {
     check_params_and_cadence();
+    check_lockstep_batch();
     check_plans();
     check_arena();
     check_chunk_photons();

@@ -92,9 +92,6 @@ constexpr uint64_t kTableEntries = 1ull << 26;
  * lockstep waves too: with fewer, their 64-photon batches leave most of the
  * chip's 8192 waves without one. */
 constexpr double kSecondCycle = 200000.0;
-/* Absorptions of a wave in its shortest chunk (a chunk of another set costs
- * a flush of the slot, about 10 us). */
-constexpr double kChunkSteps = 512.0;
 constexpr uint32_t kLockBlock = 256;
 
 /* Absorptions to a set's first roulette, and from there to the second (0: the
@@ -266,13 +263,35 @@ uint32_t cuts_for(double n)
 /* Plans the lockstep launches of a batch; leaves p->lock off where they don't
  * apply: with the rejection sampler, with a cap on the absorptions, where the
  * caller chose a launch shape, with more than TMC_LOCK_SHELLS shells, where the weight tables or a first
- * cycle are longer than is worth laying out, and beside a server that has the device.  TMC_OK, or TMC_E_HIP. */
-int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_batch_options* o, uint64_t kcap,
+ * cycle are longer than is worth laying out, where walk_multi is faster (tmc::lockstep_batch), and beside a server
+ * that has the device.  `once`: the plan is made for one run.  TMC_OK, or TMC_E_HIP. */
+int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_batch_options* o, bool once, uint64_t kcap,
               const std::vector<tmc::BatchSet>& hs, const std::vector<Cadence>& cad, tmc_batch_plan* p)
 {
     LockPlan& l = p->lock;
     if (o->sampler != TMC_SAMPLER_ANALYTIC || o->block || o->waves_per_simd || o->copies || o->chunk_work
         || kcap != 0xFFFFFFFFull || p->shells_max > TMC_LOCK_SHELLS || p->photons == 0 || tmc::serving())
+        return TMC_OK;
+
+    /* launch shape */
+    int per_cu = 0;
+    if (tmc::lock_sets_occupancy(p->math, kLockBlock, p->shells_max, &per_cu) != hipSuccess)
+        return TMC_E_HIP;
+    if (per_cu <= 0)
+        return TMC_OK;
+    l.cus = (uint32_t)c->compute_units;
+    l.grid = (uint32_t)per_cu * l.cus;
+    const double waves = (double)l.grid * (kLockBlock / 64u);
+
+    std::vector<tmc::LockLoad> load;
+    for (uint32_t i = 0; i < nsets; ++i) {
+        if (!sets[i].params.photons)
+            continue;
+        if (cad[i].k1 == 0)
+            return TMC_OK;
+        load.push_back({ (double)sets[i].params.photons, (double)cad[i].k1 });
+    }
+    if (!tmc::lockstep_batch(load, waves, once))
         return TMC_OK;
 
     /* the sets' cadences and tables, and their parts */
@@ -288,8 +307,6 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
         const uint64_t n = sets[i].params.photons;
         if (n == 0)
             continue;
-        if (cad[i].k1 == 0)
-            return TMC_OK;
         const uint32_t cuts = std::max(cuts_for((double)n), l.cycles + 2u);
         /* (later cycles can be a step longer than the second; two entries are
          * read ahead of the last) */
@@ -323,18 +340,8 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
     }
     l.parts = (uint32_t)parts.size();
 
-    /* launch shape */
-    int per_cu = 0;
-    if (tmc::lock_sets_occupancy(p->math, kLockBlock, p->shells_max, &per_cu) != hipSuccess)
-        return TMC_E_HIP;
-    if (per_cu <= 0)
-        return TMC_OK;
-    l.cus = (uint32_t)c->compute_units;
-    l.grid = (uint32_t)per_cu * l.cus;
-
     /* slices, places and queues: chunks of a wave's 32nd of a launch's work,
      * longest first */
-    const double waves = (double)l.grid * (kLockBlock / 64u);
     struct Run { /* chunks of a part, of one length */
         double steps;
         uint32_t part, first, each, chunks;
@@ -373,9 +380,9 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
         }
         for (size_t j = begin; j < i; ++j) {
             const Cadence& k = cad[parts[j].set];
-            cut(0, (uint32_t)j, parts[j].count, (double)k.k1, std::max(kChunkSteps, steps[0] / waves / 32.0));
+            cut(0, (uint32_t)j, parts[j].count, (double)k.k1, std::max(tmc::kLockChunkSteps, steps[0] / waves / 32.0));
             if (l.cycles > 1u)
-                cut(1, (uint32_t)j, ls[j].cap[0], (double)k.k2, std::max(kChunkSteps, steps[1] / waves / 32.0));
+                cut(1, (uint32_t)j, ls[j].cap[0], (double)k.k2, std::max(tmc::kLockChunkSteps, steps[1] / waves / 32.0));
             cut(2, (uint32_t)j, ls[j].cap[l.cycles - 1u], (double)k.k2, 1.0);
         }
         for (uint32_t level = 0; level < 3u; ++level) {
@@ -453,7 +460,7 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
     return TMC_OK;
 }
 
-int plan_create_locked(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_batch_options* o,
+int plan_create_locked(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_batch_options* o, bool once,
                        tmc_batch_plan** out)
 {
     if (o->sampler > TMC_SAMPLER_REJECTION || o->math > TMC_MATH_OWN)
@@ -594,7 +601,7 @@ int plan_create_locked(tmc::Context* c, const tmc_set* sets, uint32_t nsets, con
 
     int lrc = TMC_OK;
     try {
-        lrc = plan_lock(c, sets, nsets, o, kcap, hs, cad, p);
+        lrc = plan_lock(c, sets, nsets, o, once, kcap, hs, cad, p);
     } catch (const std::bad_alloc&) {
         p->lock.on = false; /* (its queue is the largest of the host's tables) */
     }
@@ -718,8 +725,9 @@ TMC_EXPORT uint64_t tmc_batch_tally_words(const tmc_set* sets, uint32_t nsets)
     return w;
 }
 
-TMC_EXPORT int tmc_batch_plan_create(const tmc_set* sets, uint32_t nsets, const tmc_batch_options* opt,
-                                     tmc_batch_plan** plan)
+namespace {
+
+int plan_create(const tmc_set* sets, uint32_t nsets, const tmc_batch_options* opt, bool once, tmc_batch_plan** plan)
 {
     if (!plan)
         return TMC_E_INVALID;
@@ -737,7 +745,15 @@ TMC_EXPORT int tmc_batch_plan_create(const tmc_set* sets, uint32_t nsets, const 
     rc = tmc::acquire_context(&c);
     if (rc != TMC_OK)
         return rc;
-    return plan_create_locked(c, sets, nsets, &o, plan);
+    return plan_create_locked(c, sets, nsets, &o, once, plan);
+}
+
+} // namespace
+
+TMC_EXPORT int tmc_batch_plan_create(const tmc_set* sets, uint32_t nsets, const tmc_batch_options* opt,
+                                     tmc_batch_plan** plan)
+{
+    return plan_create(sets, nsets, opt, false, plan);
 }
 
 TMC_EXPORT int tmc_batch_plan_run(tmc_batch_plan* plan, uint64_t* tallies, tmc_batch_stats* stats)
@@ -764,7 +780,7 @@ TMC_EXPORT int tmc_batch_run(const tmc_set* sets, uint32_t nsets, const tmc_batc
                              tmc_batch_stats* stats)
 {
     tmc_batch_plan* plan = nullptr;
-    int rc = tmc_batch_plan_create(sets, nsets, opt, &plan);
+    int rc = plan_create(sets, nsets, opt, true, &plan);
     if (rc != TMC_OK)
         return rc;
     rc = tmc_batch_plan_run(plan, tallies, stats);

@@ -146,6 +146,54 @@ bool tmc::cohort_shape(uint64_t photons, uint64_t most, double L, uint32_t shell
     return true;
 }
 
+/* Measured on MI355X, equal sets, a run of a kept plan by walk_multi and by the
+ * lockstep launches.  Launching 64 photons and appending their survivors costs
+ * about 17 ps a photon, which a cycle of 30 absorptions (1.95 and 1.65 ps each)
+ * earns back: 131e6 photons in 2000 sets, first cycles of 2, 5, 10, 31 and, 20e6
+ * in 300 sets, 73 absorptions: 1.46 and 2.84, 2.20 and 3.26, 3.22 and 4.26, 8.66
+ * and 8.53, 3.26 and 2.83 ms.  In shorter cycles it is for the batches that
+ * walk_multi's lanes walk in one claim each, 0.5 ms however few they are
+ * (cycles of 10: 64 sets of 2^16 photons 603 and 553 us, 8 of 2^18 582 and 533,
+ * of 2^20 659 and 789; 2000 of one photon 381 and 417), down to cycles of 8 (of 2:
+ * 8 sets of 2^14 386 and 449 us, of 2^18 621 and 1098).
+ *
+ * All waves append to the count of the set they walk, and additions to one
+ * address take more than 11 ns each, while 8192 waves end a batch of 64 photons
+ * every 0.1 k1 ns: with k1 below 120 and not enough sets under way at a time
+ * they wait for one another (eight sets of 2^22 photons, cycles of 31: 2.60
+ * and 4.62 ms, of 73: 5.61 and 6.57, of 2^20, 73: 1.65 and 1.69).
+ *
+ * A plan made for one run has to earn what laying it out and releasing it takes
+ * more, 0.1 ms and 0.1 us a set, and 0.3 ms for large lists (planned, run and
+ * released, default physics: 2000 sets of 64 photons 863 and 920 us, of 1000
+ * 1394 and 1296; 10,000 of 1000 4816 and 5670; 8 of 2^20 1845 and 1981; cycles of
+ * 10, 64 of 2^14 681 and 519, of 2^16 706 and 792; albedo 0.99: 2000 of 1000 7022
+ * and 5655, 8 of 2^18 4701 and 3568). */
+bool tmc::lockstep_batch(const std::vector<LockLoad>& sets, double waves, bool once)
+{
+    double photons = 0.0, steps = 0.0;
+    for (const LockLoad& s : sets) {
+        photons += s.photons;
+        steps += s.photons * s.k1;
+    }
+    const double n = (double)sets.size(), mean = photons > 0.0 ? steps / photons : 0.0;
+    constexpr double many = 4194304.0;
+    if (mean < 8.0 || (mean < 30.0 && (photons >= many || n > 1000.0)))
+        return false;
+    if (once && (steps < 40.0 * n * n || (photons >= many && mean < 100.0) || (photons > many / 4.0 && mean < 30.0)))
+        return false;
+    /* work of the sets whose waves wait for their count: a wave's 32nd of a
+     * launch is a chunk */
+    const double each = std::max(kLockChunkSteps, steps / 64.0 / waves / 32.0);
+    double waits = 0.0;
+    for (const LockLoad& s : sets) {
+        const double chunks = s.photons / 64.0 / std::ceil(each / s.k1);
+        if (s.k1 * std::max(1.0, waves / chunks) < 120.0)
+            waits += s.photons * s.k1;
+    }
+    return waits <= steps / 8.0;
+}
+
 /* Entries of the binary32 walk's weight table (0: the walk multiplies).
  * The table is built per workgroup when the launch starts, so small runs
  * multiply; it must span the first cycle and eight more (a photon survives

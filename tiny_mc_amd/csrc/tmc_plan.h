@@ -84,6 +84,21 @@ struct CohortShape {
  * on cus compute units; false if the run is not one for the cohort walk. */
 bool cohort_shape(uint64_t photons, uint64_t most, double L, uint32_t shells, uint32_t cus, CohortShape* shape);
 
+/* A set of a batch as lockstep_batch() sees it: photons, and absorptions to the
+ * first roulette. */
+struct LockLoad {
+    double photons, k1;
+};
+
+/* Absorptions of a lockstep wave of a batch in its shortest chunk (a chunk of
+ * another set costs a flush of the wave's sums, about 10 us). */
+constexpr double kLockChunkSteps = 512.0;
+
+/* Whether the lockstep launches of a batch are at least as fast as the
+ * lane-per-photon ones (walk_multi), on `waves` resident waves; `once`: the
+ * plan is made for a single run.  (tmc_plan.cpp has the reasons.) */
+bool lockstep_batch(const std::vector<LockLoad>& sets, double waves, bool once);
+
 /* Entries of the single run's weight table for these parameters and the
  * caller's request (tmc_options.weight_table; 0: none). */
 uint32_t weight_table_entries(const tmc_params* p, uint32_t precision, uint64_t photons, uint32_t request);
