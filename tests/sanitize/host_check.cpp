@@ -23,11 +23,14 @@
     } while (0)
 
 static size_t g_largest = 0; // of the host's allocations
+static long g_fail_new = -1; // the one that fails (0: the next)
 
 void* operator new(size_t n)
 {
     if (n > g_largest)
         g_largest = n;
+    if (g_fail_new >= 0 && g_fail_new-- == 0)
+        throw std::bad_alloc();
     if (void* p = std::malloc(n ? n : 1))
         return p;
     throw std::bad_alloc();
@@ -284,6 +287,34 @@ void batch_walks()
     CHECK(fake::live_bytes() == 0);
 }
 
+// Each of the host's own allocations of a run fails in turn: the run takes the
+// lane-per-photon walk, and nothing is thrown at the caller.
+void failed_host_allocations()
+{
+    for (const Form& f : kForms) {
+        fake::reset();
+        CHECK(run(params(f.photons), f.precision) == TMC_OK && fake::launched().*f.kernel > 0);
+        const int ordinary = fake::launched().*f.kernel;
+        for (long n = 0;; ++n) {
+            fake::reset();
+            const tmc_params p = params(f.photons);
+            std::vector<uint64_t> tally(4 * (size_t)p.shells);
+            tmc_options o;
+            tmc_options_default(&o);
+            o.precision = f.precision;
+            g_fail_new = n;
+            CHECK(tiny_mc_gpu_run_ex(&p, 1, &o, tally.data(), nullptr) == TMC_OK);
+            const bool failed = g_fail_new < 0;
+            g_fail_new = -1;
+            CHECK(failed ? fake::launched().walk == 1 : fake::launched().*f.kernel == ordinary);
+            if (!failed)
+                break;
+        }
+    }
+    tiny_mc_gpu_shutdown();
+    CHECK(fake::live_bytes() == 0);
+}
+
 const struct {
     const char* name;
     void (*check)();
@@ -295,6 +326,7 @@ const struct {
     { "capped_runs", capped_runs },
     { "all_waves_at_once", all_waves_at_once },
     { "batch_walks", batch_walks },
+    { "failed_host_allocations", failed_host_allocations },
 };
 
 } // namespace

@@ -821,13 +821,17 @@ int tmc::run_walk(Context* c, const tmc_params* p, uint64_t seed, const tmc_opti
      * server has the device */
     if (work == c->d_work && !o->block && !o->grid && !o->chunk && !o->weight_table && p->photons && !tmc::serving()
         && ensure_lockstep(c)) {
-        int rc;
-        if (o->precision == TMC_PRECISION_FP32) {
-            rc = run_cohort(c, p, seed, o, kcap, tally, st);
-            if (rc == TMC_E_UNSUPPORTED)
-                rc = run_lock(c, p, seed, o, kcap, tally, st);
-        } else {
-            rc = run_prec(c, p, seed, o, kcap, tally, st);
+        int rc = TMC_E_UNSUPPORTED;
+        try {
+            if (o->precision == TMC_PRECISION_FP32) {
+                rc = run_cohort(c, p, seed, o, kcap, tally, st);
+                if (rc == TMC_E_UNSUPPORTED)
+                    rc = run_lock(c, p, seed, o, kcap, tally, st);
+            } else {
+                rc = run_prec(c, p, seed, o, kcap, tally, st);
+            }
+        } catch (const std::bad_alloc&) {
+            /* (all that they allocate is there before the first launch) */
         }
         if (rc == TMC_OK && st) {
             st->photons = p->photons;
