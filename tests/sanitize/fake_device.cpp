@@ -21,6 +21,7 @@
 
 namespace fake {
 
+std::vector<std::pair<uint64_t, uint64_t>> slices;
 long fail_alloc = -1;
 size_t alloc_limit = SIZE_MAX;
 bool overflow = false;
@@ -149,6 +150,7 @@ void reset()
     fail_alloc = -1;
     alloc_limit = SIZE_MAX;
     overflow = false;
+    slices.clear();
 }
 
 void hold(bool on)
@@ -351,6 +353,8 @@ hipError_t launch_lock(uint32_t, uint32_t, bool, const LockArgs& a, uint32_t gri
     counted(&Launches::lock);
     lock_grid = grid;
     lock_block = block;
+    if (!a.level)
+        slices.push_back({ a.first_photon, a.photons });
     if (!a.cap_ends)
         touch(a.out, (size_t)a.stripes * a.out_cap);
     if (a.level)
@@ -385,6 +389,10 @@ hipError_t launch_prec_table(uint32_t precision, const PrecArgs& a, uint32_t* co
 hipError_t launch_prec(uint32_t, uint32_t, const PrecArgs& a, uint32_t, uint32_t, hipStream_t)
 {
     counted(&Launches::prec);
+    if (!a.level)
+        slices.push_back({ a.first_photon, a.photons });
+    if (a.cycles)
+        touch(a.out.photon, 4ull * a.stripes * a.out_cap - 4u, 4);
     if (overflow)
         a.work[2] |= TMC_LOCK_OVERFLOW;
     return launch_status();

@@ -9,6 +9,8 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <utility>
+#include <vector>
 
 namespace fake {
 
@@ -33,6 +35,8 @@ extern bool overflow;
 
 // A launch of lockstep waves: workgroups and threads of the last one.
 extern uint32_t lock_grid, lock_block;
+// First photon and photons of each first level since reset().
+extern std::vector<std::pair<uint64_t, uint64_t>> slices;
 // Entries of the last weight table.
 extern uint32_t table_entries;
 

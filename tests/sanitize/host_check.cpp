@@ -315,6 +315,62 @@ void failed_host_allocations()
     CHECK(fake::live_bytes() == 0);
 }
 
+// A survivor that finds no room in its list: the call is repeated by the other
+// walk, and the next one is in lockstep again.
+void full_lists()
+{
+    const Form lock[] = { kForms[1], { 300000, TMC_PRECISION_FP32_WEIGHT, &fake::Launches::prec }, kForms[3] };
+    for (const Form& f : lock) {
+        fake::reset();
+        fake::overflow = true;
+        CHECK(run(params(f.photons), f.precision) == TMC_OK);
+        CHECK(fake::launched().*f.kernel > 0 && fake::launched().walk == 1);
+        fake::reset();
+        CHECK(run(params(f.photons), f.precision) == TMC_OK);
+        CHECK(fake::launched().*f.kernel > 0 && fake::launched().walk == 0);
+    }
+    for (const bool keep : { false, true }) {
+        fake::reset();
+        fake::overflow = true;
+        CHECK(batch(50000, 3, 2.0f, keep) == TMC_OK);
+        CHECK(fake::launched().lock_sets > 0 && fake::launched().batch == 1);
+        fake::reset();
+        CHECK(batch(50000, 3, 2.0f, keep) == TMC_OK);
+        CHECK(fake::launched().lock_sets > 0 && fake::launched().batch == 0);
+    }
+    tiny_mc_gpu_shutdown();
+    CHECK(fake::live_bytes() == 0);
+}
+
+// The slices of a large run: all its photons in order, at most 2^27 in each and
+// one high index word, and lists whose places the launches find there.
+void slices()
+{
+    const uint64_t photons[] = { 1u << 17, 3000017, 1ull << 27, (1ull << 27) + 1, (1ull << 28) - 1, 5ull << 27 };
+    const uint64_t firsts[] = { 0, 1, (1ull << 32) - 1, (1ull << 32) - (1ull << 26), (7ull << 32) - 40000 };
+    for (const uint32_t precision : { TMC_PRECISION_FP32, TMC_PRECISION_FP32_COMPENSATED, TMC_PRECISION_FP64 })
+        for (const uint64_t n : photons)
+            for (const uint64_t first : firsts) {
+                fake::reset();
+                const tmc_params p = params(n);
+                std::vector<uint64_t> tally(4 * (size_t)p.shells);
+                tmc_options o;
+                tmc_options_default(&o);
+                o.precision = precision;
+                o.first_photon = first;
+                CHECK(tiny_mc_gpu_run_ex(&p, 1, &o, tally.data(), nullptr) == TMC_OK && fake::launched().walk == 0);
+                uint64_t at = first;
+                for (const auto& s : fake::slices) {
+                    CHECK(s.first == at && s.second > 0 && s.second <= 1ull << 27);
+                    CHECK(s.first >> 32 == (s.first + s.second - 1) >> 32);
+                    at += s.second;
+                }
+                CHECK(at == first + n);
+            }
+    tiny_mc_gpu_shutdown();
+    CHECK(fake::live_bytes() == 0);
+}
+
 const struct {
     const char* name;
     void (*check)();
@@ -327,6 +383,8 @@ const struct {
     { "all_waves_at_once", all_waves_at_once },
     { "batch_walks", batch_walks },
     { "failed_host_allocations", failed_host_allocations },
+    { "full_lists", full_lists },
+    { "slices", slices },
 };
 
 } // namespace

@@ -80,6 +80,67 @@ void check_lockstep_batch()
     }
 }
 
+// The weight table's sequence against the cadence and a walk of its own, and
+// rooms that end it before a roulette, at one and after one.
+void check_weight_sequence()
+{
+    for (const tmc_params& p : { params(2, 20, 101, 50), params(10, 10, 51, 100), params(0.5f, 50, 201, 20),
+                                 params(100, 1e-30f, 3, 50), params(1, 0, 3, 50), params(0.01f, 100, 401, 10) }) {
+        const float a = tmc::derived_albedo(&p);
+        uint32_t k1 = 0, k2 = 0;
+        CHECK(tmc::weight_cadence(&p, 1u << 20, &k1, &k2));
+        for (const uint32_t cuts : { 1u, 3u, 30u })
+            for (const uint32_t room : { 1u, k1 - 1u, k1, k1 + 1u, k1 + k2, 300000u }) {
+                std::vector<float> weight(room);
+                std::vector<uint32_t> cut(cuts, 0u);
+                float w_end = -1.0f;
+                const uint32_t n = tmc::weight_sequence(&p, room, cuts, weight.data(), cut.data(), &w_end);
+                CHECK(n <= cuts);
+                CHECK(n == cuts || (n ? cut[n - 1] : 0u) <= room);
+                if (n > 0)
+                    CHECK(cut[0] == k1);
+                if (n > 1)
+                    CHECK(cut[1] == k1 + k2);
+                CHECK((n == 0) == (room < k1));
+                const uint32_t entries = n == cuts ? cut[n - 1] : room;
+                volatile float w = 1.0f; // (rounded to binary32 at every step)
+                uint32_t c = 0;
+                for (uint32_t k = 0; k < entries; ++k) {
+                    CHECK(weight[k] == w);
+                    w = w * a;
+                    if (w < 0.001f) {
+                        w = w / 0.1f;
+                        CHECK(c < n && cut[c] == k + 1);
+                        ++c;
+                    }
+                }
+                CHECK(c == n && w_end == w);
+            }
+    }
+}
+
+// The cohort walk's launch shape: every photon in a cohort, waves for three
+// coordinates of each, blocks of sums that fit the run's words.
+void check_cohort_shape()
+{
+    tmc::CohortShape s;
+    for (const uint32_t cus : { 1u, 7u, 256u })
+        for (const uint64_t n : { 1ull, 2ull, 63ull, 64ull, 65ull, 512ull, 4097ull, 32768ull, 49152ull, 131072ull })
+            for (const double L : { 1.0, 199.0, 200.0, 1e5 })
+                for (const uint32_t shells : { 1u, 101u, 451u, (uint32_t)TMC_MAX_SHELLS }) {
+                    CHECK(tmc::cohort_shape(n, n, L, shells, cus, &s));
+                    CHECK(s.group >= 1 && s.group <= 64 && (s.group & (s.group - 1)) == 0);
+                    CHECK((uint64_t)s.group * s.groups >= n && (uint64_t)s.group * (s.groups - 1) < n);
+                    CHECK(s.moving * 64 >= 3 * s.group && s.drawing >= 1 && s.drawing + s.moving == 15);
+                    CHECK(s.grid >= 1 && s.grid <= cus && s.grid <= s.groups);
+                    CHECK(s.copies >= 1 && s.copies <= 8);
+                    CHECK((uint64_t)s.copies * (4 + 4ull * shells) <= 4 + 4ull * TMC_MAX_SHELLS);
+                    CHECK(!tmc::cohort_shape(n, n - 1, L, shells, cus, &s));
+                }
+    CHECK(!tmc::cohort_shape(0, 100, 80.0, 101, 256, &s));
+    CHECK(!tmc::cohort_shape(1, 100, 80.0, 101, 0, &s));
+}
+
 void check_params_and_cadence()
 {
     const float inf = std::numeric_limits<float>::infinity(), nan = std::numeric_limits<float>::quiet_NaN();
@@ -363,6 +424,8 @@ int main()
 {
     check_params_and_cadence();
     check_lockstep_batch();
+    check_weight_sequence();
+    check_cohort_shape();
     check_plans();
     check_arena();
     check_chunk_photons();
