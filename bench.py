@@ -240,6 +240,7 @@ def sweep_leg(tuned_runs=3, default_runs=2):
         "chunks": st.chunks,
         "lane_utilisation": st.lane_utilisation,
         "autotune_seconds": tune_s,
+        # the shape of the persistent launches; with automatic options the plan walks in lockstep instead
         "launch": {"passes": st.passes, "grid": st.grid, "block": st.block, "waves_per_simd": st.waves_per_simd,
                    "copies": st.copies, "chunk_work": st.chunk_work, "hip_graph": True,
                    "options": {"block": tuned.block, "waves_per_simd": tuned.waves_per_simd, "copies": tuned.copies,
@@ -447,7 +448,7 @@ def main():
         "data": "synthetic",
         "config": {
             "workload": f"plain walk at scale: {args.photons} photons, default physics (mu_a=2/cm, mu_s=20/cm, "
-                        "101 shells x 50 um, cutoff 0.001, roulette 0.1), one launch per step",
+                        "101 shells x 50 um, cutoff 0.001, roulette 0.1), one run per step",
             "photons_per_step": args.photons,
             "shells": 101,
             "sampler": args.sampler,

@@ -115,7 +115,8 @@ typedef struct tmc_run_stats {
     uint32_t sampler;
     uint32_t precision;
     uint32_t math;
-    uint32_t weight_table; /* entries of the weight table used (0: none) */
+    uint32_t weight_table; /* entries of the weight table used (0: none); runs in lockstep have tables of their own
+                              and give those that the lane-per-photon walk would use */
 } tmc_run_stats;
 
 /* Default options (analytic sampler, automatic launch shape, photon 0). */
@@ -231,9 +232,10 @@ int tiny_mc_gpu_check_shell_index(const tmc_params* p, uint32_t first_bits, uint
 
 /* ------------------------------------------------------------------------
  * Batched sweep: many parameter sets in a few launches back to back.  With
- * the analytic sampler and every launch option automatic, waves walk 64
- * photons of a set in lockstep and survivors of a roulette go through lists
- * that the plan holds; otherwise one persistent launch (one per LDS size
+ * the analytic sampler, every launch option automatic and first cycles long
+ * enough to gain by it, waves walk 64 photons of a set in lockstep and
+ * survivors of a roulette go through lists that the plan holds; otherwise one
+ * persistent launch (one per LDS size
  * class of the sets, up to three).  Same results.
  *
  * No counterpart in the reference (it has one compile-time parameter set);

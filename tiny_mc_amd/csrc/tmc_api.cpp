@@ -1,10 +1,11 @@
 /* C ABI of the photon-transport path (include/tiny_mc_gpu.h).
  *
  * Host side of one run: validate the params.h-style parameters, derive the
- * binary32 constants exactly as photon.c:8-9 does, clear the device tallies
- * and claim counter, launch the persistent walk kernel once, and copy the
- * 128-bit integer tallies back.  The conversion to the reference's heat /
- * heat2 units is done in double on the host.
+ * binary32 constants exactly as photon.c:8-9 does, form the weights, and launch
+ * the lockstep walks, whose last workgroup writes the 128-bit integer tallies
+ * into host memory; or, where those don't apply, clear the device words, launch
+ * the persistent walk kernel once, and copy the tallies back.  The conversion to
+ * the reference's heat / heat2 units is done in double on the host.
  */
 #include <hip/hip_runtime.h>
 
@@ -288,17 +289,6 @@ bool weigh(Context* c, const tmc_params* p, uint64_t seed, uint64_t kcap, uint32
     return true;
 }
 
-/* Roulettes the table of a run of n photons spans: as many as one of its
- * photons survives but in one run in a thousand (that photon walks on without
- * the table). */
-uint32_t cuts_for(double n)
-{
-    uint32_t cuts = 3;
-    for (; n >= 1.0 && cuts < TMC_COHORT_CUTS; n *= 0.1)
-        ++cuts;
-    return cuts;
-}
-
 /* About the absorptions of a photon's first cycle (the weight falls to a
  * thousandth), at most kcap. */
 double first_cycle(const tmc_params* p, uint64_t kcap)
@@ -366,7 +356,7 @@ int run_cohort(Context* c, const tmc_params* p, uint64_t seed, const tmc_options
     if (!tmc::cohort_shape(p->photons, most, first_cycle(p, kcap), p->shells, (uint32_t)c->compute_units, &shape))
         return TMC_E_UNSUPPORTED;
     tmc::CohortArgs a;
-    if (!weigh(c, p, seed, kcap, cuts_for((double)p->photons), &a))
+    if (!weigh(c, p, seed, kcap, tmc::cuts_for((double)p->photons), &a))
         return TMC_E_UNSUPPORTED;
     a.build = a.entries <= TMC_COHORT_BUILD ? a.entries : 0u;
     if (tmc::cohort_lds_bytes(p->shells, a.build) > 160u * 1024u)
@@ -499,7 +489,7 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
     for (; rest > (double)kHandOver; rest *= 0.1)
         ++levels;
     tmc::CohortArgs a;
-    if (!weigh(c, p, seed, kcap, levels + cuts_for(rest), &a))
+    if (!weigh(c, p, seed, kcap, levels + tmc::cuts_for(rest), &a))
         return TMC_E_UNSUPPORTED;
     if (tmc::cohort_lds_bytes(p->shells, 0) > 160u * 1024u)
         return TMC_E_UNSUPPORTED;
@@ -677,7 +667,7 @@ int run_prec(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
     /* the table: the cuts that the last survivors are expected to need, each
      * cycle's length from its logarithm, and slack for the roundings on the way */
     const double l = -std::log(a.albedo_d), first = std::log(1000.0) / l, later = std::log(10.0) / l;
-    a.cuts = cuts_for((double)slice);
+    a.cuts = tmc::cuts_for((double)slice);
     const double room = 1.001 * (first + a.cuts * later) + 3.0 * a.cuts + 64.0;
     if (room > (double)tmc::kTableEntries - 16.0)
         return TMC_E_UNSUPPORTED;

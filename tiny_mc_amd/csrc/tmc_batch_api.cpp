@@ -21,7 +21,8 @@
  * chunk queue and cursor; the tallies and counters are shared.
  *
  * Lockstep: with the analytic sampler and automatic options the launches are
- * those of tmc_lock.hip and tmc_cohort.hip instead: waves carry 64 photons of
+ * those of tmc_lock.hip and tmc_cohort.hip instead, unless the sets' first
+ * cycles are too short for that (tmc::lockstep_batch): waves carry 64 photons of
  * a set in lockstep to the first roulette, and append the tenth that survives
  * to the set's places in a list; where a batch leaves enough of them they are
  * walked to the second roulette the same way, and workgroups carry what is
@@ -87,7 +88,7 @@ constexpr size_t kParts = 1u << 20;
 /* Places of a slice's first list: 0.9 GB. */
 constexpr uint64_t kSlicePlaces = 1ull << 25;
 /* Entries of the weight tables of a batch: 1 GB. */
-constexpr uint64_t kTableEntries = 1ull << 26;
+constexpr uint64_t kBatchEntries = 1ull << 26;
 /* Expected survivors of a roulette from which on the next cycle is walked by
  * lockstep waves too: with fewer, their 64-photon batches leave most of the
  * chip's 8192 waves without one. */
@@ -250,16 +251,6 @@ hipError_t launch_shape(const tmc_batch_plan* p, const tmc_batch_options* o, uin
     return hipSuccess;
 }
 
-/* Roulettes of a weight table for n photons: three more than the last of
- * them is expected to survive. */
-uint32_t cuts_for(double n)
-{
-    uint32_t cuts = 3;
-    for (; n >= 1.0 && cuts < TMC_COHORT_CUTS; n *= 0.1)
-        ++cuts;
-    return cuts;
-}
-
 /* Plans the lockstep launches of a batch; leaves p->lock off where they don't
  * apply: with the rejection sampler, with a cap on the absorptions, where the
  * caller chose a launch shape, with more than TMC_LOCK_SHELLS shells, where the weight tables or a first
@@ -307,7 +298,7 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
         const uint64_t n = sets[i].params.photons;
         if (n == 0)
             continue;
-        const uint32_t cuts = std::max(cuts_for((double)n), l.cycles + 2u);
+        const uint32_t cuts = std::max(tmc::cuts_for((double)n), l.cycles + 2u);
         /* (later cycles can be a step longer than the second; two entries are
          * read ahead of the last) */
         const uint64_t room = cad[i].k1 + (uint64_t)(cuts - 1u) * (cad[i].k2 + 2u) + 64u;
@@ -324,7 +315,7 @@ int plan_lock(tmc::Context* c, const tmc_set* sets, uint32_t nsets, const tmc_ba
         s.entries = (uint32_t)room;
         s.cuts = cuts;
         entries += room + 2u;
-        if (entries > kTableEntries)
+        if (entries > kBatchEntries)
             return TMC_OK;
         for (uint64_t done = 0; done < n;) {
             s.first_photon = hs[i].first_photon + done;

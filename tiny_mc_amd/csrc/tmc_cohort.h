@@ -9,6 +9,16 @@ namespace tmc {
 
 /* Roulettes a weight table spans at most. */
 #define TMC_COHORT_CUTS 30u
+/* Roulettes the weight table of n photons spans: three more than the last of
+ * them is expected to survive, so that one run in a thousand has a photon that
+ * outlives it (and walks on without the table). */
+inline uint32_t cuts_for(double n)
+{
+    uint32_t cuts = 3;
+    for (; n >= 1.0 && cuts < TMC_COHORT_CUTS; n *= 0.1)
+        ++cuts;
+    return cuts;
+}
 /* Entries of the largest weight table the workgroups build in LDS, each for
  * itself; a longer one is converted once, by a launch ahead (8 us, where 256
  * workgroups reading 8 KB each from the host's memory take 25). */

@@ -28,7 +28,7 @@
  * drawing waves (16 waves a compute unit, about 3800 cycles a round of 24
  * rows).  Measured on MI355X, whole calls, lane per photon -> this walk: 20
  * photons at default physics 77 -> 22 us, 32,768 173 -> 48 us; 4096 at albedo
- * 0.99 (720 absorptions each) 1147 -> 53 us; 16,384 photons at albedo 0.9999
+ * 0.99 (720 absorptions each) 1147 -> 54 us; 16,384 photons at albedo 0.9999
  * through 20,000 absorptions 1.9 ms, 1.7e11 absorptions/s.
  *
  * Same words, same operations and the same integer sums as step(): results

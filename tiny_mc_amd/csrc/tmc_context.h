@@ -17,7 +17,10 @@ namespace tmc {
  * [1] absorptions, [2] truncated photons, [3] unused), then the 4 * shells
  * tally words.  The context allocates them once at the largest shell count
  * (run_work_words(TMC_MAX_SHELLS) words, 256 KiB) and keeps them until
- * shutdown, so no single run allocates or frees device memory. */
+ * shutdown, so no run of the lane-per-photon walk allocates or frees device
+ * memory.  The lockstep walks' 20 MB are kept in the same way from the first run
+ * on, and their lists, which grow with the largest run so far (to 0.6 GB, a
+ * precision variant's to 1.1 GB). */
 constexpr size_t kRunCounterWords = 4;
 constexpr size_t run_work_words(uint32_t shells) { return kRunCounterWords + 4 * (size_t)shells; }
 
@@ -60,8 +63,9 @@ int acquire_context(Context** out);
 /* One single run (tiny_mc_gpu_run_ex) with its counters and tallies in the
  * device words `work` (run_work_words(p->shells) of them): clears them with
  * a kernel, launches the walk, copies the tallies to `tally` (host) and
- * synchronises the context's stream.  Allocates nothing.  Call with
- * api_mutex() held; p is checked. */
+ * synchronises the context's stream.  Allocates nothing, but for the lockstep
+ * walks, which are for the context's own words only.  Call with api_mutex()
+ * held; p is checked. */
 int run_walk(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* o, unsigned long long* work,
              uint64_t* tally, tmc_run_stats* st);
 

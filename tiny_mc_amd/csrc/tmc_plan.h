@@ -69,7 +69,7 @@ struct CohortShape {
  * photon's absorptions, so the lines are numbers of photons (256 workgroups of
  * two cohorts of 64 photons, and of three).  Measured, cohort walk against
  * lockstep waves (walk_lock), default physics and albedo 0.99: 32,768 photons
- * 43 / 49 and 151 / 183 us, 40,960 54 / 51 and 210 / 188 us; rejection sampler
+ * 45 / 50 and 157 / 188 us, 40,960 54 / 51 and 210 / 188 us; rejection sampler
  * 49,152 75 / 75 and 316 / 386 us, 2^16 100 / 76 and 442 / 402 us.  Against lane
  * per photon (walk_f32): 2^17 121 / 185 us and 544 / 1218 us; 2^18 208 / 213 us
  * and 1008 / 1484 us; 2^19 381 / 304 us and 1963 / 1880 us. */
