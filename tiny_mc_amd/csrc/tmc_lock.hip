@@ -177,12 +177,17 @@ __device__ __forceinline__ void lock_cycle_counted(LockPhoton& p, uint32_t k1, u
 }
 
 /* Adds a workgroup's counts, each times its absorption's images, to a block of
- * the global sums. */
+ * the global sums.  A pair's absorptions go to four threads, or to one for each
+ * 32: every thread adds to the pair's words, and additions to one word take 7 to
+ * 16 ns each.  (With all threads at work on few shells 2^22 photons at default
+ * physics took 1994 us with one shell, 1354 with 8 and 884 with 24; so they take
+ * 782, 607 and 593, and 581 with 101 either way.) */
 __device__ __forceinline__ void count_flush(const uint32_t* counts, const Images* entry, uint32_t k1,
                                             unsigned long long* g, uint32_t shells)
 {
     const uint32_t last = shells - 1u, pairs = last + TMC_LOCK_HOT;
-    const uint32_t parts = pairs < blockDim.x ? blockDim.x / pairs : 1u; /* threads to a pair */
+    const uint32_t most = k1 / 32u > 4u ? k1 / 32u : 4u, room = pairs < blockDim.x ? blockDim.x / pairs : 1u;
+    const uint32_t parts = room < most ? room : most; /* threads to a pair */
     for (uint32_t i = threadIdx.x; i < pairs * parts; i += blockDim.x) {
         const uint32_t q = i % pairs;
         unsigned __int128 h = 0, h2 = 0;
