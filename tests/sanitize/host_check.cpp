@@ -371,6 +371,38 @@ void slices()
     CHECK(fake::live_bytes() == 0);
 }
 
+// Large runs of short cycles and of the precision variants with the rejection
+// sampler by the lane-per-photon walk; the sizes up to there in lockstep.
+void run_walks()
+{
+    const uint32_t rej = TMC_SAMPLER_REJECTION;
+    const struct {
+        float mu_a, mu_s;
+        uint32_t precision, sampler;
+        uint64_t most; // in lockstep
+    } lines[] = { { 100.0f, 1.0f, TMC_PRECISION_FP32, 0, 1ull << 26 },
+                  { 100.0f, 1.0f, TMC_PRECISION_FP32, rej, 5ull << 23 },
+                  { 20.0f, 5.0f, TMC_PRECISION_FP32, rej, 1ull << 26 },
+                  { 20.0f, 5.0f, TMC_PRECISION_FP32_WEIGHT, 0, 1ull << 26 },
+                  { 20.0f, 5.0f, TMC_PRECISION_FP32_COMPENSATED, rej, 1ull << 25 },
+                  { 20.0f, 5.0f, TMC_PRECISION_FP64, 0, 1ull << 25 },
+                  { 10.0f, 10.0f, TMC_PRECISION_FP64, rej, 1ull << 24 },
+                  { 2.0f, 20.0f, TMC_PRECISION_FP32_WEIGHT, rej, 1ull << 22 } };
+    for (const auto& l : lines)
+        for (const uint64_t over : { 0u, 1u }) {
+            fake::reset();
+            CHECK(run(params(l.most + over, l.mu_a, l.mu_s), l.precision, 0, 0, l.sampler) == TMC_OK);
+            CHECK(fake::launched().walk == (int)over);
+            CHECK((fake::launched().lock + fake::launched().prec > 0) == !over);
+        }
+    for (const uint32_t precision : { TMC_PRECISION_FP32, TMC_PRECISION_FP32_WEIGHT, TMC_PRECISION_FP64 }) {
+        fake::reset();
+        CHECK(run(params(1ull << 27, 10.0f, 10.0f), precision) == TMC_OK && fake::launched().walk == 0);
+    }
+    tiny_mc_gpu_shutdown();
+    CHECK(fake::live_bytes() == 0);
+}
+
 const struct {
     const char* name;
     void (*check)();
@@ -385,6 +417,7 @@ const struct {
     { "failed_host_allocations", failed_host_allocations },
     { "full_lists", full_lists },
     { "slices", slices },
+    { "run_walks", run_walks },
 };
 
 } // namespace

@@ -10,7 +10,7 @@ from test_sanitize import BUILD, SAN_ENV, built  # noqa: F401  (built: the fixtu
 
 @pytest.mark.parametrize("name", ["failed_allocations", "server_during_run", "memory_beside_server", "enormous_set",
                                   "capped_runs", "all_waves_at_once", "batch_walks",
-                                  "failed_host_allocations", "full_lists", "slices"])
+                                  "failed_host_allocations", "full_lists", "slices", "run_walks"])
 def test_host(built, name):  # noqa: F811
     r = subprocess.run([os.path.join(BUILD, "host_check"), name], capture_output=True, text=True, timeout=120,
                        env=SAN_ENV)

@@ -480,8 +480,12 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
      * the survivors costs what the step saves (2^27 photons, lane per photon
      * and here: albedo 1/6 1548 and 1685 us, with the rejection sampler 2216
      * and 2290 us; albedo 0.5 2849 and 2784 us, 4885 and 4696 us; 2^26 at 1/6
-     * 1049 and 850 us) */
-    if (p->photons > (1ull << 26) && first_cycle(p, kcap) < 8.0)
+     * 1049 and 850 us; rejection sampler at 0.01 and 0.09, 4 * 2^23 photons 663
+     * and 485, 684 and 635 us, 6 * 2^23 685 and 687, 814 and 909, 2^26 773 and
+     * 868, 970 and 1176; at 0.2, 2^26 1399 and 1306) */
+    const double first = first_cycle(p, kcap);
+    if (first < 8.0
+        && p->photons > (o->sampler == TMC_SAMPLER_REJECTION && first < 4.0 ? 5ull << 23 : 1ull << 26))
         return TMC_E_UNSUPPORTED;
     const uint64_t slice = std::min<uint64_t>(p->photons, 1ull << tmc::kSliceLog);
     uint32_t levels = 1;
@@ -648,12 +652,32 @@ int run_lock(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* 
  * a wave on each SIMD. */
 constexpr double kPackPhotons = 65536.0;
 
+/* Photons of the largest run of a precision variant for the lockstep waves.
+ * Short cycles end there for the reason they do in binary32, and the passes of a
+ * wave over the directions that the rejection sampler draws again cost more than
+ * lockstep saves on a full chip, which fewer photons of long walks fill.
+ * Measured, lane per photon and here: weight from counts, albedo 0.01, 2^26
+ * photons 804 and 776 us, 2^27 1222 and 1477; binary64 2^25 766 and 773, 2^26 1306
+ * and 1509; albedo 0.5 2^27 4.50 and 4.28, 11.13 and 11.35 ms.  Rejection sampler,
+ * weight from counts: albedo 0.2 2^25 1117 and 1118, 2^26 2025 and 2141 us; 0.5
+ * 2^24 1122 and 1089, 2^25 1988 and 2071 us; 0.8 2^23 1543 and 1553, 2^24 2895 and
+ * 2973 us; default 2^22 1904 and 1873, 2^23 3447 and 3509, 2^24 6470 and 6772 us;
+ * albedo 0.97 2^23 9780 and 9875 us. */
+uint64_t prec_most(const tmc_options* o, double first)
+{
+    const bool rejection = o->sampler == TMC_SAMPLER_REJECTION;
+    if (first < 8.0)
+        return rejection || o->precision == TMC_PRECISION_FP64 ? 1ull << 25 : 1ull << 26;
+    return !rejection ? 1ull << 36 : first < 25.0 ? 1ull << 24 : 1ull << 22;
+}
+
 /* One run with a precision variant's arithmetic by lockstep waves.
  * TMC_E_UNSUPPORTED: not one for them. */
 int run_prec(Context* c, const tmc_params* p, uint64_t seed, const tmc_options* o, uint64_t kcap, uint64_t* tally,
              tmc_run_stats* st)
 {
-    if (p->photons == 0 || p->photons > (1ull << 36) || p->shells > TMC_LOCK_SHELLS || kcap != 0xFFFFFFFFull)
+    if (p->photons == 0 || p->shells > TMC_LOCK_SHELLS || kcap != 0xFFFFFFFFull
+        || p->photons > prec_most(o, first_cycle(p, kcap)))
         return TMC_E_UNSUPPORTED;
     tmc::PrecArgs a;
     std::memset(&a, 0, sizeof a);
