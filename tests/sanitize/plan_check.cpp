@@ -56,7 +56,7 @@ tmc_params params(float mu_a, float mu_s, uint32_t shells, float mps, uint64_t p
 void check_lockstep_batch()
 {
     using tmc::LockLoad;
-    constexpr double waves = 6144.0;
+    constexpr double waves = 8192.0;
     auto equal = [](size_t n, double photons, double k1) { return std::vector<LockLoad>(n, LockLoad{ photons, k1 }); };
     for (const bool once : { false, true }) {
         CHECK(!tmc::lockstep_batch({}, waves, once));
@@ -69,6 +69,10 @@ void check_lockstep_batch()
         CHECK(!tmc::lockstep_batch(equal(64, 1 << 20, 10.0), waves, once));
         CHECK(!tmc::lockstep_batch(equal(8, 1 << 22, 31.0), waves, once));
         CHECK(!tmc::lockstep_batch(equal(8, 1 << 22, 73.0), waves, once));
+        CHECK(!tmc::lockstep_batch(equal(4, 1 << 21, 73.0), waves, once));
+        CHECK(tmc::lockstep_batch(equal(4, 1 << 21, 211.0), waves, once));
+        CHECK(tmc::lockstep_batch(equal(1, 1 << 20, 31.0), waves, once) == !once);
+        CHECK(tmc::lockstep_batch(equal(64, 1 << 15, 31.0), waves, once));
         CHECK(tmc::lockstep_batch(equal(2000, 64, 73.0), waves, once) == !once);
         CHECK(tmc::lockstep_batch(equal(300, 65536, 73.0), waves, once) == !once);
         // a large set of short cycles among others that take most of the time

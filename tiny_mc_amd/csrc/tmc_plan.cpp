@@ -159,16 +159,19 @@ bool tmc::cohort_shape(uint64_t photons, uint64_t most, double L, uint32_t shell
  *
  * All waves append to the count of the set they walk, and additions to one
  * address take more than 11 ns each, while 8192 waves end a batch of 64 photons
- * every 0.1 k1 ns: with k1 below 120 and not enough sets under way at a time
- * they wait for one another (eight sets of 2^22 photons, cycles of 31: 2.60
- * and 4.62 ms, of 73: 5.61 and 6.57, of 2^20, 73: 1.65 and 1.69).
+ * every 0.1 k1 ns: with not enough sets under way at a time they wait for one
+ * another, and more so where lockstep has little to gain (eight sets of 2^22
+ * photons, cycles of 31: 2.60 and 4.62 ms, of 73: 5.61 and 6.57, of 2^20, 73:
+ * 1.65 and 1.69; four of 2^21, 31: 1.03 and 1.29, 54: 1.47 and 1.65, 73: 1.71 and
+ * 1.92, 211: 4.85 and 3.92).
  *
  * A plan made for one run has to earn what laying it out and releasing it takes
  * more, 0.1 ms and 0.1 us a set, and 0.3 ms for large lists (planned, run and
- * released, default physics: 2000 sets of 64 photons 863 and 920 us, of 1000
- * 1394 and 1296; 10,000 of 1000 4816 and 5670; 8 of 2^20 1845 and 1981; cycles of
- * 10, 64 of 2^14 681 and 519, of 2^16 706 and 792; albedo 0.99: 2000 of 1000 7022
- * and 5655, 8 of 2^18 4701 and 3568). */
+ * released, default physics: one set of 64 photons 222 and 231 us, of 1000 561
+ * and 338; 2000 sets of 64 863 and 920, of 1000 1394 and 1296; 10,000 of 1000 4816
+ * and 5670; 8 of 2^20 1845 and 1981; cycles of 31, one of 2^20 655 and 718, 64 of
+ * 2^16 856 and 810; of 10, 64 of 2^14 681 and 519, of 2^16 706 and 792; albedo
+ * 0.99, 2000 of 1000 7022 and 5655, 8 of 2^18 4701 and 3568). */
 bool tmc::lockstep_batch(const std::vector<LockLoad>& sets, double waves, bool once)
 {
     double photons = 0.0, steps = 0.0;
@@ -180,7 +183,9 @@ bool tmc::lockstep_batch(const std::vector<LockLoad>& sets, double waves, bool o
     constexpr double many = 4194304.0;
     if (mean < 8.0 || (mean < 30.0 && (photons >= many || n > 1000.0)))
         return false;
-    if (once && (steps < 40.0 * n * n || (photons >= many && mean < 100.0) || (photons > many / 4.0 && mean < 30.0)))
+    if (once && (steps < 40.0 * n * n || (mean < 100.0 && (steps < 30000.0 || photons >= many))
+                 || (mean < 30.0 && photons > many / 4.0)
+                 || (mean >= 30.0 && mean < 100.0 && photons >= many / 4.0 && photons >= many / 16.0 * n)))
         return false;
     /* work of the sets whose waves wait for their count: a wave's 32nd of a
      * launch is a chunk */
@@ -188,7 +193,7 @@ bool tmc::lockstep_batch(const std::vector<LockLoad>& sets, double waves, bool o
     double waits = 0.0;
     for (const LockLoad& s : sets) {
         const double chunks = s.photons / 64.0 / std::ceil(each / s.k1);
-        if (s.k1 * std::max(1.0, waves / chunks) < 120.0)
+        if (s.k1 * std::max(1.0, waves / chunks) < (s.k1 < 100.0 ? 200.0 : 120.0))
             waits += s.photons * s.k1;
     }
     return waits <= steps / 8.0;
