@@ -456,10 +456,11 @@ std::vector<Slice> slices_of(uint64_t first, uint64_t photons, uint64_t most)
 /* Threads of a lockstep launch's workgroups for `waves` waves of work: half of
  * TMC_LOCK_BLOCK where that leaves fewer waves on the fullest compute unit, if
  * the waves are all resident (half as large, at least twice as many workgroups
- * are: 8 of them take 60 KB of LDS, with the rejection sampler 6 take 90) (albedo 0.99: 50,000 photons, 98 workgroups of
- * eight waves or 196 of four, 237 and 198 us; 180,000 421 and 352 us), else
- * TMC_LOCK_BLOCK, with half as many sums to add up (2^17 photons at default
- * physics 58 and 61 us), which is what a cycle of fewer than 64 steps takes. */
+ * are: 8 of them take 60 KB of LDS, with the rejection sampler 6 take 90), else
+ * TMC_LOCK_BLOCK, with half as many sums to add up, which is what a cycle of
+ * fewer than 64 steps takes.  (Albedo 0.99: 50,000 photons, 98 workgroups of
+ * eight waves or 196 of four, 237 and 198 us; 180,000 421 and 352 us; 2^17
+ * photons at default physics 58 and 61 us.) */
 uint32_t lock_block_for(double waves, uint32_t steps, uint32_t grid_most, uint32_t cus)
 {
     const auto fullest = [=](double per_wg) { return per_wg * std::ceil(std::ceil(waves / per_wg) / (double)cus); };
